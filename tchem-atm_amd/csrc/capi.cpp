@@ -21,14 +21,16 @@
 #include "aerosol_model.hpp"
 #include "device_mech.hpp"
 #include "kinetic_model.hpp"
+#include "lowered.hpp"
 #include "mechanism.hpp"
 #include "schedule.hpp"
 
 namespace tchem_amd {
 hipError_t launchIntegrator(const IntegratorArgs& a, int precision, int grid, size_t lds, hipStream_t stream);
-hipError_t integratorMaxBlocksPerCU(int precision, int sparse, int m, int threads, size_t lds, int* blocks, bool rec);
+hipError_t integratorMaxBlocksPerCU(int precision, int sparse, int m, const DevLowered& w, int threads, size_t lds,
+                                    int* blocks, bool rec);
 int sparseMaxCellsPerGroup(int precision, int m);
-size_t integratorStaticLds(int precision, int sparse, int m);
+size_t integratorStaticLds(int precision, int sparse, int m, const DevLowered& w);
 hipError_t launchResetCounter(int* counter, hipStream_t stream);
 hipError_t launchAutotuneSample(int n, long long stride, int nb, int np, int iters, const double* state,
                                 const double* photo, const tchem_time_advance_t* tadv, double* st0, double* ph,
@@ -44,8 +46,7 @@ hipError_t launchAerosol(const IntegratorArgs& a, int grid, size_t lds, hipStrea
 hipError_t launchAerosolRhs(const IntegratorArgs& a, size_t lds, hipStream_t stream);
 hipError_t launchLoopControl(int n, const double* t_out, const tchem_time_advance_t* tadv, double fraction, int* ctl,
                              bool reset, hipStream_t stream);
-size_t adjointCellBytes(const DevMech& M, const DevSparse& S);
-hipError_t adjointMaxBlocksPerCU(int m, int threads, size_t lds, int* blocks);
+hipError_t adjointMaxBlocksPerCU(int m, const DevLowered& w, int threads, size_t lds, int* blocks);
 hipError_t launchAdjoint(const AdjointArgs& a, int grid, size_t lds, hipStream_t stream);
 hipError_t launchE3smKinetics(const DevE3sm& E, int mode, int nBatch, const double* state, const double* photo,
                               int nPhoto, const double* ext, double* out, int ldOut, hipStream_t stream);
@@ -113,9 +114,11 @@ struct tchem_kmcd_s {
   bool cb05Kinetics = true;  // ... with the CB05 rate constants (runDeviceBatch, source term, Jacobian, adjoint)
   std::string e3smBoxError;  // empty when the E3SM box model (AtmosphericChemistryE3SM) can run
   DevE3sm e3{};             // E3SM kinetics tables (every mechanism the loader reads)
-  SparseSchedule sched, schedT;  // forward and transposed (adjoint) programs
   DevMech dev{};
-  DevSparse sparse{}, sparseT{};
+  // encoded sparse programs (enabled 0: none): FP64 and FP32 entries, and
+  // the adjoint's forward and transposed programs on their own cell layout
+  DevLowered low64{}, low32{}, lowAdj{}, lowAdjT{};
+  const DevLowered& lowered(int precision) const { return precision == TCHEM_PRECISION_FP64 ? low64 : low32; }
   std::vector<void*> allocations;
   int device = 0;
   int numCUs = 0;
@@ -123,6 +126,7 @@ struct tchem_kmcd_s {
   int* queue = nullptr;
   double* kf = nullptr;  // [capacity][nReac] rate constants of the last batch
   size_t kfCapacity = 0;  // cells
+  int nnzF = 0;           // entries of the factor in the fill-reducing order (0: no sparse schedule)
   int graphs = 0;         // live captured graphs that read this kmcd's tables
   ~tchem_kmcd_s() {
     if (kf) allocations.push_back(kf);
@@ -141,8 +145,7 @@ struct tchem_amd_s {
 struct tchem_amcd_s {
   tchem_kmcd_s* kmcd = nullptr;  // not owned
   DevAerosol X{};
-  DevSparse S{};                 // programs over the mt unknowns (S.enabled = 0: dense form only)
-  SparseSchedule sched;
+  DevLowered W{};                // programs over the mt unknowns (W.enabled = 0: dense form only)
   int stateDim = 0;
   std::vector<void*> allocations;
   int device = 0;
@@ -204,6 +207,12 @@ int upload(tchem_kmcd_s* k, const std::vector<T>& v, const T** out) {
   return TCHEM_OK;
 }
 
+// Tolerances are staged where one cell still fits beside them.
+void stageTolerances(DevLowered& w, int m, size_t cellBytes, size_t maxLds) {
+  w.tolStaged = 1;
+  if (sparseStageBytes(w, m, false) + cellBytes > maxLds) w.tolStaged = 0;
+}
+
 // Options after validation, with the LU form resolved.
 int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, tchem_atmchem_options_t* o,
                    const char* who) {
@@ -223,7 +232,7 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   // enough to fill its 256 x 256 tiles (m >= 128)
   if (o->lu == TCHEM_LU_AUTO && o->precision == TCHEM_PRECISION_MIXED && o->cells_per_block <= 1 &&
       k->dev.m >= 128 && k->dev.m <= 255 && k->dev.oMfjTermW != 0 && mfmaCellLdsBytes(k->dev) <= k->maxLds &&
-      (!k->sparse.enabled || double(k->sparse.nnzF) >= 0.3 * double(k->dev.m) * double(k->dev.m)))
+      (k->nnzF == 0 || double(k->nnzF) >= 0.3 * double(k->dev.m) * double(k->dev.m)))
     o->lu = TCHEM_LU_MFMA;
   if (o->lu == TCHEM_LU_MFMA) {
     if (o->precision != TCHEM_PRECISION_MIXED)
@@ -242,28 +251,29 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   if (o->programs < TCHEM_PROGRAMS_AUTO || o->programs > TCHEM_PROGRAMS_MEMORY)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": unknown programs placement");
   const size_t bytesA = o->precision == TCHEM_PRECISION_FP64 ? sizeof(double) : sizeof(float);
-  const size_t staticLds = integratorStaticLds(o->precision, 1, k->dev.m);
+  const DevLowered& W = k->lowered(o->precision);
+  const size_t staticLds = integratorStaticLds(o->precision, 1, k->dev.m, W);
   const size_t maxLds = k->maxLds > staticLds ? k->maxLds - staticLds : 0;
-  const size_t cellB = sparseCellBytes(k->dev, k->sparse, bytesA);
+  const size_t cellB = size_t(W.cellBytes);
   // AUTO: programs staged into LDS when that still leaves room for as many
   // cells per workgroup as reading them from memory would (the kernel is
   // latency bound: resident cells set its throughput); memory otherwise
   if (o->programs == TCHEM_PROGRAMS_AUTO) {
     const int cap = sparseMaxCellsPerGroup(o->precision, k->dev.m);
-    const size_t prog = sparseProgramBytes(k->sparse);
-    const size_t coefB = sparseCoefBytes(k->sparse);
+    const size_t prog = sparseStageBytes(W, k->dev.m, true);
+    const size_t coefB = sparseStageBytes(W, k->dev.m, false);
     const size_t inMem = coefB < maxLds ? std::min<size_t>(cap, cellB ? (maxLds - coefB) / cellB : 0) : 0;
     const size_t inLds = prog < maxLds ? std::min<size_t>(cap, cellB ? (maxLds - prog) / cellB : 0) : 0;
     o->programs = (inLds >= 1 && inLds >= inMem) ? TCHEM_PROGRAMS_LDS : TCHEM_PROGRAMS_MEMORY;
   }
   const bool staged = o->programs == TCHEM_PROGRAMS_LDS;
   auto sparseFits = [&](int cells) {
-    return (staged ? sparseProgramBytes(k->sparse) : sparseCoefBytes(k->sparse)) + size_t(cells) * cellB <= maxLds;
+    return sparseStageBytes(W, k->dev.m, staged) + size_t(cells) * cellB <= maxLds;
   };
   if (o->lu == TCHEM_LU_AUTO)
-    o->lu = (k->sparse.enabled && sparseFits(1)) ? TCHEM_LU_SPARSE : TCHEM_LU_DENSE;
+    o->lu = (W.enabled && sparseFits(1)) ? TCHEM_LU_SPARSE : TCHEM_LU_DENSE;
   if (o->lu == TCHEM_LU_SPARSE) {
-    if (!k->sparse.enabled)
+    if (!W.enabled)
       return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": mechanism has no sparse schedule");
     const int cap = sparseMaxCellsPerGroup(o->precision, k->dev.m);
     if (o->cells_per_block == 0) {
@@ -293,9 +303,10 @@ bool sparseStaged(const tchem_atmchem_options_t& o) { return o.programs == TCHEM
 size_t ldsBytes(const tchem_kmcd_s* k, const tchem_atmchem_options_t& o) {
   if (o.lu == TCHEM_LU_MFMA) return mfmaCellLdsBytes(k->dev);
   const size_t bytesA = o.precision == TCHEM_PRECISION_FP64 ? sizeof(double) : sizeof(float);
-  if (o.lu == TCHEM_LU_SPARSE)
-    return (sparseStaged(o) ? sparseProgramBytes(k->sparse) : sparseCoefBytes(k->sparse)) +
-           size_t(o.cells_per_block) * sparseCellBytes(k->dev, k->sparse, bytesA);
+  if (o.lu == TCHEM_LU_SPARSE) {
+    const DevLowered& W = k->lowered(o.precision);
+    return sparseStageBytes(W, k->dev.m, sparseStaged(o)) + size_t(o.cells_per_block) * size_t(W.cellBytes);
+  }
   return integratorLdsBytes(k->dev, bytesA);
 }
 
@@ -323,8 +334,8 @@ int resolveBlocksPerCU(const tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& 
   *bpc = o.blocks_per_cu;
   if (*bpc > 0) return TCHEM_OK;
   const int sparse = o.lu == TCHEM_LU_MFMA ? 3 : (o.lu == TCHEM_LU_SPARSE ? (sparseStaged(o) ? 1 : 2) : 0);
-  hipError_t e = integratorMaxBlocksPerCU(o.precision, sparse, kmcd->dev.m, 64 * o.cells_per_block,
-                                          ldsBytes(kmcd, o), bpc, rec);
+  hipError_t e = integratorMaxBlocksPerCU(o.precision, sparse, kmcd->dev.m, kmcd->lowered(o.precision),
+                                          64 * o.cells_per_block, ldsBytes(kmcd, o), bpc, rec);
   if (e != hipSuccess) return hipFail(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
   if (*bpc < 1) *bpc = 1;
   return TCHEM_OK;
@@ -343,15 +354,12 @@ int runIntegrator(tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& o, const do
   if (hipGetDevice(&cur) != hipSuccess || cur != kmcd->device)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": kmcd belongs to another device");
   a.M = kmcd->dev;
-  a.S = kmcd->sparse;
+  a.W = kmcd->lowered(o.precision);
   a.sparse = o.lu == TCHEM_LU_MFMA ? 3 : (o.lu == TCHEM_LU_SPARSE ? (sparseStaged(o) ? 1 : 2) : 0);
   if (!a.queue) a.queue = kmcd->queue;
   a.persistent = (o.schedule == TCHEM_SCHEDULE_PERSISTENT) ? 1 : 0;
   a.cellsPerGroup = o.cells_per_block;
-  a.cellBytes = (a.sparse == 1 || a.sparse == 2)
-                    ? int(sparseCellBytes(kmcd->dev, kmcd->sparse,
-                                          o.precision == TCHEM_PRECISION_FP64 ? sizeof(double) : sizeof(float)))
-                    : 0;
+  a.cellBytes = (a.sparse == 1 || a.sparse == 2) ? a.W.cellBytes : 0;
   if (!ratesReady) {
     hipError_t e = launchRates(kmcd->dev, a.nBatch, a.state, a.photo, lscale, lstride, const_cast<double*>(a.kf), a.skip,
                                s);
@@ -403,7 +411,7 @@ int adjointCheck(const tchem_kmcd_s* k, int nBatch, int maxSteps, const char* wh
   if (nBatch < 0) return setError(TCHEM_ERR_INVALID, std::string(who) + ": negative nBatch");
   if (maxSteps < 1 || maxSteps > (1 << 24))
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": maxSteps must be in [1, 2^24]");
-  if (!k->sparse.enabled || !k->sparseT.enabled)
+  if (!k->low64.enabled || !k->lowAdj.enabled || !k->lowAdjT.enabled)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": mechanism has no sparse (transposed) schedule");
   return TCHEM_OK;
 }
@@ -557,17 +565,12 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
   d.oPhotoSlot = addI(t.photoSlot);
   d.oReacSpec = addI(t.reacSpec);
   d.oReacPow = addI(t.reacPow);
-  d.oOmegaReac = addI(t.omegaReac);
-  d.oSegBegin = addI(t.segBegin);
-  d.oSegEnd = addI(t.segEnd);
-  d.oRowSegPtr = addI(t.rowSegPtr);
   d.oPairPtr = addI(t.pairPtr);
   d.oPairSlot = addI(t.pairSlot);
   d.oJnzRowCol = addI(rowcol);
   d.oJnzPtr = addI(t.jnzPtr);
   d.oJcPair = addI(t.jcPair);
   d.oRatePar = addD(t.ratePar);
-  d.oOmegaCoef = addD(t.omegaCoef);
   d.oEmission = addD(t.emission);
   d.oJcCoef = addD(t.jcCoef);
   d.oSerOmegaPtr = addI(t.serOmegaPtr);
@@ -628,55 +631,31 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
     d.oMfjTermW = addI(termW);
     d.oMfjTermC = addI(termC);
   }
-  // sparse schedules (mechanisms they cannot express run the dense form only)
-  auto words = [](const std::vector<unsigned>& v) { return std::vector<int>(v.begin(), v.end()); };
-  auto pack = [&](const SparseSchedule& sc, DevSparse& sp) {
-    sp.enabled = 1;
-    sp.nnzF = sc.nnzF;
-    sp.zeroSlot = sc.zeroSlot;
-    sp.trashSlot = sc.trashSlot;
-    sp.pairSlots = sc.pairSlots;
-    sp.oEvalHdr = addI(words(sc.evalHdr));
-    sp.oEvalBody = addI(words(sc.evalBody));
-    sp.evalBodyWords = int(sc.evalBody.size());
-    sp.oCoef = addD(sc.coefTable);
-    sp.nCoef = int(sc.coefTable.size());
-    sp.ropRounds = sc.ropRounds;
-    sp.pairRounds = sc.pairRounds;
-    sp.segRounds = sc.segRounds;
-    sp.jacRounds = sc.jacRounds;
-    sp.pairBody = sc.pairBody;
-    sp.segBody = sc.segBody;
-    sp.jacBody = sc.jacBody;
-    sp.nutRounds = sc.nutRounds;
-    sp.jtvRounds = sc.jtvRounds;
-    sp.nutBody = sc.nutBody;
-    sp.jtvBody = sc.jtvBody;
-    sp.oProgHdr = addI(words(sc.progHdr));
-    sp.oProgBody = addI(words(sc.progBody));
-    sp.luRounds = sc.luRounds;
-    sp.backRounds = sc.backRounds;
-    sp.fwdRounds = sc.fwdRounds;
-    sp.backBody = sc.backBody;
-    sp.fwdBody = sc.fwdBody;
+  // sparse programs (mechanisms they cannot express, or whose cell region
+  // exceeds the LDS, run the dense form only)
+  auto pack = [&](const SparseSchedule& sc, int bytesT, bool adjoint, DevLowered* w) {
+    LoweredProgram p = lowerProgram(t, sc, bytesT, adjoint);
+    stageTolerances(p.d, t.m, size_t(p.d.cellBytes), k->maxLds);
+    if (sparseStageBytes(p.d, t.m, false) + size_t(p.d.cellBytes) > k->maxLds) return;
+    *w = p.d;
+    w->oWords = addI(std::vector<int>(p.words.begin(), p.words.end()));
+    w->oCoef = addD(p.coef);
   };
   try {
     if (!k->boxModel) throw std::runtime_error("no box model");
-    k->sched = buildSparseSchedule(t);
-    pack(k->sched, k->sparse);
-  } catch (const std::exception&) {
-    k->sparse = DevSparse{};
-  }
-  if (k->sparse.enabled) {
-    // the adjoint shares the cell layout of the forward programs: the
-    // transposed factor pattern has the same size
-    try {
-      k->schedT = buildSparseSchedule(t, true);
-      if (k->schedT.nnzF == k->sched.nnzF && k->schedT.pairSlots == k->sched.pairSlots)
-        pack(k->schedT, k->sparseT);
-    } catch (const std::exception&) {
-      k->sparseT = DevSparse{};
+    const SparseSchedule fwd = buildSparseSchedule(t);
+    k->nnzF = fwd.nnzF;
+    pack(fwd, 8, false, &k->low64);
+    pack(fwd, 4, false, &k->low32);
+    // the adjoint shares one cell layout between the forward programs and
+    // the transposed ones: the transposed factor pattern has the same size
+    const SparseSchedule trn = buildSparseSchedule(t, true);
+    if (k->low64.enabled && trn.nnzF == fwd.nnzF && trn.pairSlots == fwd.pairSlots) {
+      pack(fwd, 8, true, &k->lowAdj);
+      pack(trn, 8, true, &k->lowAdjT);
     }
+  } catch (const std::exception&) {
+    // what was encoded so far stands
   }
   {
     // E3SM kinetics tables straight from the loader's data
@@ -1044,18 +1023,19 @@ int tchem_adjoint_backward(int nBatch, const double* lambda, double* lambda_out,
   if (hipGetDevice(&cur) != hipSuccess || cur != kmcd->device)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": kmcd belongs to another device");
   const DevMech& M = kmcd->dev;
-  const size_t cellB = adjointCellBytes(M, kmcd->sparse);
+  const size_t cellB = adjointCellBytes(M, kmcd->lowAdj, kmcd->lowAdjT);
+  const size_t stageB = sparseStageBytes(kmcd->lowAdjT, 0, false);
   int cpg = 8;
-  while (cpg > 1 && size_t(cpg) * cellB > kmcd->maxLds) --cpg;
-  if (cellB > kmcd->maxLds)
+  while (cpg > 1 && stageB + size_t(cpg) * cellB > kmcd->maxLds) --cpg;
+  if (stageB + cellB > kmcd->maxLds)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": one cell needs " + std::to_string(cellB) +
                                                " bytes of LDS, device limit " + std::to_string(kmcd->maxLds));
-  const size_t lds = size_t(cpg) * cellB;
+  const size_t lds = stageB + size_t(cpg) * cellB;
   const AdjointLayout W = adjointLayout(M, nBatch, maxSteps);
   char* ws = static_cast<char*>(workspace);
   AdjointArgs a{};
   a.fw.M = M;
-  a.fw.S = kmcd->sparse;
+  a.fw.W = kmcd->lowAdj;
   a.fw.nBatch = nBatch;
   a.fw.kf = reinterpret_cast<const double*>(ws + W.kf);
   a.fw.queue = kmcd->queue;
@@ -1068,7 +1048,7 @@ int tchem_adjoint_backward(int nBatch, const double* lambda, double* lambda_out,
   a.fw.rec.ckpt = reinterpret_cast<double*>(ws + W.ckpt);
   a.fw.rec.consts = reinterpret_cast<double*>(ws + W.consts);
   a.fw.rec.maxSteps = maxSteps;
-  a.ST = kmcd->sparseT;
+  a.WT = kmcd->lowAdjT;
   a.header = reinterpret_cast<const int*>(ws + W.header);
   a.tol = reinterpret_cast<const double*>(ws + W.tol);
   a.newton = reinterpret_cast<const int*>(ws + W.newton);
@@ -1079,7 +1059,7 @@ int tchem_adjoint_backward(int nBatch, const double* lambda, double* lambda_out,
   a.cellsPerGroup = cpg;
   a.cellBytes = int(cellB);
   int bpc = 0;
-  hipError_t e = adjointMaxBlocksPerCU(M.m, 64 * cpg, lds, &bpc);
+  hipError_t e = adjointMaxBlocksPerCU(M.m, kmcd->lowAdjT, 64 * cpg, lds, &bpc);
   if (e != hipSuccess) return hipFail(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
   if (bpc < 1) bpc = 1;
   const int groups = (nBatch + cpg - 1) / cpg;
@@ -1591,8 +1571,7 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
   try {
     std::vector<std::array<int, 2>> ent;  // (row, col) of every transfer derivative, table order
     const MechTables ta = aerosolTables(t, am, &ent);
-    h->sched = buildSparseSchedule(ta, false);
-    const SparseSchedule& sc = h->sched;
+    const SparseSchedule sc = buildSparseSchedule(ta, false);
     auto position = [&](int r, int c) {  // the LDS slot of factor entry (r, c)
       for (int q = sc.rowPtr[r]; q < sc.rowPtr[r + 1]; ++q)
         if (sc.colIdx[q] == c) return sc.slotOf[size_t(q)];
@@ -1600,40 +1579,13 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
     };
     X.oJpos = int(ib.size());
     for (const auto& e : ent) ib.push_back(position(e[0], e[1]));
-    auto addI = [&](const std::vector<unsigned>& v) {
-      const int off = int(pib.size());
-      pib.insert(pib.end(), v.begin(), v.end());
-      while (pib.size() % 4) pib.push_back(0);
-      return off;
-    };
-    DevSparse& sp = h->S;
-    sp.enabled = 1;
-    sp.nnzF = sc.nnzF;
-    sp.zeroSlot = sc.zeroSlot;
-    sp.trashSlot = sc.trashSlot;
-    sp.pairSlots = sc.pairSlots;
-    sp.oEvalHdr = addI(sc.evalHdr);
-    sp.oEvalBody = addI(sc.evalBody);
-    sp.evalBodyWords = int(sc.evalBody.size());
-    sp.oCoef = 0;
-    pdb = sc.coefTable;
-    sp.nCoef = int(sc.coefTable.size());
-    sp.ropRounds = sc.ropRounds;
-    sp.pairRounds = sc.pairRounds;
-    sp.segRounds = sc.segRounds;
-    sp.jacRounds = sc.jacRounds;
-    sp.pairBody = sc.pairBody;
-    sp.segBody = sc.segBody;
-    sp.jacBody = sc.jacBody;
-    sp.oProgHdr = addI(sc.progHdr);
-    sp.oProgBody = addI(sc.progBody);
-    sp.luRounds = sc.luRounds;
-    sp.backRounds = sc.backRounds;
-    sp.fwdRounds = sc.fwdRounds;
-    sp.backBody = sc.backBody;
-    sp.fwdBody = sc.fwdBody;
+    LoweredProgram p = lowerProgram(ta, sc, 8, false);
+    stageTolerances(p.d, mt, aerosolSparseCellBytes(p.d, X), kmcd->maxLds);
+    h->W = p.d;
+    pib.assign(p.words.begin(), p.words.end());
+    pdb = std::move(p.coef);
   } catch (const std::exception&) {
-    h->S = DevSparse{};  // the dense form still runs
+    h->W = DevLowered{};  // the dense form still runs
     pib.clear();
     pdb.clear();
   }
@@ -1652,7 +1604,7 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
     return hipFail(e, "hipMemcpy");
   X.ib = static_cast<const int*>(pi);
   X.db = static_cast<const double*>(pd);
-  if (h->S.enabled) {
+  if (h->W.enabled) {
     void* qi = nullptr;
     void* qd = nullptr;
     if ((e = hipMalloc(&qi, sizeof(int) * pib.size())) != hipSuccess) return hipFail(e, "hipMalloc");
@@ -1666,8 +1618,8 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
     X.pdb = static_cast<const double*>(qd);
   }
   const bool denseFits = aerosolCellsPerGroup(kmcd->dev, X, kmcd->maxLds) >= 1;
-  const bool sparseFits = h->S.enabled && aerosolSparseCellBytes(kmcd->dev, h->S, X) <= kmcd->maxLds;
-  if (!sparseFits) h->S = DevSparse{};
+  const bool sparseFits = h->W.enabled && sparseStageBytes(h->W, mt, false) + aerosolSparseCellBytes(h->W, X) <= kmcd->maxLds;
+  if (!sparseFits) h->W = DevLowered{};
   if (!denseFits && !sparseFits)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": one cell does not fit the LDS");
   *out = h.release();
@@ -1683,7 +1635,6 @@ namespace {
 IntegratorArgs aerosolArgs(tchem_amcd_s* h, int nBatch) {
   IntegratorArgs a{};
   a.M = h->kmcd->dev;
-  a.S = h->kmcd->sparse;
   a.X = h->X;
   a.nBatch = nBatch;
   a.cellBytes = int((aerosolLdsBytes(a.M, a.X) + 15) & ~size_t(15));
@@ -1720,9 +1671,9 @@ int tchem_aerosolchem_run_device_batch(const tchem_atmchem_options_t* opts, int 
   if (!amcd || nBatch < 0) return setError(TCHEM_ERR_INVALID, std::string(who) + ": bad argument");
   if (opts && opts->precision != TCHEM_PRECISION_FP64)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": the aerosol integrator is FP64 only");
-  if (opts && opts->lu == TCHEM_LU_SPARSE && !amcd->S.enabled)
+  if (opts && opts->lu == TCHEM_LU_SPARSE && !amcd->W.enabled)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": no sparse programs for this model");
-  const bool sparse = amcd->S.enabled && !(opts && opts->lu == TCHEM_LU_DENSE);
+  const bool sparse = amcd->W.enabled && !(opts && opts->lu == TCHEM_LU_DENSE);
   if (!sparse && aerosolCellsPerGroup(amcd->kmcd->dev, amcd->X, amcd->kmcd->maxLds) < 1)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": the dense form needs at most 128 unknowns");
   if (nBatch == 0) return TCHEM_OK;
@@ -1747,18 +1698,20 @@ int tchem_aerosolchem_run_device_batch(const tchem_atmchem_options_t* opts, int 
   a.kf = k->kf;
   a.numberConc = number_conc;
   int cells = aerosolCellsPerGroup(a.M, a.X, k->maxLds);
+  size_t stageB = 0;
   if (sparse) {
     a.sparse = 1;
-    a.S = amcd->S;
-    a.cellBytes = int(aerosolSparseCellBytes(a.M, a.S, a.X));
-    cells = int(k->maxLds / size_t(a.cellBytes));
+    a.W = amcd->W;
+    a.cellBytes = int(aerosolSparseCellBytes(a.W, a.X));
+    stageB = sparseStageBytes(a.W, a.X.mt, false);
+    cells = int((k->maxLds - stageB) / size_t(a.cellBytes));
     if (cells > 8) cells = 8;
   }
   if (cells < 1) return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": one cell does not fit the LDS");
   const int perGroup = cells < nBatch ? cells : nBatch;
   a.cellsPerGroup = perGroup;
   const int grid = (nBatch + perGroup - 1) / perGroup;
-  e = launchAerosol(a, grid, size_t(perGroup) * size_t(a.cellBytes), s);
+  e = launchAerosol(a, grid, stageB + size_t(perGroup) * size_t(a.cellBytes), s);
   if (e != hipSuccess) return hipFail(e, "aerosol integrator launch");
   return TCHEM_OK;
 }

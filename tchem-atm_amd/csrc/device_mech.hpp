@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/tchem_atm.h"
+#include "lowered.hpp"
 
 namespace tchem_amd {
 
@@ -17,10 +18,9 @@ struct DevMech {
   // instead of twenty.
   const int* ib;
   const double* db;
-  int oPerm, oRateKind, oConvExp, oPhotoSlot, oReacSpec, oReacPow, oOmegaReac, oSegBegin, oSegEnd, oRowSegPtr,
-      oPairPtr, oPairSlot, oJnzRowCol, oJnzPtr, oJcPair, oSerOmegaPtr, oSerOmegaReac, oSerJRowCol, oSerJPtr,
-      oSerJPair;
-  int oRatePar, oOmegaCoef, oEmission, oJcCoef, oSerOmegaCoef, oSerJCoef;
+  int oPerm, oRateKind, oConvExp, oPhotoSlot, oReacSpec, oReacPow, oPairPtr, oPairSlot, oJnzRowCol, oJnzPtr, oJcPair,
+      oSerOmegaPtr, oSerOmegaReac, oSerJRowCol, oSerJPtr, oSerJPair;
+  int oRatePar, oEmission, oJcCoef, oSerOmegaCoef, oSerJCoef;
   // the serial Jacobian lists regrouped for the MFMA form's assembly
   // (m <= 255 only; offsets 0 otherwise): per column quarter, each of the
   // 256 threads of the workgroup walks its own run of terms, stored
@@ -33,17 +33,12 @@ struct DevMech {
   __host__ __device__ const int* photoSlot() const { return ib + oPhotoSlot; }   // [nReac]
   __host__ __device__ const int* reacSpec() const { return ib + oReacSpec; }     // [nReac][maxR]
   __host__ __device__ const int* reacPow() const { return ib + oReacPow; }       // [nReac][maxR]
-  __host__ __device__ const int* omegaReac() const { return ib + oOmegaReac; }   // [nnzOmega]
-  __host__ __device__ const int* segBegin() const { return ib + oSegBegin; }     // [nSeg]
-  __host__ __device__ const int* segEnd() const { return ib + oSegEnd; }         // [nSeg]
-  __host__ __device__ const int* rowSegPtr() const { return ib + oRowSegPtr; }   // [m+1]
   __host__ __device__ const int* pairPtr() const { return ib + oPairPtr; }       // [nReac+1]
   __host__ __device__ const int* pairSlot() const { return ib + oPairSlot; }     // [nPairs]
   __host__ __device__ const int* jnzRowCol() const { return ib + oJnzRowCol; }   // [nnzJ] row * 65536 + col
   __host__ __device__ const int* jnzPtr() const { return ib + oJnzPtr; }         // [nnzJ+1]
   __host__ __device__ const int* jcPair() const { return ib + oJcPair; }         // [nContrib]
   __host__ __device__ const double* ratePar() const { return db + oRatePar; }    // [nReac][8]
-  __host__ __device__ const double* omegaCoef() const { return db + oOmegaCoef; }// [nnzOmega]
   __host__ __device__ const double* emission() const { return db + oEmission; }  // [m]
   __host__ __device__ const double* jcCoef() const { return db + oJcCoef; }      // [nContrib]
   // serial gathers of the dense form (mechanism.hpp)
@@ -64,47 +59,13 @@ struct DevMech {
   }
 };
 
-// Device view of the compiled sparse programs (schedule.hpp); arrays live
-// in the mechanism's int / double buffers, addressed by offsets.
-struct DevSparse {
-  int enabled;  // 0: mechanism has no sparse programs
-  int nnzF, zeroSlot, trashSlot, pairSlots;
-  // evaluation program (staged into LDS) and its coefficient table
-  int oEvalHdr, oEvalBody, evalBodyWords, oCoef, nCoef;
-  int ropRounds, pairRounds, segRounds, jacRounds;
-  int pairBody, segBody, jacBody;
-  int nutRounds, jtvRounds, nutBody, jtvBody;  // adjoint sections (transposed programs only)
-  // LU program: the LU and BACK sections are staged into LDS, FWD (factor
-  // reuse) is read from memory
-  int oProgHdr, oProgBody;
-  int luRounds, backRounds, fwdRounds;
-  int backBody, fwdBody;
-};
-
-// LDS layout of a sparse-form workgroup: LU program headers and staged
-// bodies, evaluation program headers and bodies, coefficient table, then one
-// cell region per wavefront.  Word counts are rounded up to 4 (16 bytes).
-__host__ __device__ inline size_t al4(size_t words) { return (words + 3) & ~size_t(3); }
-__host__ __device__ inline size_t sparseLuHdrWords(const DevSparse& S) { return al4(size_t(S.luRounds + S.backRounds)); }
-// LU and BACK bodies plus the slack the interpreter may read past the last round
-__host__ __device__ inline size_t sparseLuBodyWords(const DevSparse& S) { return al4(size_t(S.fwdBody) + 64 * 5); }
-__host__ __device__ inline size_t sparseEvalHdrWords(const DevSparse& S) {
-  return al4(size_t(S.ropRounds + S.pairRounds + S.segRounds + S.jacRounds));
-}
-__host__ __device__ inline size_t sparseEvalOffsetWords(const DevSparse& S) {
-  return sparseLuHdrWords(S) + sparseLuBodyWords(S);
-}
-__host__ __device__ inline size_t sparseCoefOffsetWords(const DevSparse& S) {
-  return sparseEvalOffsetWords(S) + sparseEvalHdrWords(S) + al4(size_t(S.evalBodyWords));
-}
-__host__ __device__ inline size_t sparseProgramBytes(const DevSparse& S) {
-  return 4 * sparseCoefOffsetWords(S) + ((8 * size_t(S.nCoef) + 15) & ~size_t(15));
-}
-// With the programs in device memory only the coefficient table is staged:
-// it sits at the start of the workgroup's LDS, before the cell regions (its
-// entries are read on the critical path of every segment and Jacobian round).
-__host__ __device__ inline size_t sparseCoefBytes(const DevSparse& S) {
-  return (8 * size_t(S.nCoef) + 15) & ~size_t(15);
+// LDS a workgroup of the sparse form stages before its cell regions: the
+// instruction stream (staged form), the coefficient table (read on the
+// critical path of every segment round) and, where they fit, the tolerances
+// of m unknowns.
+__host__ __device__ inline size_t sparseStageBytes(const DevLowered& W, int m, bool staged) {
+  return (staged ? 4 * size_t(W.stagedWords) : 0) + ((8 * size_t(W.nCoef) + 15) & ~size_t(15)) +
+         (W.tolStaged ? 16 * size_t(m) : 0);
 }
 
 // Forward record of the discrete adjoint: accepted step sizes and the state
@@ -130,7 +91,7 @@ struct DevAerosol {
   int oGas, oAero;  // [nSimpol] gas unknown (internal order), aerosol species within a particle
   int oPar;         // [nSimpol][8] B1 B2 B3 B4 diffusion mw Nstar computeAlpha
   // sparse form: the mechanism's programs compiled over the mt unknowns
-  // (IntegratorArgs::S) live in these buffers; oJpos indexes X.ib:
+  // (IntegratorArgs::W) live in these buffers; oJpos indexes X.ib:
   // [nPart * nSimpol][2 + 2 nAero] factor positions of the transfer
   // derivatives (g,g), (a,g), (g, particle species i), (a, particle species i)
   const int* pib;
@@ -140,7 +101,7 @@ struct DevAerosol {
 
 struct IntegratorArgs {
   DevMech M;
-  DevSparse S;
+  DevLowered W;                      // sparse forms: the encoded programs of the launch's precision
   int nBatch;
   const double* tol_newton;          // [2]
   const double* tol_time;            // [m][2]
@@ -169,15 +130,13 @@ struct IntegratorArgs {
 // the source term, reciprocal pivots and interchanges over mt, SIMPOL
 // constants [nSimpol][4], particle sums [nPart][4] and transfer terms
 // [nPart * nSimpol][6].
-// LDS bytes of one cell of the sparse aerosol integrator: the sparse cell
-// region (sparseCellBytes, reciprocal pivots over mt) plus the unknown copy,
-// source term and SIMPOL scratch of aerosolLdsBytes.
-inline size_t aerosolSparseCellBytes(const DevMech& M, const DevSparse& S, const DevAerosol& X) {
+// LDS bytes of one cell of the sparse aerosol integrator: the cell region of
+// the encoded programs plus the unknown copy, source term and SIMPOL scratch
+// of aerosolLdsBytes.
+inline size_t aerosolSparseCellBytes(const DevLowered& W, const DevAerosol& X) {
   auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  return al(8 * size_t(S.trashSlot + 1)) + al(8 * size_t(X.mt + 2)) + al(8 * size_t(S.pairSlots)) +
-         al(8 * (size_t(M.nSpec) + 2 * size_t(M.nReac + 1) + size_t(M.nSeg + 1))) +
-         al(8 * (2 * size_t(X.mt) + 4 * size_t(X.nSimpol) + 4 * size_t(X.nPart) +
-                 6 * size_t(X.nPart) * size_t(X.nSimpol)));
+  return size_t(W.cellBytes) + al(8 * (2 * size_t(X.mt) + 4 * size_t(X.nSimpol) + 4 * size_t(X.nPart) +
+                                       6 * size_t(X.nPart) * size_t(X.nSimpol)));
 }
 
 inline size_t aerosolLdsBytes(const DevMech& M, const DevAerosol& X, bool withMatrix = true) {
@@ -203,17 +162,6 @@ __host__ __device__ inline size_t integratorLdsBytes(const DevMech& M, size_t by
 }
 
 
-// LDS bytes of one cell region of the sparse form: factor entries + RHS +
-// zero and trash slots, reciprocal pivots (+ a zero for column m and a
-// trash slot) and the Jacobian derivative pairs in TA precision, then
-// doubles for concentrations, rate constants (+ a zero), rates of progress
-// (+ zero slot) and source-term segment sums (+ trash slot).
-__host__ __device__ inline size_t sparseCellBytes(const DevMech& M, const DevSparse& S, size_t bytesA) {
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  return al(bytesA * size_t(S.trashSlot + 1)) + al(bytesA * size_t(M.m + 2)) + al(bytesA * size_t(S.pairSlots)) +
-         al(sizeof(double) * (size_t(M.nSpec) + size_t(M.nReac + 1) + size_t(M.nReac + 1) + size_t(M.nSeg + 1)));
-}
-
 // Tables of the E3SM/UCI kinetics (ReactionRates / RateofProgress /
 // NetProductionRates of the reference): every rate-constant form the loader
 // reads, in the reference's parameter layout, indexed into the kmcd's int
@@ -236,8 +184,8 @@ struct DevE3sm {
 
 // Arguments of the discrete adjoint kernel (backward sweep over a record).
 struct AdjointArgs {
-  IntegratorArgs fw;        // M, S (forward programs), nBatch, kf, rec, queue
-  DevSparse ST;             // transposed programs
+  IntegratorArgs fw;        // M, W (forward programs), nBatch, kf, rec, queue
+  DevLowered WT;            // transposed programs, same cell layout
   const int* header;        // [4] nBatch, maxSteps of the record
   const double* tol;        // [2] Newton atol, rtol of the recording run
   const int* newton;        // [nBatch][2] max Newton iterations, Jacobian interval
@@ -249,10 +197,13 @@ struct AdjointArgs {
   int cellBytes;            // LDS bytes of one cell region
 };
 
-// LDS of the adjoint beyond the sparse cell region: mu, w, v, grad
-__host__ __device__ inline size_t adjointExtraBytes(const DevMech& M) {
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  return al(8 * size_t(M.m + 1)) + al(8 * size_t(M.nReac + 2)) + al(8 * size_t(M.m + 1)) + al(8 * size_t(M.nReac));
+// LDS bytes of one cell of the adjoint: the region of both programs, then
+// the gradient
+__host__ __device__ inline size_t adjointRegionBytes(const DevLowered& W, const DevLowered& WT) {
+  return size_t(W.cellBytes > WT.cellBytes ? W.cellBytes : WT.cellBytes);
+}
+inline size_t adjointCellBytes(const DevMech& M, const DevLowered& W, const DevLowered& WT) {
+  return adjointRegionBytes(W, WT) + ((8 * size_t(M.nReac) + 15) & ~size_t(15));
 }
 
 }  // namespace tchem_amd

@@ -25,7 +25,6 @@
 
 #include "detmath.h"
 #include "device_mech.hpp"
-#include "schedule.hpp"
 
 namespace tchem_amd {
 
@@ -82,12 +81,6 @@ __device__ __forceinline__ float readlane(float v, int l) {
 }
 
 __device__ __forceinline__ unsigned long long ballot(bool p) { return __ballot(p); }
-
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, kWave));
-  return v;
-}
 
 // value of slot `idx` (lane idx % 64, register slot idx / 64) on every lane
 template <int QM, typename TA>
@@ -495,554 +488,13 @@ __device__ void lu_back(const CellLds<TA>& L, int m, int lane, TA (&b)[QM]) {
   }
 }
 
-// ---- sparse form ------------------------------------------------------------
-// Compiled schedules (schedule.hpp): the iteration matrix is held as the
-// nonzeros of its symbolic LU pattern, factorised without interchanges in
-// the fill-reducing order by list-scheduled rounds; the RHS is stored after
-// the matrix entries and eliminated alongside.
+}  // namespace
+}  // namespace tchem_amd
 
-template <typename TA>
-struct SpLds {
-  const unsigned* hdr;    // LU program headers (LU + BACK sections), shared by the workgroup
-  const unsigned* body;   // LU program bodies
-  const unsigned* ehdr;   // evaluation program headers
-  const unsigned* ebody;  // evaluation program bodies
-  const double* coef;     // stoichiometric coefficient table
-  TA* A;        // [trashSlot+1] factor entries, RHS, zero slot, trash slot
-  TA* rdiag;    // [m+2] reciprocal pivots, rdiag[m] = 0, rdiag[m+1] = trash
-  TA* dpr;      // [pairSlots] Jacobian derivative pairs, dpr[nPairs] = 0
-  double* c;    // [nSpec]
-  double* kf;   // [nReac+1], kf[nReac] = 0
-  double* rop;  // [nReac+1], rop[nReac] = 0
-  double* seg;  // [nSeg+1], seg[nSeg] = trash
-  const double* src;  // nullable: this cell's external sources [m], reference order
-  // discrete adjoint only (nullptr otherwise)
-  double* mu;   // [m+1] adjoint vector, mu[m] = 0
-  double* w;    // [nReac+2] nu_r . mu, w[nReac] = 0, w[nReac+1] = trash
-  double* v;    // [m+1] J^T mu, v[m] = trash
-};
+#include "sparse_exec.hpp"
 
-// STAGED: programs at the start of the workgroup's LDS, then one cell region
-// per wavefront; otherwise the programs are read from device memory (they
-// stay resident in L2) and the cell regions start at 0, or, with COEF, after
-// the coefficient table staged at the start of the LDS (sparseCoefBytes).
-template <typename TA, bool STAGED, bool COEF = false>
-__device__ SpLds<TA> carve_sparse(char* base, const DevMech& M, const DevSparse& S, int cellBytes, int wave) {
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  SpLds<TA> L;
-  char* cell;
-  if (STAGED) {
-    const unsigned* w = reinterpret_cast<const unsigned*>(base);
-    L.hdr = w;
-    L.body = w + sparseLuHdrWords(S);
-    L.ehdr = w + sparseEvalOffsetWords(S);
-    L.ebody = L.ehdr + sparseEvalHdrWords(S);
-    L.coef = reinterpret_cast<const double*>(w + sparseCoefOffsetWords(S));
-    cell = base + sparseProgramBytes(S) + size_t(wave) * size_t(cellBytes);
-  } else {
-    L.hdr = reinterpret_cast<const unsigned*>(M.ib + S.oProgHdr);
-    L.body = reinterpret_cast<const unsigned*>(M.ib + S.oProgBody);
-    L.ehdr = reinterpret_cast<const unsigned*>(M.ib + S.oEvalHdr);
-    L.ebody = reinterpret_cast<const unsigned*>(M.ib + S.oEvalBody);
-    L.coef = COEF ? reinterpret_cast<const double*>(base) : M.db + S.oCoef;
-    cell = base + (COEF ? sparseCoefBytes(S) : 0) + size_t(wave) * size_t(cellBytes);
-  }
-  size_t off = 0;
-  L.A = reinterpret_cast<TA*>(cell);
-  off += al(sizeof(TA) * size_t(S.trashSlot + 1));
-  L.rdiag = reinterpret_cast<TA*>(cell + off);
-  off += al(sizeof(TA) * size_t(M.m + 2));
-  L.dpr = reinterpret_cast<TA*>(cell + off);
-  off += al(sizeof(TA) * size_t(S.pairSlots));
-  L.c = reinterpret_cast<double*>(cell + off);
-  L.kf = L.c + M.nSpec;
-  L.rop = L.kf + M.nReac + 1;
-  L.seg = L.rop + M.nReac + 1;
-  L.mu = L.w = L.v = nullptr;
-  L.src = nullptr;
-  return L;
-}
-
-// x^n for small n >= 0 by repeated multiplication (exact for n <= 2; at
-// most n-1 roundings above); powers up to 3 without a loop (selects, the
-// same products in the same order)
-__device__ __forceinline__ double ipow(double x, int n) {
-  double r = n >= 1 ? x : 1.0;
-  r = n >= 2 ? r * x : r;
-  r = n >= 3 ? r * x : r;
-  for (int i = 3; i < n; ++i) r *= x;
-  return r;
-}
-// packed reactant field: species | power << 12, kNone for no reactant (a
-// factor 1: power 0 of an in-range slot, no branch)
-__device__ __forceinline__ double reactant_factor(const double* c, unsigned f) {
-  const bool none = f == SparseSchedule::kNone;
-  return ipow(c[none ? 0u : (f & 0xfff)], none ? 0 : int(f >> 12));
-}
-
-// Rates of progress (kRop rounds) and, with pairs, the derivatives
-// d rop_r / d c_s (kPair rounds) at the concentrations in LDS: the same
-// products in the same order as the dense form.  Rounds are independent;
-// the next round's two words are loaded while a round computes.
-template <typename TA>
-__device__ __forceinline__ void sp_rates(const DevSparse& S, const SpLds<TA>& L, int lane, bool pairs) {
-  {
-    const unsigned* b = L.ebody;
-    unsigned w0 = b[lane], w1 = b[kWave + lane];
-    for (int g = 0; g < S.ropRounds; ++g) {
-      b += 2 * kWave;
-      const unsigned n0 = b[lane], n1 = b[kWave + lane];
-      const int r = int(w0 & 0xffff);
-      L.rop[r] = L.kf[r] * reactant_factor(L.c, w0 >> 16) * reactant_factor(L.c, w1 & 0xffff) *
-                 reactant_factor(L.c, w1 >> 16);
-      w0 = n0;
-      w1 = n1;
-    }
-  }
-  if (!pairs) return;
-  const unsigned* b = L.ebody + S.pairBody;
-  unsigned w0 = b[lane], w1 = b[kWave + lane];
-  for (int g = 0; g < S.pairRounds; ++g) {
-    b += 2 * kWave;
-    const unsigned n0 = b[lane], n1 = b[kWave + lane];
-    const int r = int(w0 & 0x3fff), js = int((w0 >> 14) & 3);
-    const unsigned f0 = w0 >> 16, f1 = w1 & 0xffff, f2 = w1 >> 16;
-    const unsigned fs = js == 0 ? f0 : (js == 1 ? f1 : f2);
-    const int ns = int(fs >> 12);
-    double d = L.kf[r] * double(ns) * ipow(L.c[fs & 0xfff], ns - 1);
-    if (js != 0) d *= reactant_factor(L.c, f0);
-    if (js != 1) d *= reactant_factor(L.c, f1);
-    if (js != 2) d *= reactant_factor(L.c, f2);
-    L.dpr[g * kWave + lane] = TA(d);
-    w0 = n0;
-    w1 = n1;
-  }
-}
-
-// one segment-sum round, LEN entries per lane (w[0] = target, w[1..] = (reaction | coef << 16))
-template <int LEN, typename TA>
-__device__ __forceinline__ void seg_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], const SpLds<TA>& L) {
-  const unsigned t = w[0] & ~SparseSchedule::kCont;
-  double acc = (w[0] & SparseSchedule::kCont) ? L.seg[t] : 0.0;
-  double cf[LEN], rv[LEN];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    cf[j] = L.coef[w[1 + j] >> 16];
-    rv[j] = L.rop[w[1 + j] & 0xffff];
-  }
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) acc += cf[j] * rv[j];
-  L.seg[t] = acc;
-}
-// one Jacobian round: A[t] = (cont ? A[t] : diag) + scale * sum coef * dpr, in TA precision
-template <int LEN, typename TA>
-__device__ __forceinline__ void jac_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], const SpLds<TA>& L,
-                                          TA tdiag, TA tscale) {
-  const unsigned t = w[0] & 0x3fffffffu;
-  const TA init = (w[0] & SparseSchedule::kCont) ? L.A[t] : (((w[0] >> 30) & 1u) ? tdiag : TA(0));
-  TA cf[LEN], dv[LEN];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    cf[j] = TA(L.coef[w[1 + j] >> 16]);
-    dv[j] = L.dpr[w[1 + j] & 0xffff];
-  }
-  TA sum = TA(0);
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) sum += cf[j] * dv[j];
-  L.A[t] = init + tscale * sum;
-}
-
-// nu_r . mu (kNuT): w[t] = (cont ? w[t] : 0) + sum coef * mu[species]
-template <int LEN, typename TA>
-__device__ __forceinline__ void nut_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], const SpLds<TA>& L) {
-  const unsigned t = w[0] & ~SparseSchedule::kCont;
-  double acc = (w[0] & SparseSchedule::kCont) ? L.w[t] : 0.0;
-  double cf[LEN], mv[LEN];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    cf[j] = L.coef[w[1 + j] >> 16];
-    mv[j] = L.mu[w[1 + j] & 0xffff];
-  }
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) acc += cf[j] * mv[j];
-  L.w[t] = acc;
-}
-// J^T mu (kJtv): v[t] = (cont ? v[t] : 0) + sum dpr[pair] * w[reaction]
-template <int LEN, typename TA>
-__device__ __forceinline__ void jtv_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], const SpLds<TA>& L) {
-  const unsigned t = w[0] & ~SparseSchedule::kCont;
-  double acc = (w[0] & SparseSchedule::kCont) ? L.v[t] : 0.0;
-  double dv[LEN], wv[LEN];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    dv[j] = double(L.dpr[w[1 + j] & 0xffff]);
-    wv[j] = L.w[w[1 + j] >> 16];
-  }
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) acc += dv[j] * wv[j];
-  L.v[t] = acc;
-}
-
-// Round driver for programs read from device memory, where a round's words
-// take longer to arrive than a round takes to run: the words of round r + 2
-// are loaded while round r runs, into three register sets used in rotation
-// (no copies, so no wait until a set's round comes up), and the headers come
-// through scalar loads.  exec(h, w) runs one round with header h and this
-// lane's words w; size(h) is the round's body length in words.  The loads
-// stop at the last round, so nothing past the program is read.
-template <class Size, class Exec>
-__device__ __forceinline__ void pipelined_rounds(const unsigned* hdr, const unsigned* body, int nr, int lane,
-                                                 Size size, Exec exec) {
-  constexpr int kW = 1 + SparseSchedule::kMaxChain;
-  if (nr <= 0) return;
-  using cptr = const __attribute__((address_space(4))) unsigned*;
-  const cptr sh = (cptr)hdr;
-  unsigned wa[kW], wb[kW], wc[kW];
-  auto load = [&](unsigned (&w)[kW], const unsigned* b) {
-#pragma unroll
-    for (int j = 0; j < kW; ++j) w[j] = b[kWave * j + lane];
-  };
-  unsigned h0 = sh[0];
-  unsigned h1 = nr > 1 ? sh[1] : 0u;
-  const unsigned* b1 = body + size(h0);  // body of round r + 1
-  load(wa, body);
-  if (nr > 1) load(wb, b1);
-  int r = 0;
-  // one round: run round r from `cur`, load round r + 2 into `nxt2`
-  auto step = [&](unsigned (&cur)[kW], unsigned (&nxt2)[kW]) -> bool {
-    const unsigned* b2 = b1 + size(h1);
-    unsigned h2 = 0u;
-    if (r + 2 < nr) {
-      h2 = sh[r + 2];
-      load(nxt2, b2);
-    }
-    exec(h0, cur);
-    if (++r >= nr) return false;
-    h0 = h1;
-    h1 = h2;
-    b1 = b2;
-    return true;
-  };
-  while (step(wa, wc) && step(wb, wa) && step(wc, wb)) {
-  }
-}
-
-// Runs nr chained rounds of the evaluation program starting at header
-// index r0 and body word offset body0: kSeg / kJac rounds, and with ADJ
-// also kNuT / kJtv.  Rounds run in order (a chain split over rounds
-// continues in a later one); the next round's words are loaded while a
-// round computes.
-template <bool ADJ, typename TA>
-__device__ __forceinline__ void eval_rounds(const SpLds<TA>& L, int lane, int r0, int nr, int body0, double diag, double scale) {
-  constexpr int kW = 1 + SparseSchedule::kMaxChain;
-  const unsigned* hdr = L.ehdr + r0;
-  const unsigned* b = L.ebody + body0;
-  const TA tdiag = TA(diag), tscale = TA(scale);
-  unsigned w[kW];
-#pragma unroll
-  for (int j = 0; j < kW; ++j) w[j] = b[kWave * j + lane];
-  unsigned h = nr > 0 ? __builtin_amdgcn_readfirstlane(hdr[0]) : 0u;
-  for (int r = 0; r < nr; ++r) {
-    const unsigned hn = r + 1 < nr ? hdr[r + 1] : 0u;
-    const int kind = int(h >> 16), len = int(h & 0xffff);
-    b += kWave * (1 + len);
-    unsigned wn[kW];
-#pragma unroll
-    for (int j = 0; j < kW; ++j) wn[j] = b[kWave * j + lane];
-    if (kind == SparseSchedule::kSeg) {
-      switch (len) {
-        case 1: seg_round<1>(w, L); break;
-        case 2: seg_round<2>(w, L); break;
-        case 3: seg_round<3>(w, L); break;
-        default: seg_round<4>(w, L); break;
-      }
-    } else if (!ADJ || kind == SparseSchedule::kJac) {
-      switch (len) {
-        case 1: jac_round<1>(w, L, tdiag, tscale); break;
-        case 2: jac_round<2>(w, L, tdiag, tscale); break;
-        case 3: jac_round<3>(w, L, tdiag, tscale); break;
-        default: jac_round<4>(w, L, tdiag, tscale); break;
-      }
-    } else if (kind == SparseSchedule::kNuT) {
-      switch (len) {
-        case 1: nut_round<1>(w, L); break;
-        case 2: nut_round<2>(w, L); break;
-        case 3: nut_round<3>(w, L); break;
-        default: nut_round<4>(w, L); break;
-      }
-    } else {
-      switch (len) {
-        case 1: jtv_round<1>(w, L); break;
-        case 2: jtv_round<2>(w, L); break;
-        case 3: jtv_round<3>(w, L); break;
-        default: jtv_round<4>(w, L); break;
-      }
-    }
-    h = __builtin_amdgcn_readfirstlane(hn);
-#pragma unroll
-    for (int j = 0; j < kW; ++j) w[j] = wn[j];
-  }
-}
-
-// eval_rounds (kSeg / kJac only) for programs in device memory
-template <typename TA>
-__device__ __forceinline__ void eval_rounds_pf(const SpLds<TA>& L, int lane, int r0, int nr, int body0, double diag,
-                                               double scale) {
-  constexpr int kW = 1 + SparseSchedule::kMaxChain;
-  const TA tdiag = TA(diag), tscale = TA(scale);
-  pipelined_rounds(
-      L.ehdr + r0, L.ebody + body0, nr, lane, [](unsigned h) { return kWave * (1 + int(h & 0xffff)); },
-      [&](unsigned h, const unsigned (&w)[kW]) {
-        const int kind = int(h >> 16), len = int(h & 0xffff);
-        if (kind == SparseSchedule::kSeg) {
-          switch (len) {
-            case 1: seg_round<1>(w, L); break;
-            case 2: seg_round<2>(w, L); break;
-            case 3: seg_round<3>(w, L); break;
-            default: seg_round<4>(w, L); break;
-          }
-        } else {
-          switch (len) {
-            case 1: jac_round<1>(w, L, tdiag, tscale); break;
-            case 2: jac_round<2>(w, L, tdiag, tscale); break;
-            case 3: jac_round<3>(w, L, tdiag, tscale); break;
-            default: jac_round<4>(w, L, tdiag, tscale); break;
-          }
-        }
-      });
-}
-
-// Source-term segment sums (kSeg rounds) and, with jac, A = diag * I +
-// scale * J on the factor pattern (kJac rounds; fill positions cleared).
-template <typename TA, bool PF = false>
-__device__ void sp_sums(const DevSparse& S, const SpLds<TA>& L, int lane, bool jac, double diag, double scale) {
-  if constexpr (PF)
-    eval_rounds_pf(L, lane, S.ropRounds + S.pairRounds, S.segRounds + (jac ? S.jacRounds : 0), S.segBody, diag,
-                   scale);
-  else
-    eval_rounds<false>(L, lane, S.ropRounds + S.pairRounds, S.segRounds + (jac ? S.jacRounds : 0), S.segBody, diag,
-                       scale);
-}
-
-// per-species sums of the segment sums plus emission and external sources
-// (register layout)
-template <int QM>
-__device__ __forceinline__ void row_sums(const DevMech& M, const double* seg, const double* src, int lane,
-                                         double (&f)[QM]) {
-#pragma unroll
-  for (int q = 0; q < QM; ++q) {
-    const int a = lane + kWave * q;
-    double s = 0.0;
-    if (a < M.m) {
-      s = M.emission()[a];
-      if (src) s += src[M.perm()[a]];
-      const int s1 = M.rowSegPtr()[a + 1];
-      for (int g = M.rowSegPtr()[a]; g < s1; ++g) s += seg[g];
-    }
-    f[q] = s;
-  }
-}
-
-// One chained-update round with LEN entries per lane (w[0] = target,
-// w[1..LEN] = entries): every load is issued before the first use.
-template <int LEN, typename TA>
-__device__ __forceinline__ void upd_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], TA* A) {
-  TA acc = A[w[0]];
-  TA l[LEN], u[LEN];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    l[j] = A[w[1 + j] & 0xffff];
-    u[j] = A[w[1 + j] >> 16];
-  }
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) acc -= l[j] * u[j];
-  A[w[0]] = acc;
-}
-// Reciprocal of a pivot: the correctly rounded quotient in FP64; in FP32 the
-// hardware reciprocal (within 1 ulp: one instruction instead of the eleven of
-// a correctly rounded division, well inside the FP32 factorisation's own
-// rounding).  Zero and non-finite pivots give non-finite reciprocals in both.
-template <typename TA>
-__device__ __forceinline__ TA pivot_recip(TA p) {
-  if constexpr (sizeof(TA) == sizeof(float))
-    return __builtin_amdgcn_rcpf(p);
-  else
-    return TA(1) / p;
-}
-// A kMulUpd round with LEN chain entries per lane (w[3..3+LEN)); returns
-// true for a zero or non-finite pivot on a lane that stores one.
-template <int LEN, typename TA>
-__device__ __forceinline__ bool mulupd_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], TA* A, TA* rdiag,
-                                             int m) {
-  const int t = int(w[0]);
-  const int ik = int(w[1] & 0xffff), kj = int(w[1] >> 16);
-  const int kk = int(w[2] & 0x7fff), ri = int(w[2] >> 16);
-  const bool mul = (w[2] & 0x8000u) != 0;
-  const TA p = A[kk];
-  const TA a = A[ik];
-  const TA b = A[kj];
-  TA acc = A[t];
-  TA lo[LEN > 0 ? LEN : 1], hi[LEN > 0 ? LEN : 1];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    lo[j] = A[w[3 + j] & 0xffff];
-    hi[j] = A[w[3 + j] >> 16];
-  }
-  const TA inv = pivot_recip(p);
-  const TA l = a == TA(0) ? TA(0) : a * inv;
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) acc -= lo[j] * hi[j];
-  A[t] = mul ? l : acc - l * b;
-  rdiag[ri] = inv;
-  return ri != m + 1 && !(p != TA(0) && isfinite(p) && isfinite(inv));
-}
-template <int LEN, typename TA>
-__device__ __forceinline__ void back_round(const unsigned (&w)[1 + SparseSchedule::kMaxChain], TA* A,
-                                           const TA* rdiag, int rhs0) {
-  TA acc = A[w[0]];
-  TA U[LEN], b[LEN], r[LEN];
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) {
-    const int k = int(w[1 + j] >> 16);
-    U[j] = A[w[1 + j] & 0xffff];
-    b[j] = A[rhs0 + k];
-    r[j] = rdiag[k];
-  }
-#pragma unroll
-  for (int j = 0; j < LEN; ++j) acc -= U[j] * (b[j] * r[j]);
-  A[w[0]] = acc;
-}
-
-// Runs rounds of the LU / substitution program (schedule.hpp): multiplier
-// and pivot records (kMul), chained updates A[t] -= sum A[lo] * A[hi] (kUpd),
-// multipliers fused with updates that scale A[ik] themselves, plus chained
-// updates (kMulUpd)
-// and column-oriented back-substitution updates
-// A[t] -= sum A[lo] * (A[rhs0 + k] * rdiag[k]) (kBack).  Lanes of a round
-// touch disjoint targets; rounds run in order.  Branch free per lane
-// (padding reads zero slots, writes trash slots); the header two rounds
-// ahead and the next round's words are loaded while a round runs, so a
-// round waits only for its matrix data.  Returns false when a pivot is
-// zero or not finite.
-template <typename TA>
-__device__ bool run_program(const unsigned* hdr, const unsigned* body, int nRounds, TA* A, TA* rdiag, int m,
-                            int rhs0, int trash, int lane) {
-  constexpr int kW = 1 + SparseSchedule::kMaxChain;
-  bool bad = false;
-  if (nRounds <= 0) return true;
-  unsigned h0 = __builtin_amdgcn_readfirstlane(hdr[0]);
-  unsigned h1 = nRounds > 1 ? hdr[1] : 0u;
-  unsigned w[kW];
-#pragma unroll
-  for (int j = 0; j < kW; ++j) w[j] = body[kWave * j + lane];
-  for (int r = 0; r < nRounds; ++r) {
-    const unsigned h2 = r + 2 < nRounds ? hdr[r + 2] : 0u;
-    const int kind = int(h0 >> 16), len = int(h0 & 0xffff);
-    const unsigned* bnext = body + (kind == SparseSchedule::kMul ? kWave : kWave * (1 + len));
-    unsigned wn[kW];
-#pragma unroll
-    for (int j = 0; j < kW; ++j) wn[j] = bnext[kWave * j + lane];
-    if (kind == SparseSchedule::kMul) {
-      const int dst = int(w[0] & 0xffff), src = int(w[0] >> 16);
-      const bool piv = (dst & 0x8000) != 0;
-      const int ai = piv ? trash : dst;
-      const int ri = piv ? (dst & 0x7fff) : m + 1;
-      const TA p = A[src];
-      const TA a = A[ai];
-      const TA inv = pivot_recip(p);
-      A[ai] = a * inv;
-      rdiag[ri] = inv;
-      bad |= piv && !(p != TA(0) && isfinite(p) && isfinite(inv));
-    } else if (kind == SparseSchedule::kUpd) {
-      switch (len) {
-        case 1: upd_round<1>(w, A); break;
-        case 2: upd_round<2>(w, A); break;
-        case 3: upd_round<3>(w, A); break;
-        default: upd_round<4>(w, A); break;
-      }
-    } else if (kind == SparseSchedule::kMulUpd) {
-      static_assert(SparseSchedule::kMaxMulUpdChain == 2, "kMulUpd chain cases");
-      switch (len) {
-        case 2: bad |= mulupd_round<0>(w, A, rdiag, m); break;
-        case 3: bad |= mulupd_round<1>(w, A, rdiag, m); break;
-        default: bad |= mulupd_round<2>(w, A, rdiag, m); break;
-      }
-    } else {
-      switch (len) {
-        case 1: back_round<1>(w, A, rdiag, rhs0); break;
-        case 2: back_round<2>(w, A, rdiag, rhs0); break;
-        case 3: back_round<3>(w, A, rdiag, rhs0); break;
-        default: back_round<4>(w, A, rdiag, rhs0); break;
-      }
-    }
-    wave_sync();
-    body = bnext;
-    h0 = __builtin_amdgcn_readfirstlane(h1);
-    h1 = h2;
-#pragma unroll
-    for (int j = 0; j < kW; ++j) w[j] = wn[j];
-  }
-  return ballot(bad) == 0;
-}
-
-// run_program for programs in device memory (pipelined_rounds)
-template <typename TA>
-__device__ bool run_program_pf(const unsigned* hdr, const unsigned* body, int nRounds, TA* A, TA* rdiag, int m,
-                               int rhs0, int trash, int lane) {
-  constexpr int kW = 1 + SparseSchedule::kMaxChain;
-  bool bad = false;
-  pipelined_rounds(
-      hdr, body, nRounds, lane,
-      [](unsigned h) { return int(h >> 16) == SparseSchedule::kMul ? kWave : kWave * (1 + int(h & 0xffff)); },
-      [&](unsigned h, const unsigned (&w)[kW]) {
-        const int kind = int(h >> 16), len = int(h & 0xffff);
-        if (kind == SparseSchedule::kMul) {
-          const int dst = int(w[0] & 0xffff), src = int(w[0] >> 16);
-          const bool piv = (dst & 0x8000) != 0;
-          const int ai = piv ? trash : dst;
-          const int ri = piv ? (dst & 0x7fff) : m + 1;
-          const TA p = A[src];
-          const TA a = A[ai];
-          const TA inv = pivot_recip(p);
-          A[ai] = a * inv;
-          rdiag[ri] = inv;
-          bad |= piv && !(p != TA(0) && isfinite(p) && isfinite(inv));
-        } else if (kind == SparseSchedule::kUpd) {
-          switch (len) {
-            case 1: upd_round<1>(w, A); break;
-            case 2: upd_round<2>(w, A); break;
-            case 3: upd_round<3>(w, A); break;
-            default: upd_round<4>(w, A); break;
-          }
-        } else if (kind == SparseSchedule::kMulUpd) {
-          switch (len) {
-            case 2: bad |= mulupd_round<0>(w, A, rdiag, m); break;
-            case 3: bad |= mulupd_round<1>(w, A, rdiag, m); break;
-            default: bad |= mulupd_round<2>(w, A, rdiag, m); break;
-          }
-        } else {
-          switch (len) {
-            case 1: back_round<1>(w, A, rdiag, rhs0); break;
-            case 2: back_round<2>(w, A, rdiag, rhs0); break;
-            case 3: back_round<3>(w, A, rdiag, rhs0); break;
-            default: back_round<4>(w, A, rdiag, rhs0); break;
-          }
-        }
-        wave_sync();
-      });
-  return ballot(bad) == 0;
-}
-
-// the LU / substitution interpreter for programs staged in LDS or read from
-// device memory
-template <bool STAGED, typename TA>
-__device__ __forceinline__ bool program(const unsigned* hdr, const unsigned* body, int nRounds, TA* A, TA* rdiag,
-                                        int m, int rhs0, int trash, int lane) {
-  if constexpr (STAGED)
-    return run_program(hdr, body, nRounds, A, rdiag, m, rhs0, trash, lane);
-  else
-    return run_program_pf(hdr, body, nRounds, A, rdiag, m, rhs0, trash, lane);
-}
+namespace tchem_amd {
+namespace {
 
 // ---- backends -----------------------------------------------------------------
 // Both provide: Lds (per-cell LDS view), Fact (state of the stored factors),
@@ -1056,11 +508,17 @@ struct DenseBackend {
   static constexpr bool kCollective = false;  // factorisation by the whole workgroup (collective_solve)
   using Lds = CellLds<TA>;
   struct Fact { int nswp = 0; };
-  // unknowns, state row length, state column and tolerance row of unknown ai
+  // unknowns, state row length, state column and tolerances of unknown ai
   static __device__ __forceinline__ int unknowns(const IntegratorArgs& a) { return a.M.m; }
   static __device__ __forceinline__ int rowDim(const IntegratorArgs& a) { return a.M.nSpec + 3; }
   static __device__ __forceinline__ int column(const IntegratorArgs& a, int ai) { return 3 + a.M.perm()[ai]; }
-  static __device__ __forceinline__ int tolIndex(const IntegratorArgs& a, int ai) { return a.M.perm()[ai]; }
+  static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds&, int ai, double& atol,
+                                                   double& rtol) {
+    const int xs = a.M.perm()[ai];
+    atol = a.tol_time[2 * xs];
+    rtol = a.tol_time[2 * xs + 1];
+  }
+  static __device__ __forceinline__ void ready(const IntegratorArgs&, const Lds&, int) {}
   // per-cell bindings: this cell's external sources
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
@@ -1093,62 +551,62 @@ struct DenseBackend {
   }
 };
 
+// time tolerances of unknown ai from the staged table at LDS address tol, or
+// (index: its row) from the caller's
+template <class Index>
+__device__ __forceinline__ void staged_tolerance(const IntegratorArgs& a, unsigned tol, int ai, Index index,
+                                                 double& atol, double& rtol) {
+  if (a.W.tolStaged) {
+    const vec2<double> t = lds_get<vec2<double>>(tol + 16 * ai);
+    atol = t.x;
+    rtol = t.y;
+  } else {
+    const int xs = index(ai);
+    atol = a.tol_time[2 * xs];
+    rtol = a.tol_time[2 * xs + 1];
+  }
+}
+
+// Sparse form: the encoded programs (lowered.hpp), from device memory or
+// staged into the workgroup's LDS.
 template <typename TA_, int QM, bool STAGED>
 struct SparseBackend {
   using TA = TA_;
   static constexpr bool kCollective = false;  // factorisation by the whole workgroup (collective_solve)
-  using Lds = SpLds<TA>;
+  // QM 4 instances take the programs of cell regions above 64 KiB too
+  static constexpr int SH = QM < 4 ? 0 : (sizeof(TA) == 8 ? 3 : 2);
+  using Lds = SpLds<TA, STAGED>;
   struct Fact {};
   static __device__ __forceinline__ int unknowns(const IntegratorArgs& a) { return a.M.m; }
   static __device__ __forceinline__ int rowDim(const IntegratorArgs& a) { return a.M.nSpec + 3; }
   static __device__ __forceinline__ int column(const IntegratorArgs& a, int ai) { return 3 + a.M.perm()[ai]; }
-  static __device__ __forceinline__ int tolIndex(const IntegratorArgs& a, int ai) { return a.M.perm()[ai]; }
+  static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds& L, int ai, double& atol,
+                                                   double& rtol) {
+    staged_tolerance(a, L.tol, ai, [&](int i) { return a.M.perm()[i]; }, atol, rtol);
+  }
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
   }
-  // the mechanism program (LU and BACK sections) is copied into the
-  // workgroup's LDS once; every wavefront of the workgroup reads it.  With
-  // the programs in device memory the coefficient table alone is copied.
   static __device__ void stage(const IntegratorArgs& a, char* base) {
-    const DevSparse& S = a.S;
-    if (!STAGED) {
-      double* cd = reinterpret_cast<double*>(base);
-      for (int i = threadIdx.x; i < S.nCoef; i += blockDim.x) cd[i] = a.M.db[S.oCoef + i];
-      __syncthreads();
-      return;
-    }
-    unsigned* dst = reinterpret_cast<unsigned*>(base);
-    auto copy = [&](size_t at, const int* src, int n) {
-      for (int i = threadIdx.x; i < n; i += blockDim.x) dst[at + size_t(i)] = unsigned(src[i]);
-    };
-    copy(0, a.M.ib + S.oProgHdr, S.luRounds + S.backRounds);
-    copy(sparseLuHdrWords(S), a.M.ib + S.oProgBody, S.fwdBody + 64 * SparseSchedule::kSlack);
-    const size_t e0 = sparseEvalOffsetWords(S);
-    copy(e0, a.M.ib + S.oEvalHdr, S.ropRounds + S.pairRounds + S.segRounds + S.jacRounds);
-    copy(e0 + sparseEvalHdrWords(S), a.M.ib + S.oEvalBody, S.evalBodyWords);
-    double* cd = reinterpret_cast<double*>(dst + sparseCoefOffsetWords(S));
-    for (int i = threadIdx.x; i < S.nCoef; i += blockDim.x) cd[i] = a.M.db[S.oCoef + i];
+    stage_sparse<STAGED>(a.W, reinterpret_cast<const unsigned*>(a.M.ib) + a.W.oWords, a.M.db + a.W.oCoef, base);
+    double* tol = reinterpret_cast<double*>(base + sparseStageBytes(a.W, 0, STAGED));
+    const int n = a.W.tolStaged ? 2 * a.M.m : 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) tol[i] = a.tol_time[2 * a.M.perm()[i >> 1] + (i & 1)];
     __syncthreads();
   }
   static __device__ Lds carve(char* base, const IntegratorArgs& a, int wave) {
-    return carve_sparse<TA, STAGED, !STAGED>(base, a.M, a.S, a.cellBytes, wave);
+    return carve_sparse<TA, STAGED>(a.W, reinterpret_cast<const unsigned*>(a.M.ib) + a.W.oWords, a.M.m, base,
+                                    a.cellBytes, wave);
   }
-  // zero slots read by padded records
-  static __device__ void init(const IntegratorArgs& a, const Lds& L, int lane) {
-    if (lane == 0) {
-      L.kf[a.M.nReac] = 0.0;
-      L.rop[a.M.nReac] = 0.0;
-      L.dpr[a.M.nPairs] = TA(0);
-      L.A[a.S.zeroSlot] = TA(0);
-      L.rdiag[a.M.m] = TA(0);
-    }
-    wave_sync();
+  static __device__ void init(const IntegratorArgs& a, const Lds& L, int lane) { sp_init(a.W, L, a.M.m, lane); }
+  static __device__ __forceinline__ void ready(const IntegratorArgs& a, const Lds& L, int lane) {
+    sp_scaled_rates<SH>(a.W, L, a.M.nReac, lane);
   }
   static __device__ __forceinline__ void put_c(const IntegratorArgs& a, const Lds& L, int lane, const double (&u)[QM]) {
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
-      if (i < a.M.m) L.c[i] = u[q];
+      if (i < a.M.m) lds_put<double>(L.cell + a.W.oC + 8 * i, u[q]);
     }
     wave_sync();
   }
@@ -1156,55 +614,67 @@ struct SparseBackend {
                                                   const double (&u)[QM], const double (&bc)[QM], double ch,
                                                   bool newton, bool refresh, double (&f)[QM], TA (&x)[QM]) {
     TCHEM_PT_BEGIN(rates)
+    // emission and external sources of this lane's species, on their way while the rates are computed
+#pragma unroll
+    for (int q = 0; q < QM; ++q) {
+      const int i = lane + kWave * q;
+      f[q] = 0.0;
+      if (i < a.M.m) {
+        f[q] = a.M.emission()[i];
+        if (L.src) f[q] += L.src[a.M.perm()[i]];
+      }
+    }
     put_c(a, L, lane, u);
-    sp_rates(a.S, L, lane, refresh);
+    sp_rates<SH>(a.W, L, lane, refresh);
     wave_sync();
     TCHEM_PT_END(rates, 11)
-    TCHEM_PT_BEGIN(sums)
-    sp_sums<TA, !STAGED>(a.S, L, lane, refresh, 1.0, -ch);
-    wave_sync();
-    TCHEM_PT_END(sums, 12)
     TCHEM_PT_BEGIN(rows)
-    row_sums<QM>(a.M, L.seg, L.src, lane, f);
+    sp_sums<SH>(L, a.W.oSegHdr, a.W.oSeg, a.W.nSeg, L.coef, L.cell + a.W.oS, lane);
+    wave_sync();
+    sp_rows<SH, QM>(a.W, L, lane, f);
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
       x[q] = (newton && i < a.M.m) ? TA(-(u[q] - bc[q] - ch * f[q])) : TA(0);
-      if (newton && i < a.M.m) L.A[a.S.nnzF + i] = x[q];
+      if (newton && i < a.M.m) lds_put<TA>(L.cell + a.W.oR + 2 * sizeof(TA) * i, x[q]);
     }
-    if (newton) wave_sync();
+    wave_sync();
     TCHEM_PT_END(rows, 13)
+    TCHEM_PT_BEGIN(sums)
+    if (refresh) {
+      sp_jacobian<SH>(a.W, L, lane, TA(-ch));
+      wave_sync();
+    }
+    TCHEM_PT_END(sums, 12)
   }
-  // after the BACK section the RHS holds u_ii x_i
+  // after the back substitution the right-hand side holds u_ii x_i
   static __device__ __forceinline__ void get_x(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM]) {
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
-      x[q] = (i < a.M.m) ? L.A[a.S.nnzF + i] * L.rdiag[i] : TA(0);
+      x[q] = TA(0);
+      if (i < a.M.m) {
+        const vec2<TA> v = lds_get<vec2<TA>>(L.cell + a.W.oR + 2 * sizeof(TA) * i);
+        x[q] = v.x * v.y;
+      }
     }
-  }
-  static __device__ void back(const IntegratorArgs& a, const Lds& L, int lane) {
-    TCHEM_PT_BEGIN(back)
-    program<STAGED>(L.hdr + a.S.luRounds, L.body + a.S.backBody, a.S.backRounds, L.A, L.rdiag, a.M.m, a.S.nnzF,
-                    a.S.trashSlot, lane);
-    TCHEM_PT_END(back, 10)
   }
   static __device__ __forceinline__ bool factor_solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM],
                                                       Fact&) {
     TCHEM_PT_BEGIN(lu)
-    const bool ok = program<STAGED>(L.hdr, L.body, a.S.luRounds, L.A, L.rdiag, a.M.m, a.S.nnzF, a.S.trashSlot, lane);
+    const bool ok = sp_lu<SH>(L, L.w, a.W.oLuHdr, a.W.oLu, a.W.oLu1, a.W.nLu, lane);
     TCHEM_PT_END(lu, 9)
     if (!ok) return false;
-    back(a, L, lane);
+    TCHEM_PT_BEGIN(back)
+    sp_back<SH>(a.W, L, lane);
+    TCHEM_PT_END(back, 10)
     get_x(a, L, lane, x);
     return true;
   }
   static __device__ __forceinline__ void solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM],
                                                const Fact&) {
-    const unsigned* fh = reinterpret_cast<const unsigned*>(a.M.ib + a.S.oProgHdr) + a.S.luRounds + a.S.backRounds;
-    const unsigned* fb = reinterpret_cast<const unsigned*>(a.M.ib + a.S.oProgBody) + a.S.fwdBody;
-    program<false>(fh, fb, a.S.fwdRounds, L.A, L.rdiag, a.M.m, a.S.nnzF, a.S.trashSlot, lane);  // always in memory
-    back(a, L, lane);
+    sp_lu<SH>(L, L.memory(), a.W.oFwdHdr, a.W.oFwd, a.W.oFwd1, a.W.nFwd, lane);
+    sp_back<SH>(a.W, L, lane);
     get_x(a, L, lane, x);
   }
 };
@@ -1213,12 +683,13 @@ struct CellCounters {
   int accepted = 0, rejected = 0, newton_failures = 0, newton_iterations = 0, factorizations = 0, failed = 0;
 };
 
-// wavefront-uniform copy of a value every lane holds (lets the compiler branch on it with scalar code)
-__device__ __forceinline__ double uniform_d(double v) {
-  const long long x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane(int(x & 0xffffffffll));
-  const int hi = __builtin_amdgcn_readfirstlane(int(x >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+// Whether the rounded quotient a / b is at most 1 (a >= 0; false for NaN, 0 / 0
+// and an infinite a), without the division: for finite a and b > 0 the
+// quotient rounds above 1 exactly when a > b, since a / b > 1 is at least
+// 1 + ulp(b) / b > 1 + 2^-53.  The same for an eighth: 8 a is exact (or
+// overflows, and then the quotient is above 1/8 for every b it is compared with).
+__device__ __forceinline__ bool ratio_at_most_one(double a, double b) {
+  return a < INFINITY && ((a <= b && b > 0.0) || b < 0.0);
 }
 
 // One cell of AtmosphericChemistry::runDeviceBatch
@@ -1300,6 +771,7 @@ __device__ void integrate_cell(const IntegratorArgs& a, const typename B::Lds& L
     for (int i = m + lane; i < nSpec; i += kWave) a.rec.consts[size_t(cell) * (nSpec - m) + (i - m)] = row[3 + i];
   }
   wave_sync();
+  B::ready(a, L, lane);
 
   const int max_it = ta._num_time_iterations_per_interval;
   const int max_newton = ta._max_num_newton_iterations;
@@ -1379,22 +851,19 @@ __device__ void integrate_cell(const IntegratorArgs& a, const typename B::Lds& L
         continue;
       }
       {
-        double nrm = 0.0;
+        bool over = false;
 #pragma unroll
         for (int q = 0; q < QM; ++q) {
           const int i = lane + kWave * q;
           if (i < m) {
             const double dx = double(x[q]);
             u[q] += dx;
-            double w = fabs(dx) / (atol_n + rtol_n * fabs(u[q]));
-            if (!(w == w)) w = INFINITY;
-            nrm = fmax(nrm, w);
+            over |= !ratio_at_most_one(fabs(dx), atol_n + rtol_n * fabs(u[q]));
           }
         }
-        nrm = uniform_d(wave_max(nrm));
         ++cnt.newton_iterations;
         ++nit;
-        if (nrm <= 1.0) phase = kStage;
+        if (ballot(over) == 0) phase = kStage;
       }
       continue;
     }
@@ -1422,23 +891,25 @@ __device__ void integrate_cell(const IntegratorArgs& a, const typename B::Lds& L
       phase = kNewton;
       continue;
     }
-    double e = 0.0;
+    // the largest |lte_i| / (atol_i + rtol_i |u_i|) against 1 (accept) and 1/8 (grow)
+    bool above = false, mid = false;
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int ai = lane + kWave * q;
       if (ai < m) {
-        const int xs = B::tolIndex(a, ai);
+        double at, rt;
+        B::tolerance(a, L, ai, at, rt);
         const double lte = 2.0 * k_err * h * (est[q] + f[q] / (1.0 - gam));
-        double w = fabs(lte) / (a.tol_time[2 * xs] + a.tol_time[2 * xs + 1] * fabs(u[q]));
-        if (!(w == w)) w = INFINITY;
-        e = fmax(e, w);
+        const double b = at + rt * fabs(u[q]);
+        above |= !ratio_at_most_one(fabs(lte), b);
+        mid |= !ratio_at_most_one(8.0 * fabs(lte), b);
       }
     }
-    e = uniform_d(wave_max(e));
+    const bool reject = ballot(above) != 0, keep = ballot(mid) != 0;
     ++iter;
     attempt = 0;
     phase = kStep;
-    if (e > 1.0 && h > ta._dtmin) {
+    if (reject && h > ta._dtmin) {
       ++cnt.rejected;
       dt = 0.25 * h;
       continue;
@@ -1449,7 +920,7 @@ __device__ void integrate_cell(const IntegratorArgs& a, const typename B::Lds& L
       un[q] = u[q];
       fn[q] = f[q];
     }
-    dt = (e <= 0.125) ? 2.0 * h : h;
+    dt = keep ? h : 2.0 * h;
     if (dt > ta._dtmax) dt = ta._dtmax;
     if (REC) {
       const int k = cnt.accepted;  // index of this step
@@ -1580,7 +1051,13 @@ struct MfmaBackend {
   static __device__ __forceinline__ int unknowns(const IntegratorArgs& a) { return a.M.m; }
   static __device__ __forceinline__ int rowDim(const IntegratorArgs& a) { return a.M.nSpec + 3; }
   static __device__ __forceinline__ int column(const IntegratorArgs& a, int ai) { return 3 + a.M.perm()[ai]; }
-  static __device__ __forceinline__ int tolIndex(const IntegratorArgs& a, int ai) { return a.M.perm()[ai]; }
+  static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds&, int ai, double& atol,
+                                                   double& rtol) {
+    const int xs = a.M.perm()[ai];
+    atol = a.tol_time[2 * xs];
+    rtol = a.tol_time[2 * xs + 1];
+  }
+  static __device__ __forceinline__ void ready(const IntegratorArgs&, const Lds&, int) {}
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
   }
@@ -1929,9 +1406,15 @@ struct AerosolLayout {
   static __device__ __forceinline__ int column(const IntegratorArgs& a, int ai) {
     return ai < a.M.m ? 3 + a.M.perm()[ai] : 3 + a.M.nSpec + (ai - a.M.m);
   }
-  static __device__ __forceinline__ int tolIndex(const IntegratorArgs& a, int ai) {
-    return ai < a.M.m ? a.M.perm()[ai] : ai;
+  template <class LdsT>
+  static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const LdsT&, int ai, double& atol,
+                                                   double& rtol) {
+    const int xs = ai < a.M.m ? a.M.perm()[ai] : ai;
+    atol = a.tol_time[2 * xs];
+    rtol = a.tol_time[2 * xs + 1];
   }
+  template <class LdsT>
+  static __device__ __forceinline__ void ready(const IntegratorArgs&, const LdsT&, int) {}
   // this cell's number concentrations, temperature and pressure, and the
   // SIMPOL constants (functions of T and p only)
   template <class LdsT>
@@ -2087,7 +1570,8 @@ struct AerosolBackend : AerosolLayout {
 // the gas species), read from device memory; the transfer terms and their derivatives are added to the
 // source term and to the factor entries by one lane, in the dense form's
 // order.
-struct AeroSpLds : SpLds<double> {
+struct AeroSpLds : SpLds<double, false> {
+  double* A;    // factor slots
   double* x;    // [mt] unknowns
   double* f;    // [mt] source term
   double* sc;   // [nSimpol][4]
@@ -2098,36 +1582,17 @@ struct AeroSpLds : SpLds<double> {
 };
 
 __device__ AeroSpLds carve_aero_sparse(char* base, const IntegratorArgs& a, int wave) {
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  const DevMech& M = a.M;
-  const DevSparse& S = a.S;
   const DevAerosol& X = a.X;
   AeroSpLds L;
-  L.hdr = reinterpret_cast<const unsigned*>(X.pib + S.oProgHdr);
-  L.body = reinterpret_cast<const unsigned*>(X.pib + S.oProgBody);
-  L.ehdr = reinterpret_cast<const unsigned*>(X.pib + S.oEvalHdr);
-  L.ebody = reinterpret_cast<const unsigned*>(X.pib + S.oEvalBody);
-  L.coef = X.pdb + S.oCoef;
-  char* cell = base + size_t(wave) * size_t(a.cellBytes);
-  size_t off = 0;
+  static_cast<SpLds<double, false>&>(L) = carve_sparse<double, false>(
+      a.W, reinterpret_cast<const unsigned*>(X.pib) + a.W.oWords, X.mt, base, a.cellBytes, wave);
+  char* cell = base + sparseStageBytes(a.W, X.mt, false) + size_t(wave) * size_t(a.cellBytes);
   L.A = reinterpret_cast<double*>(cell);
-  off += al(8 * size_t(S.trashSlot + 1));
-  L.rdiag = reinterpret_cast<double*>(cell + off);
-  off += al(8 * size_t(X.mt + 2));
-  L.dpr = reinterpret_cast<double*>(cell + off);
-  off += al(8 * size_t(S.pairSlots));
-  L.c = reinterpret_cast<double*>(cell + off);
-  L.kf = L.c + M.nSpec;
-  L.rop = L.kf + M.nReac + 1;
-  L.seg = L.rop + M.nReac + 1;
-  off += al(8 * (size_t(M.nSpec) + 2 * size_t(M.nReac + 1) + size_t(M.nSeg + 1)));
-  L.x = reinterpret_cast<double*>(cell + off);
+  L.x = reinterpret_cast<double*>(cell + a.W.cellBytes);
   L.f = L.x + X.mt;
   L.sc = L.f + X.mt;
   L.ps = L.sc + 4 * X.nSimpol;
   L.pd = L.ps + 4 * X.nPart;
-  L.mu = L.w = L.v = nullptr;
-  L.src = nullptr;
   L.nc = nullptr;
   L.T = L.p = 0.0;
   return L;
@@ -2137,19 +1602,27 @@ template <int QM>
 struct AerosolSparseBackend : AerosolLayout {
   using TA = double;
   static constexpr bool kCollective = false;  // factorisation by the whole workgroup (collective_solve)
+  static constexpr int SH = QM < 4 ? 0 : 3;
   using Lds = AeroSpLds;
   struct Fact {};
-  static __device__ void stage(const IntegratorArgs&, char*) {}
-  static __device__ Lds carve(char* base, const IntegratorArgs& a, int wave) { return carve_aero_sparse(base, a, wave); }
-  static __device__ void init(const IntegratorArgs& a, const Lds& L, int lane) {
-    if (lane == 0) {
-      L.kf[a.M.nReac] = 0.0;
-      L.rop[a.M.nReac] = 0.0;
-      L.dpr[a.M.nPairs] = 0.0;
-      L.A[a.S.zeroSlot] = 0.0;
-      L.rdiag[a.X.mt] = 0.0;
+  static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds& L, int ai, double& atol,
+                                                   double& rtol) {
+    staged_tolerance(a, L.tol, ai, [&](int i) { return i < a.M.m ? a.M.perm()[i] : i; }, atol, rtol);
+  }
+  static __device__ void stage(const IntegratorArgs& a, char* base) {
+    stage_sparse<false>(a.W, nullptr, a.X.pdb + a.W.oCoef, base);
+    double* tol = reinterpret_cast<double*>(base + sparseStageBytes(a.W, 0, false));
+    const int n = a.W.tolStaged ? 2 * a.X.mt : 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+      const int ai = i >> 1, xs = ai < a.M.m ? a.M.perm()[ai] : ai;
+      tol[i] = a.tol_time[2 * xs + (i & 1)];
     }
-    wave_sync();
+    __syncthreads();
+  }
+  static __device__ Lds carve(char* base, const IntegratorArgs& a, int wave) { return carve_aero_sparse(base, a, wave); }
+  static __device__ void init(const IntegratorArgs& a, const Lds& L, int lane) { sp_init(a.W, L, a.X.mt, lane); }
+  static __device__ __forceinline__ void ready(const IntegratorArgs& a, const Lds& L, int lane) {
+    sp_scaled_rates<SH>(a.W, L, a.M.nReac, lane);
   }
   static __device__ void evaluate(const IntegratorArgs& a, const Lds& L, int lane, const double (&u)[QM],
                                   const double (&bc)[QM], double ch, bool newton, bool refresh, double (&f)[QM],
@@ -2157,19 +1630,25 @@ struct AerosolSparseBackend : AerosolLayout {
     const DevMech& M = a.M;
     const DevAerosol& X = a.X;
     const int mt = X.mt;
+    double fg[QM];
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
+      fg[q] = i < M.m ? M.emission()[i] : 0.0;
       if (i < mt) L.x[i] = u[q];
       if (i < M.m) L.c[i] = u[q];
     }
     wave_sync();
-    sp_rates(a.S, L, lane, refresh);
+    sp_rates<SH>(a.W, L, lane, refresh);
     wave_sync();
-    sp_sums(a.S, L, lane, refresh, 1.0, -ch);
+    sp_sums<SH>(L, a.W.oSegHdr, a.W.oSeg, a.W.nSeg, L.coef, L.cell + a.W.oS, lane);
     wave_sync();
-    double fg[QM];
-    row_sums<QM>(M, L.seg, nullptr, lane, fg);
+    sp_rows<SH, QM>(a.W, L, lane, fg);
+    wave_sync();
+    if (refresh) {
+      sp_jacobian<SH>(a.W, L, lane, -ch);
+      wave_sync();
+    }
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
@@ -2225,7 +1704,7 @@ struct AerosolSparseBackend : AerosolLayout {
       const int i = lane + kWave * q;
       f[q] = i < mt ? L.f[i] : 0.0;
       x[q] = (newton && i < mt) ? -(u[q] - bc[q] - ch * f[q]) : 0.0;
-      if (newton && i < mt) L.A[a.S.nnzF + pivot(a, i)] = x[q];
+      if (newton && i < mt) lds_put<double>(L.cell + a.W.oR + 16 * pivot(a, i), x[q]);
     }
     if (newton) wave_sync();
   }
@@ -2238,24 +1717,22 @@ struct AerosolSparseBackend : AerosolLayout {
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
-      const int k = pivot(a, i);
-      x[q] = (i < a.X.mt) ? L.A[a.S.nnzF + k] * L.rdiag[k] : 0.0;
+      x[q] = 0.0;
+      if (i < a.X.mt) {
+        const vec2<double> v = lds_get<vec2<double>>(L.cell + a.W.oR + 16 * pivot(a, i));
+        x[q] = v.x * v.y;
+      }
     }
   }
-  static __device__ void back(const IntegratorArgs& a, const Lds& L, int lane) {
-    run_program(L.hdr + a.S.luRounds, L.body + a.S.backBody, a.S.backRounds, L.A, L.rdiag, a.X.mt, a.S.nnzF,
-                a.S.trashSlot, lane);
-  }
   static __device__ bool factor_solve(const IntegratorArgs& a, const Lds& L, int lane, double (&x)[QM], Fact&) {
-    if (!run_program(L.hdr, L.body, a.S.luRounds, L.A, L.rdiag, a.X.mt, a.S.nnzF, a.S.trashSlot, lane)) return false;
-    back(a, L, lane);
+    if (!sp_lu<SH>(L, L.w, a.W.oLuHdr, a.W.oLu, a.W.oLu1, a.W.nLu, lane)) return false;
+    sp_back<SH>(a.W, L, lane);
     get_x(a, L, lane, x);
     return true;
   }
   static __device__ void solve(const IntegratorArgs& a, const Lds& L, int lane, double (&x)[QM], const Fact&) {
-    run_program(L.hdr + a.S.luRounds + a.S.backRounds, L.body + a.S.fwdBody, a.S.fwdRounds, L.A, L.rdiag, a.X.mt,
-                a.S.nnzF, a.S.trashSlot, lane);
-    back(a, L, lane);
+    sp_lu<SH>(L, L.memory(), a.W.oFwdHdr, a.W.oFwd, a.W.oFwd1, a.W.nFwd, lane);
+    sp_back<SH>(a.W, L, lane);
     get_x(a, L, lane, x);
   }
 };
@@ -2294,6 +1771,17 @@ __global__ __launch_bounds__(64) void aerosol_rhs_kernel(IntegratorArgs a) {
 
 // Workgroup = cellsPerGroup wavefronts, one cell per wavefront at a time;
 // after staging, wavefronts never synchronise with each other.
+//
+// What bounds the sparse forms is each wavefront's chain of dependent LDS
+// rounds (a wavefront alone on its CU took 66 k cycles per CB05 Newton
+// iteration, sixteen took 76 k), not flops or bytes: the encoded programs
+// (lowered.hpp, sparse_exec.hpp) replaced an interpreter of the rounds that
+// decoded kind, length and indices per round and waited for scalar loads.
+// Measured, interpreter -> encoded: 131040 cells mixed, 80 TR-BDF2
+// iterations 305.2 -> 160.5 ms; 16411 cells FP64, 100 iterations 69.8 ->
+// 36.8 ms; one cell, 10 iterations 594 -> 309 us; E3SM 40960 cells to 1800 s
+// 63.6 -> 32.3 ms; CB05 + SOA, one particle, 8192 cells, 60 iterations 52.8
+// -> 33.7 ms (same bits).
 template <class B, int QM, int kThreads, bool REC>
 __global__ __launch_bounds__(kThreads) void trbdf2_kernel(IntegratorArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
@@ -2500,8 +1988,8 @@ __device__ __forceinline__ void store_vec(double* dst, int m, int lane, const do
 // One Newton solve of a stage, as the integrator runs it (same refresh
 // rule, convergence test and arithmetic).
 template <int QM>
-__device__ __forceinline__ void replay_newton(const IntegratorArgs& f, const SpLds<double>& L, int lane, double (&u)[QM],
-                              const double (&bc)[QM], double ch, int max_newton, int jint, double atol, double rtol) {
+__device__ __forceinline__ void replay_newton(const IntegratorArgs& f, const SpLds<double, false>& L, int lane,
+                              double (&u)[QM], const double (&bc)[QM], double ch, int max_newton, int jint, double atol, double rtol) {
   using B = SparseBackend<double, QM, false>;
   typename B::Fact fs;
   for (int nit = 0; nit < max_newton; ++nit) {
@@ -2513,58 +2001,64 @@ __device__ __forceinline__ void replay_newton(const IntegratorArgs& f, const SpL
     } else {
       B::solve(f, L, lane, x, fs);
     }
-    double nrm = 0.0;
+    bool over = false;
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
       if (i < f.M.m) {
         u[q] += x[q];
-        double w = fabs(x[q]) / (atol + rtol * fabs(u[q]));
-        if (!(w == w)) w = INFINITY;
-        nrm = fmax(nrm, w);
+        over |= !ratio_at_most_one(fabs(x[q]), atol + rtol * fabs(u[q]));
       }
     }
-    if (uniform_d(wave_max(nrm)) <= 1.0) return;
+    if (ballot(over) == 0) return;
   }
 }
 
 // Solves (I - ch J^T) mu = rhs at the Jacobian pairs in LDS; mu in registers
 // and in L.mu, w = nu . mu.  Returns false on a zero or non-finite pivot.
 template <int QM>
-__device__ __forceinline__ bool adjoint_solve(const AdjointArgs& a, const SpLds<double>& LT, int lane, double ch,
+__device__ __forceinline__ bool adjoint_solve(const AdjointArgs& a, const SpLds<double, false>& LT, int lane, double ch,
                               const double (&rhs)[QM], double (&mu)[QM]) {
-  const DevSparse& S = a.ST;
+  constexpr int SH = SparseBackend<double, QM, false>::SH;
+  const DevLowered& W = a.WT;
   const int m = a.fw.M.m;
-  eval_rounds<true>(LT, lane, S.ropRounds + S.pairRounds + S.segRounds, S.jacRounds, S.jacBody, 1.0, -ch);
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
     const int i = lane + kWave * q;
-    if (i < m) LT.A[S.nnzF + i] = rhs[q];
+    if (i < m) lds_put<double>(LT.cell + W.oR + 16 * i, rhs[q]);
   }
+  sp_jacobian<SH>(W, LT, lane, -ch);
   wave_sync();
-  const bool ok = run_program(LT.hdr, LT.body, S.luRounds, LT.A, LT.rdiag, m, S.nnzF, S.trashSlot, lane);
-  run_program(LT.hdr + S.luRounds, LT.body + S.backBody, S.backRounds, LT.A, LT.rdiag, m, S.nnzF, S.trashSlot, lane);
+  const bool ok = sp_lu<SH>(LT, LT.w, W.oLuHdr, W.oLu, W.oLu1, W.nLu, lane);
+  sp_back<SH>(W, LT, lane);
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
     const int i = lane + kWave * q;
-    mu[q] = i < m ? LT.A[S.nnzF + i] * LT.rdiag[i] : 0.0;
-    if (i < m) LT.mu[i] = mu[q];
+    mu[q] = 0.0;
+    if (i < m) {
+      const vec2<double> v = lds_get<vec2<double>>(LT.cell + W.oR + 16 * i);
+      mu[q] = v.x * v.y;
+      lds_put<double>(LT.cell + W.oMu + 8 * i, mu[q]);
+    }
   }
   wave_sync();
-  eval_rounds<true>(LT, lane, S.ropRounds + S.pairRounds + S.segRounds + S.jacRounds, S.nutRounds, S.nutBody, 0.0,
-                    0.0);
+  sp_sums<SH>(LT, W.oNutHdr, W.oNut, W.nNut, LT.coef, LT.cell + W.oW, lane);
   wave_sync();
   return ok;
 }
 
 // grad_r += c rop_r w_r
-__device__ __forceinline__ void accumulate_grad(const SpLds<double>& L, double* g, int nReac, int lane, double c) {
-  for (int r = lane; r < nReac; r += kWave) g[r] += c * L.rop[r] * L.w[r];
+__device__ __forceinline__ void accumulate_grad(const DevLowered& W, const SpLds<double, false>& L, double* g,
+                                                int nReac, int lane, double c) {
+  for (int r = lane; r < nReac; r += kWave)
+    g[r] += c * lds_get<double>(L.cell + W.oP + 8 * r) *
+            lds_get<double>(L.cell + L.w.template rec<unsigned>(W.oWmap, r / kWave, lane));
 }
 
 template <int QM>
-__device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double>& L, const SpLds<double>& LT, double* g,
-                             int cell, int lane) {
+__device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L, const SpLds<double, false>& LT,
+                             double* g, int cell, int lane) {
+  constexpr int SH = SparseBackend<double, QM, false>::SH;
   const IntegratorArgs& f = a.fw;
   const DevMech& M = f.M;
   const int m = M.m, nSpec = M.nSpec, nReac = M.nReac;
@@ -2601,6 +2095,7 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double>& L, const
     lam[q] = ai < m ? a.lambda_in[size_t(cell) * nSpec + M.perm()[ai]] : 0.0;
   }
   wave_sync();
+  sp_scaled_rates<SH>(f.W, L, nReac, lane);
 
   using B = SparseBackend<double, QM, false>;
   double* tr = a.traj + size_t(cell) * kTraj * m;
@@ -2643,31 +2138,34 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double>& L, const
       if (j == len - 1) {
         load_vec<QM>(tr + size_t(j + 1) * m, m, lane, u);
         B::put_c(f, L, lane, u);
-        sp_rates(a.ST, LT, lane, true);
+        sp_rates<SH>(a.WT, LT, lane, true);
         wave_sync();
       }
       ok &= adjoint_solve<QM>(a, LT, lane, c_bdf * h, lam, mu2);
-      accumulate_grad(LT, g, nReac, lane, c_bdf * h);
+      accumulate_grad(a.WT, LT, g, nReac, lane, c_bdf * h);
       load_vec<QM>(tr + size_t(kAdjointSegment + 1 + j) * m, m, lane, u);
       B::put_c(f, L, lane, u);
-      sp_rates(a.ST, LT, lane, true);
+      sp_rates<SH>(a.WT, LT, lane, true);
       wave_sync();
 #pragma unroll
       for (int q = 0; q < QM; ++q) rhs[q] = a_g * mu2[q];
       ok &= adjoint_solve<QM>(a, LT, lane, c_tr * h, rhs, mu1);
-      accumulate_grad(LT, g, nReac, lane, c_tr * h);
+      accumulate_grad(a.WT, LT, g, nReac, lane, c_tr * h);
       load_vec<QM>(tr + size_t(j) * m, m, lane, u);
       B::put_c(f, L, lane, u);
-      sp_rates(a.ST, LT, lane, true);
+      sp_rates<SH>(a.WT, LT, lane, true);
       wave_sync();
-      accumulate_grad(LT, g, nReac, lane, c_tr * h);
-      eval_rounds<true>(LT, lane, a.ST.ropRounds + a.ST.pairRounds + a.ST.segRounds + a.ST.jacRounds + a.ST.nutRounds,
-                        a.ST.jtvRounds, a.ST.jtvBody, 0.0, 0.0);
+      accumulate_grad(a.WT, LT, g, nReac, lane, c_tr * h);
+      sp_sums<SH>(LT, a.WT.oJtvHdr, a.WT.oJtv, a.WT.nJtv, LT.cell, LT.cell + a.WT.oV, lane);
       wave_sync();
 #pragma unroll
       for (int q = 0; q < QM; ++q) {
         const int i = lane + kWave * q;
-        lam[q] = i < m ? -a_n * mu2[q] + mu1[q] + c_tr * h * LT.v[i] : 0.0;
+        lam[q] = 0.0;
+        if (i < m) {
+          const double v = lds_get<double>(LT.cell + LT.w.template rec<unsigned>(a.WT.oVmap, q, lane));
+          lam[q] = -a_n * mu2[q] + mu1[q] + c_tr * h * v;
+        }
       }
       wave_sync();
     }
@@ -2682,37 +2180,26 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double>& L, const
   for (int r = lane; r < nReac; r += kWave) gout[r] = ok ? g[r] : NAN;
 }
 
-// One wavefront per cell, cells taken from a device work queue.
+// One wavefront per cell, cells taken from a device work queue.  Bound by the
+// same chain as trbdf2_kernel; gradient of 2000 CB05 cells over 1 ms of model
+// time, forward and backward: 583 ms with the rounds interpreted, 253 ms
+// encoded.
 template <int QM>
 __global__ __launch_bounds__(512) __attribute__((flatten)) void adjoint_kernel(AdjointArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const DevMech& M = a.fw.M;
-  SpLds<double> L = carve_sparse<double, false>(lds_raw, M, a.fw.S, a.cellBytes, wave);
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  char* x = reinterpret_cast<char*>(L.A) + sparseCellBytes(M, a.fw.S, sizeof(double));
-  L.mu = reinterpret_cast<double*>(x);
-  x += al(8 * size_t(M.m + 1));
-  L.w = reinterpret_cast<double*>(x);
-  x += al(8 * size_t(M.nReac + 2));
-  L.v = reinterpret_cast<double*>(x);
-  x += al(8 * size_t(M.m + 1));
-  double* g = reinterpret_cast<double*>(x);
-  SpLds<double> LT = L;
-  LT.hdr = reinterpret_cast<const unsigned*>(M.ib + a.ST.oProgHdr);
-  LT.body = reinterpret_cast<const unsigned*>(M.ib + a.ST.oProgBody);
-  LT.ehdr = reinterpret_cast<const unsigned*>(M.ib + a.ST.oEvalHdr);
-  LT.ebody = reinterpret_cast<const unsigned*>(M.ib + a.ST.oEvalBody);
-  LT.coef = M.db + a.ST.oCoef;
-  if (lane == 0) {
-    L.kf[M.nReac] = 0.0;
-    L.rop[M.nReac] = 0.0;
-    L.dpr[M.nPairs] = 0.0;
-    L.A[a.fw.S.zeroSlot] = 0.0;
-    L.rdiag[M.m] = 0.0;
-    L.mu[M.m] = 0.0;
-    L.w[M.nReac] = 0.0;
-  }
+  const unsigned* ib = reinterpret_cast<const unsigned*>(M.ib);
+  stage_sparse<false>(a.WT, nullptr, M.db + a.WT.oCoef, lds_raw);
+  __syncthreads();
+  // one cell region and coefficient table, two instruction streams
+  const SpLds<double, false> L = carve_sparse<double, false>(a.fw.W, ib + a.fw.W.oWords, 0, lds_raw, a.cellBytes, wave);
+  SpLds<double, false> LT = L;
+  LT.w.g = ib + a.WT.oWords;
+  double* g = reinterpret_cast<double*>(lds_raw + sparseStageBytes(a.WT, 0, false) +
+                                        size_t(wave) * size_t(a.cellBytes) + adjointRegionBytes(a.fw.W, a.WT));
+  sp_init(a.WT, L, M.m, lane);
+  if (lane == 0) lds_put<double>(L.cell + a.WT.oMu + 8 * M.m, 0.0);
   wave_sync();
   for (;;) {
     int cell = 0;
@@ -2862,6 +2349,8 @@ __global__ __launch_bounds__(64) void jacobian_kernel(DevMech M, int nBatch, con
 // ---- launchers (called from the C ABI) --------------------------------------
 
 static int qmOf(int m) { return m <= 64 ? 1 : (m <= 128 ? 2 : (m <= 256 ? 4 : 0)); }
+// instance of m unknowns whose encoded programs (sparse forms) hold shifted fields: those with QM 4
+static int qmOf(int m, const DevLowered* w) { return w && w->enabled && w->shift ? 4 : qmOf(m); }
 
 template <class B, int QM, int kThreads, bool REC = false>
 static const void* integratorFn() {
@@ -2928,7 +2417,7 @@ static const void* integratorKernel(int precision, int sparse, int qm, bool rec,
 }
 
 hipError_t launchIntegrator(const IntegratorArgs& a, int precision, int grid, size_t lds, hipStream_t stream) {
-  const int qm = qmOf(a.M.m);
+  const int qm = qmOf(a.M.m, a.sparse == 1 || a.sparse == 2 ? &a.W : nullptr);
   if (qm == 0) return hipErrorInvalidValue;
   const void* fn = integratorKernel(precision, a.sparse, qm, a.rec.h != nullptr, a.cellsPerGroup);
   if (!fn) return hipErrorInvalidValue;
@@ -2943,16 +2432,17 @@ hipError_t launchIntegrator(const IntegratorArgs& a, int precision, int grid, si
 }
 
 // static LDS of the integrator instance (profiling builds declare some)
-size_t integratorStaticLds(int precision, int sparse, int m) {
-  const int qm = qmOf(m);
+size_t integratorStaticLds(int precision, int sparse, int m, const DevLowered& w) {
+  const int qm = qmOf(m, &w);
   if (qm == 0) return 0;
   hipFuncAttributes attr;
   if (hipFuncGetAttributes(&attr, integratorKernel(precision, sparse, qm, false, 1)) != hipSuccess) return 0;
   return attr.sharedSizeBytes;
 }
 
-hipError_t integratorMaxBlocksPerCU(int precision, int sparse, int m, int threads, size_t lds, int* blocks, bool rec) {
-  const int qm = qmOf(m);
+hipError_t integratorMaxBlocksPerCU(int precision, int sparse, int m, const DevLowered& w, int threads, size_t lds,
+                                    int* blocks, bool rec) {
+  const int qm = qmOf(m, sparse == 1 || sparse == 2 ? &w : nullptr);
   if (qm == 0) return hipErrorInvalidValue;
   const void* fn = integratorKernel(precision, sparse, qm, rec, threads / 64);
   if (sparse == 3) threads = 256;
@@ -2970,11 +2460,11 @@ hipError_t launchRates(const DevMech& M, int nBatch, const double* state, const 
 }
 
 // ---- aerosol integrator launches (FP64 dense, mt <= 128 unknowns) ----
-static const void* aerosolKernel(int mt, bool sparse) {
+static const void* aerosolKernel(int mt, bool sparse, const DevLowered& w) {
   if (sparse) {
+    if (w.shift && mt <= 256) return integratorFn<AerosolSparseBackend<4>, 4, 512>();
     if (mt <= 64) return integratorFn<AerosolSparseBackend<1>, 1, 512>();
     if (mt <= 128) return integratorFn<AerosolSparseBackend<2>, 2, 512>();
-    if (mt <= 256) return integratorFn<AerosolSparseBackend<4>, 4, 512>();
     return nullptr;
   }
   if (mt <= 64) return integratorFn<AerosolBackend<1>, 1, 256>();
@@ -2993,7 +2483,7 @@ int aerosolCellsPerGroup(const DevMech& M, const DevAerosol& X, size_t maxLds) {
 
 hipError_t launchAerosol(const IntegratorArgs& a, int grid, size_t lds, hipStream_t stream) {
   const bool sparse = a.sparse != 0;
-  const void* fn = aerosolKernel(a.X.mt, sparse);
+  const void* fn = aerosolKernel(a.X.mt, sparse, a.W);
   if (!fn || a.cellsPerGroup < 1 || a.cellsPerGroup > (sparse ? 8 : 4)) return hipErrorInvalidValue;
   IntegratorArgs arg = a;
   void* params[] = {&arg};
@@ -3017,18 +2507,14 @@ static const void* adjointKernel(int qm) {
                             : reinterpret_cast<const void*>(&adjoint_kernel<4>));
 }
 
-size_t adjointCellBytes(const DevMech& M, const DevSparse& S) {
-  return sparseCellBytes(M, S, sizeof(double)) + adjointExtraBytes(M);
-}
-
-hipError_t adjointMaxBlocksPerCU(int m, int threads, size_t lds, int* blocks) {
-  const int qm = qmOf(m);
+hipError_t adjointMaxBlocksPerCU(int m, const DevLowered& w, int threads, size_t lds, int* blocks) {
+  const int qm = qmOf(m, &w);
   if (qm == 0) return hipErrorInvalidValue;
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, adjointKernel(qm), threads, lds);
 }
 
 hipError_t launchAdjoint(const AdjointArgs& a, int grid, size_t lds, hipStream_t stream) {
-  const int qm = qmOf(a.fw.M.m);
+  const int qm = qmOf(a.fw.M.m, &a.WT);
   if (qm == 0) return hipErrorInvalidValue;
   AdjointArgs arg = a;
   void* params[] = {&arg};

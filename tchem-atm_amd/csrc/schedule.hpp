@@ -6,10 +6,9 @@
 //
 // A program is a sequence of "rounds"; in a round each of the 64 lanes of
 // the wavefront executes one record.  A round is a header word
-// (len | kind << 16, read by the whole wavefront) and a body of 64-word
-// slots, slot s of lane l at body[64 * s + l], so every load of a round is
-// one conflict-free LDS access.  Both programs are copied into LDS once per
-// workgroup and read by every wavefront (cell) of the workgroup.
+// (len | kind << 16) and a body of 64-word slots, slot s of lane l at
+// body[64 * s + l].  The kernels run an encoding of these rounds (lowered.hpp)
+// that computes the same values in the same order.
 //
 // Per-cell matrix storage: the nnzF entries of the symbolic LU pattern F
 // (structure of I - J plus fill) in row-major order, the m right-hand-side
