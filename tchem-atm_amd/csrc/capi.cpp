@@ -13,6 +13,7 @@
 #include <cstring>
 #include <fstream>
 #include <memory>
+#include <numeric>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -49,15 +50,16 @@ hipError_t launchLoopControl(int n, const double* t_out, const tchem_time_advanc
 hipError_t adjointMaxBlocksPerCU(int m, const DevLowered& w, int threads, size_t lds, int* blocks);
 hipError_t launchAdjoint(const AdjointArgs& a, int grid, size_t lds, hipStream_t stream);
 hipError_t launchE3smKinetics(const DevE3sm& E, int mode, int nBatch, const double* state, const double* photo,
-                              int nPhoto, const double* ext, double* out, int ldOut, hipStream_t stream);
+                              int nPhoto, const double* ext, double* out, int ldOut, int numCUs, size_t maxLds,
+                              hipStream_t stream);
 hipError_t launchAdjointSetup(int nBatch, int maxSteps, const tchem_time_advance_t* tadv, const double* tol_newton,
                               int* header, double* tol, int* newton, hipStream_t stream);
 hipError_t launchUpdateTadv(int n, tchem_time_advance_t* tadv, const double* t_out, const double* dt_out, int* ctl,
                             hipStream_t stream);
 hipError_t launchSourceTerm(const DevMech& M, int nBatch, const double* state, const double* photo, const double* ext,
-                            double* omega, hipStream_t stream);
+                            double* omega, int numCUs, size_t maxLds, hipStream_t stream);
 hipError_t launchJacobian(const DevMech& M, int nBatch, const double* state, const double* photo, double* jac,
-                          hipStream_t stream);
+                          int numCUs, size_t maxLds, hipStream_t stream);
 }  // namespace tchem_amd
 
 using namespace tchem_amd;
@@ -580,6 +582,80 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
   d.oSerJPtr = addI(t.serJPtr);
   d.oSerJPair = addI(t.serJPair);
   d.oSerJCoef = addD(t.serJCoef);
+  // batch functions
+  auto byLength = [](const std::vector<int>& ptr) {  // rows of a CSR, longest first
+    std::vector<int> o(ptr.empty() ? 0 : ptr.size() - 1);
+    std::iota(o.begin(), o.end(), 0);
+    std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return ptr[x + 1] - ptr[x] > ptr[y + 1] - ptr[y]; });
+    return o;
+  };
+  // a CSR with rows padded to multiples of 4: padding on `item`, coefficient 0
+  auto padded = [](const std::vector<int>& ptr, const std::vector<int>& ix, const std::vector<double>& cf, int item,
+                   std::vector<int>* pPtr, std::vector<int>* pIx, std::vector<double>* pCf) {
+    pPtr->assign(1, 0);
+    for (size_t i = 0; i + 1 < ptr.size(); ++i) {
+      for (int e = ptr[i]; e < ptr[i + 1]; ++e) {
+        pIx->push_back(ix[size_t(e)]);
+        pCf->push_back(cf[size_t(e)]);
+      }
+      while (pIx->size() % 4) {
+        pIx->push_back(item);
+        pCf->push_back(0.0);
+      }
+      pPtr->push_back(int(pIx->size()));
+    }
+  };
+  {
+    const int one = 3 + t.nSpec;  // column after the row
+    auto factor = [&](int r, int j) {
+      const int sp = j < t.maxReactants ? t.reacSpec[size_t(r) * t.maxReactants + j] : -1;
+      if (sp < 0) return one | (1 << 16);
+      const int n = t.reacPow[size_t(r) * t.maxReactants + j];
+      return n < 1 ? one | (1 << 16) : (3 + (sp < t.m ? t.perm[size_t(sp)] : sp)) | (n << 16);
+    };
+    std::vector<int> order, fac, rec, cls[3];
+    for (int r = 0; r < t.nReac; ++r) {
+      const double* P = &t.ratePar[size_t(r) * 8];
+      const bool plain = t.rateKind[size_t(r)] == kRateArrhenius && P[1] == 0.0 && P[4] == 0.0;
+      cls[plain ? (P[2] == 0.0 ? 0 : 1) : 2].push_back(r);
+      for (int j = 0; j < t.maxReactants; ++j) fac.push_back(factor(r, j));
+      for (int p = t.pairPtr[r]; p < t.pairPtr[r + 1]; ++p) {
+        const int js = t.pairSlot[p];
+        std::vector<int> other;
+        for (int j = 0; j < std::max(3, t.maxReactants); ++j)
+          if (j != js) other.push_back(factor(r, j));
+        const int sp = t.reacSpec[size_t(r) * t.maxReactants + js];  // an active species
+        rec.insert(rec.end(), {r | (js << 24), (3 + t.perm[size_t(sp)]) | (t.reacPow[size_t(r) * t.maxReactants + js] << 16),
+                               other[0], other[1]});
+      }
+    }
+    for (const auto& v : cls) order.insert(order.end(), v.begin(), v.end());
+    order.push_back(int(cls[0].size()));
+    order.push_back(int(cls[0].size() + cls[1].size()));
+    d.oRateOrder = addI(order);
+    d.oReacFactor = addI(fac);
+    d.oPairRecord = addI(rec);
+    std::vector<int> pp, pi;
+    std::vector<double> pc;
+    padded(t.serOmegaPtr, t.serOmegaReac, t.serOmegaCoef, t.nReac, &pp, &pi, &pc);
+    d.oPadOmegaPtr = addI(pp);
+    d.oPadOmegaReac = addI(pi);
+    d.oPadOmegaCoef = addD(pc);
+    std::vector<int> jp, ji;
+    std::vector<double> jc;
+    padded(t.serJPtr, t.serJPair, t.serJCoef, t.nPairs(), &jp, &ji, &jc);
+    d.oPadJPtr = addI(jp);
+    d.oPadJPair = addI(ji);
+    d.oPadJCoef = addD(jc);
+    std::vector<int> map((size_t(t.m) * t.m + 1) / 2, 0);
+    if (t.nSerJ() < 0xffff)
+      for (int n = 0; n < t.nSerJ(); ++n) {
+        const size_t at = size_t(t.perm[size_t(t.serJRow[n])]) * t.m + t.perm[size_t(t.serJCol[n])];
+        map[at / 2] = int(unsigned(map[at / 2]) | (unsigned(1 + n) << (16 * (at % 2))));
+      }
+    d.oOmegaOrder = addI(byLength(t.serOmegaPtr));
+    d.oJacMap = addI(map);
+  }
   d.oMfjQuarter = d.oMfjTermW = d.oMfjTermC = 0;
   if (t.m <= 255 && t.nPairs() < (1 << 14)) {
     // the MFMA form's assembly lists: the structural entries of each column
@@ -689,7 +765,13 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
       ri.push_back(j.reaction);
       rp.insert(rp.end(), {j.k0_A, j.k0_B, j.k0_C, j.kinf_A, j.kinf_B, j.kinf_C, j.Fc, j.A, j.B, j.C});
     }
-    for (const auto& a : km.adjustReaction) adj.insert(adj.end(), {a.reaction, a.species});
+    std::vector<std::vector<int>> adjOf(static_cast<size_t>(km.nReac));
+    for (const auto& a : km.adjustReaction) adjOf[size_t(a.reaction)].push_back(a.species);
+    std::vector<int> adjPtr(1, 0);
+    for (const auto& v : adjOf) {
+      adj.insert(adj.end(), v.begin(), v.end());
+      adjPtr.push_back(int(adj.size()));
+    }
     for (const auto& o : km.prodO1D) {
       pI.insert(pI.end(), {o.reactions[0], o.reactions[1], o.reactions[2], o.photolysis_reaction, o.species1,
                            o.species2, o.species3});
@@ -700,7 +782,6 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
     E.nCmaq = int(ci.size());
     E.nJpl = int(ji.size());
     E.nRJpl = int(ri.size());
-    E.nAdjust = int(km.adjustReaction.size());
     E.nProd = int(km.prodO1D.size());
     E.oArrIdx = addI(ai);
     E.oArrPar = addD(ap);
@@ -712,14 +793,46 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
     E.oJplPar = addD(jp);
     E.oRJplIdx = addI(ri);
     E.oRJplPar = addD(rp);
-    E.oAdjust = addI(adj);
+    E.oAdjPtr = addI(adjPtr);
+    E.oAdjSpec = addI(adj);
+    std::vector<char> formed(static_cast<size_t>(km.nReac), 0);
+    for (const std::vector<int>* v : {&ai, &ti, &ci, &ji, &ri})
+      for (int r : *v) formed[size_t(r)] = 1;
+    std::vector<int> given;
+    for (int r = 0; r < km.nReac; ++r)
+      if (!formed[size_t(r)]) given.push_back(r);
+    E.nGiven = int(given.size());
+    E.oGiven = addI(given);
     E.oProdI = addI(pI);
     E.oProdD = addD(pD);
     E.oConvExp = addI(km.convExponent);
     E.oNreac = addI(km.reacNreac);
-    E.oNprod = addI(km.reacNprod);
     E.oSidx = addI(km.reacSidx);
     E.oNuki = addD(km.reacNuki);
+    const int ma = km.nActive(), joff = km.maxSpecInReac / 2;
+    std::vector<std::vector<std::pair<int, double>>> net(static_cast<size_t>(ma));
+    for (int r = 0; r < km.nReac; ++r) {
+      for (int j = 0; j < km.reacNreac[r]; ++j)
+        if (km.sidx(r, j) < ma) net[size_t(km.sidx(r, j))].push_back({r, km.nuki(r, j)});
+      for (int j = 0; j < km.reacNprod[r]; ++j)
+        if (km.sidx(r, j + joff) < ma) net[size_t(km.sidx(r, j + joff))].push_back({r, km.nuki(r, j + joff)});
+    }
+    std::vector<int> ptr(1, 0), reac;
+    std::vector<double> coefs;
+    for (const auto& v : net) {
+      for (const auto& e : v) {
+        reac.push_back(e.first);
+        coefs.push_back(e.second);
+      }
+      ptr.push_back(int(reac.size()));
+    }
+    std::vector<int> pp, pi;
+    std::vector<double> pc;
+    padded(ptr, reac, coefs, km.nReac, &pp, &pi, &pc);
+    E.oNetPtr = addI(pp);
+    E.oNetReac = addI(pi);
+    E.oNetCoef = addD(pc);
+    E.oNetOrder = addI(byLength(ptr));
   }
   ib.push_back(0);
   db.push_back(0.0);
@@ -892,7 +1005,7 @@ int tchem_atmchem_e3sm_run_device_batch(const tchem_atmchem_options_t* opts, int
   // rate constants from the E3SM kinetics (constant over the interval: they
   // depend on T, p, the photolysis rates and constant species only)
   hipError_t e = launchE3smKinetics(kmcd->e3, 3, nBatch, state, nPhotoRates ? photo_rates : nullptr, nPhotoRates,
-                                    nullptr, kmcd->kf, kmcd->e3.nReac, s);
+                                    nullptr, kmcd->kf, kmcd->e3.nReac, kmcd->numCUs, kmcd->maxLds, s);
   if (e != hipSuccess) return hipFail(e, "e3sm_kinetics_kernel launch");
   IntegratorArgs a{};
   a.nBatch = nBatch;
@@ -928,8 +1041,8 @@ int tchem_sourceterm_run_device_batch(int nBatch, const double* state, const dou
   if (nBatch == 0) return TCHEM_OK;
   if (!state || !omega) return setError(TCHEM_ERR_INVALID, "sourceterm: null device array");
   if (kmcd->dev.nPhoto == 0) photo_rates = nullptr;
-  hipError_t e = launchSourceTerm(kmcd->dev, nBatch, state, photo_rates, external_sources, omega,
-                                  static_cast<hipStream_t>(stream));
+  hipError_t e = launchSourceTerm(kmcd->dev, nBatch, state, photo_rates, external_sources, omega, kmcd->numCUs,
+                                  kmcd->maxLds, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hipFail(e, "sourceterm_kernel launch");
   return TCHEM_OK;
 }
@@ -945,7 +1058,8 @@ int tchem_jacobian_run_device_batch(int nBatch, const double* state, const doubl
   if (kmcd->dev.nPhoto == 0) photo_rates = nullptr;
   const size_t lds = integratorLdsBytes(kmcd->dev, sizeof(double));
   if (lds > kmcd->maxLds) return setError(TCHEM_ERR_UNSUPPORTED, "jacobian: mechanism too large for LDS");
-  hipError_t e = launchJacobian(kmcd->dev, nBatch, state, photo_rates, jac, static_cast<hipStream_t>(stream));
+  hipError_t e = launchJacobian(kmcd->dev, nBatch, state, photo_rates, jac, kmcd->numCUs, kmcd->maxLds,
+                                static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hipFail(e, "jacobian_kernel launch");
   return TCHEM_OK;
 }
@@ -1426,7 +1540,7 @@ int runE3sm(const char* who, int mode, int nBatch, const double* state, const do
   if (hipGetDevice(&cur) != hipSuccess || cur != kmcd->device)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": kmcd belongs to another device");
   hipError_t e = launchE3smKinetics(E, mode, nBatch, state, nPhoto ? photo : nullptr, nPhoto, ext, out, ldOut,
-                                    static_cast<hipStream_t>(stream));
+                                    kmcd->numCUs, kmcd->maxLds, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hipFail(e, "e3sm_kinetics_kernel launch");
   return TCHEM_OK;
 }

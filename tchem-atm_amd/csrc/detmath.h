@@ -45,11 +45,12 @@ TCHEM_DM_FN double tchem_exp(double x) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
-  if (!(x == x)) return x;
-  if (x > 709.782712893384) return HUGE_VAL;
-  if (x < -745.1332191019412) return 0.0;
-  const double k = rint(x * TCHEM_DM_INV_LN2);
-  const double r = (x - k * TCHEM_DM_LN2_HI) - k * TCHEM_DM_LN2_LO;
+  /* the special cases are selected at the end, without a branch, so that
+     independent exponentials can overlap */
+  const int over = x > 709.782712893384, under = x < -745.1332191019412, nan = !(x == x);
+  const double y = (over || under || nan) ? 0.0 : x;
+  const double k = rint(y * TCHEM_DM_INV_LN2);
+  const double r = (y - k * TCHEM_DM_LN2_HI) - k * TCHEM_DM_LN2_LO;
   double p = 1.6059043836821613e-10; /* 1/13! */
   p = fma(p, r, 2.08767569878681e-09);
   p = fma(p, r, 2.505210838544172e-08);
@@ -64,7 +65,8 @@ TCHEM_DM_FN double tchem_exp(double x) {
   p = fma(p, r, 0.5);
   p = fma(p, r, 1.0);
   p = fma(p, r, 1.0);
-  return ldexp(p, (int)k);
+  const double e = ldexp(p, (int)k);
+  return nan ? x : (over ? HUGE_VAL : (under ? 0.0 : e));
 }
 
 TCHEM_DM_FN double tchem_log(double x) {

@@ -20,6 +20,8 @@ struct DevMech {
   const double* db;
   int oPerm, oRateKind, oConvExp, oPhotoSlot, oReacSpec, oReacPow, oPairPtr, oPairSlot, oJnzRowCol, oJnzPtr, oJcPair,
       oSerOmegaPtr, oSerOmegaReac, oSerJRowCol, oSerJPtr, oSerJPair;
+  int oRateOrder, oReacFactor, oPairRecord, oPadOmegaPtr, oPadOmegaReac, oPadOmegaCoef, oPadJPtr, oPadJPair, oPadJCoef,
+      oOmegaOrder, oJacMap;
   int oRatePar, oEmission, oJcCoef, oSerOmegaCoef, oSerJCoef;
   // the serial Jacobian lists regrouped for the MFMA form's assembly
   // (m <= 255 only; offsets 0 otherwise): per column quarter, each of the
@@ -49,6 +51,26 @@ struct DevMech {
   __host__ __device__ const int* serJPtr() const { return ib + oSerJPtr; }           // [nSerJ+1]
   __host__ __device__ const int* serJPair() const { return ib + oSerJPair; }         // [nSerContrib]
   __host__ __device__ const double* serJCoef() const { return db + oSerJCoef; }
+  // batch functions.  rateOrder: reactions by class of rate constant, then
+  // the ends of the first two classes; reacFactor: [nReac][maxR] state row
+  // column | power << 16 (absent: the column after the row, power 1);
+  // pairRecord: reaction | slot << 24, column | n_s << 16, the first two other
+  // factors; padded
+  // serial lists (multiples of 4, padding on the item after the last, with
+  // coefficient 0); species by descending length of their list; and for every
+  // dense Jacobian position (reference order, row-major, two to a word) 1 +
+  // its serial entry, 0 where there is none
+  __host__ __device__ const int* rateOrder() const { return ib + oRateOrder; }    // [nReac + 2]
+  __host__ __device__ const int* reacFactor() const { return ib + oReacFactor; }
+  __host__ __device__ const int4* pairRecord() const { return reinterpret_cast<const int4*>(ib + oPairRecord); }
+  __host__ __device__ const int* padOmegaPtr() const { return ib + oPadOmegaPtr; }
+  __host__ __device__ const int* padOmegaReac() const { return ib + oPadOmegaReac; }
+  __host__ __device__ const double* padOmegaCoef() const { return db + oPadOmegaCoef; }
+  __host__ __device__ const int* padJPtr() const { return ib + oPadJPtr; }
+  __host__ __device__ const int* padJPair() const { return ib + oPadJPair; }
+  __host__ __device__ const double* padJCoef() const { return db + oPadJCoef; }
+  __host__ __device__ const int* omegaOrder() const { return ib + oOmegaOrder; }  // [m]
+  __host__ __device__ const unsigned* jacMap() const { return reinterpret_cast<const unsigned*>(ib + oJacMap); }
   __host__ __device__ const int* mfjQuarter() const { return ib + oMfjQuarter; }  // [5] first term row of each quarter
   // [rows][256] term words: derivative pair (bits 0-13), stage index of the
   // entry (bits 14-28, on its last term), diagonal entry (bit 29), last
@@ -171,15 +193,21 @@ struct DevE3sm {
   const double* db;
   int nSpec, nConst, nReac, maxSpec, M_index;
   double convPPM;
-  int nArr, nTroe, nCmaq, nJpl, nRJpl, nAdjust, nProd;
+  int nArr, nTroe, nCmaq, nJpl, nRJpl, nProd;
   int oArrIdx, oArrPar;      // [nArr], [nArr][5] A B C D E
   int oTroeIdx, oTroePar;    // [nTroe], [nTroe][8] k0_A(x1e6) k0_B k0_C kinf_A kinf_B kinf_C Fc N
   int oCmaqIdx, oCmaqPar;    // [nCmaq], [nCmaq][6] A1 B1 C1 A2(x1e6) B2 C2
   int oJplIdx, oJplPar;      // [nJpl], [nJpl][7] k0_A k0_B k0_C kinf_A kinf_B kinf_C Fc
   int oRJplIdx, oRJplPar;    // [nRJpl], [nRJpl][10] + A B C
-  int oAdjust;               // [nAdjust][2] reaction, species
+  int oAdjPtr, oAdjSpec;     // [nReac + 1], [nAdjust] species a reaction's rate constant is multiplied with
+  int nGiven, oGiven;        // reactions without a rate form
   int oProdI, oProdD;        // [nProd][7] reactions[3], photolysis reaction, species 1-3; [nProd][6] A1 C1 A2 C2 A3 C3
-  int oConvExp, oNreac, oNprod, oSidx, oNuki;  // per reaction; [nReac][maxSpec]
+  int oConvExp, oNreac, oSidx, oNuki;  // per reaction; [nReac][maxSpec]
+  // net production rates, per active species: its entries in the order of
+  // the reference's loops (reaction order; reactants, then products), padded
+  // to multiples of 4 with coefficient 0 on item nReac, and the species by
+  // descending length of their list
+  int oNetPtr, oNetReac, oNetCoef, oNetOrder;
 };
 
 // Arguments of the discrete adjoint kernel (backward sweep over a record).

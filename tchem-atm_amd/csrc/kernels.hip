@@ -157,14 +157,6 @@ __device__ CellLds<TA> carve(char* base, const DevMech& M, bool withMatrix = tru
   return L;
 }
 
-template <typename TA>
-__device__ void load_rate_constants(const DevMech& M, const CellLds<TA>& L, int lane, double T, double p,
-                                    const double* photo) {
-  const double t_1 = 1.0 / T;
-  const double conv = M.convPPM * p * t_1;
-  for (int r = lane; r < M.nReac; r += kWave) L.kf[r] = rate_constant(M, r, T, p, t_1, conv, photo);
-}
-
 // rate of progress of reaction r at the concentrations in LDS
 __device__ __forceinline__ double rate_of_progress(const DevMech& M, const double* c, const double* kf, int r) {
   double v = kf[r];
@@ -1828,125 +1820,6 @@ __global__ __launch_bounds__(256) void rates_kernel(DevMech M, int nBatch, const
   kf[idx] = lscale ? k * tchem_exp(lscale[size_t(cell) * lstride + r]) : k;
 }
 
-// ---- E3SM / UCI kinetics batch functions --------------------------------------
-// ReactionRates / RateofProgress / NetProductionRates of the reference's
-// E3SM kinetics (src/core/impl/TChem_Impl_{KForward,KForwardJPL,AdjustReactions,
-// RateofProgress,NetProductionRates}.hpp), one wavefront per cell:
-//   mode 0: kf   (ReactionRates)
-//   mode 1: rop  (RateofProgress; photolysis rates replace kf of the first nPhoto reactions)
-//   mode 2: omega of the active species (NetProductionRates: external sources + nu . rop)
-//   mode 3: kf with the photolysis rates applied (the box model's rate constants)
-// Species concentrations are the state row's species block (active then constant).
-
-__device__ __forceinline__ double t300_pow(double T, double B) { return B == 0.0 ? 1.0 : pow(T / 300.0, B); }
-__device__ __forceinline__ double exp_or_one(double C, double t_1) { return C == 0.0 ? 1.0 : exp(C * t_1); }
-
-__global__ __launch_bounds__(64) void e3sm_kinetics_kernel(DevE3sm E, int mode, int nBatch, const double* state,
-                                                         const double* photo, int nPhoto, const double* ext,
-                                                         double* out, int ldOut) {
-  extern __shared__ __align__(16) char lds_raw[];
-  const int cell = blockIdx.x, lane = threadIdx.x;
-  if (cell >= nBatch) return;
-  double* x = reinterpret_cast<double*>(lds_raw);  // [nSpec]
-  double* kf = x + E.nSpec;                         // [nReac]
-  double* rop = kf + E.nReac;                       // [nReac]
-  double* om = rop + E.nReac;                       // [m]
-  const int m = E.nSpec - E.nConst;
-  const double* row = state + size_t(cell) * (E.nSpec + 3);
-  const double p = row[1], T = row[2];
-  const double t_1 = 1.0 / T;
-  const double conv = E.convPPM * p * t_1;
-  for (int i = lane; i < E.nSpec; i += kWave) x[i] = row[3 + i];
-  for (int r = lane; r < E.nReac; r += kWave)
-    kf[r] = (mode >= 1 && photo && r < nPhoto) ? photo[size_t(cell) * nPhoto + r] : 0.0;
-  wave_sync();
-  const int* ib = E.ib;
-  const double* db = E.db;
-  // KForward (TChem_Impl_KForward.hpp:52-141): Arrhenius and Troe without the
-  // conv factor, CMAQ_H2O2 with it
-  for (int i = lane; i < E.nArr; i += kWave) {
-    const double* P = db + E.oArrPar + 5 * i;
-    kf[ib[E.oArrIdx + i]] = P[0] * exp(P[2] * t_1) * (P[1] == 0.0 ? 1.0 : pow(T / P[3], P[1])) *
-                            (P[4] == 0.0 ? 1.0 : (1.0 + P[4] * p));
-  }
-  for (int i = lane; i < E.nTroe; i += kWave) {
-    const double* P = db + E.oTroePar + 8 * i;
-    const double k0 = P[0] * exp_or_one(P[2], t_1) * t300_pow(T, P[1]);
-    const double k0_kinf = k0 / (P[3] * exp_or_one(P[5], t_1) * t300_pow(T, P[4]));
-    kf[ib[E.oTroeIdx + i]] = k0 / (1.0 + k0_kinf) * pow(P[6], 1.0 / (1.0 + pow(log10(k0_kinf) / P[7], 2.0)));
-  }
-  for (int i = lane; i < E.nCmaq; i += kWave) {
-    const double* P = db + E.oCmaqPar + 6 * i;
-    const int r = ib[E.oCmaqIdx + i];
-    kf[r] = (P[0] * exp(P[2] * t_1) * t300_pow(T, P[1]) + P[3] * exp(P[5] * t_1) * t300_pow(T, P[4]) * conv) *
-            pow(conv, double(ib[E.oConvExp + r]));
-  }
-  // KForwardJPL (TChem_Impl_KForwardJPL.hpp:44-143), m = [M]
-  const double mM = E.M_index >= 0 ? x[E.M_index] : 0.0;
-  for (int i = lane; i < E.nJpl + E.nRJpl; i += kWave) {
-    const bool rj = i >= E.nJpl;
-    const int j = rj ? i - E.nJpl : i;
-    const double* P = db + (rj ? E.oRJplPar + 10 * j : E.oJplPar + 7 * j);
-    const double k0 = P[0] * exp_or_one(P[2], t_1) * t300_pow(T, P[1]);
-    const double kinf = P[3] * exp_or_one(P[5], t_1) * t300_pow(T, P[4]);
-    const double xpo = k0 * mM / kinf;
-    const double lx = log10(xpo);
-    const double factor = P[6] == 1.0 ? 1.0 : pow(P[6], 1.0 / (1.0 + lx * lx));
-    double k = k0 / (1.0 + xpo) * factor;
-    if (rj) k /= P[7] * exp_or_one(P[9], t_1) * t300_pow(T, P[8]);
-    kf[ib[(rj ? E.oRJplIdx : E.oJplIdx) + j]] = k;
-  }
-  wave_sync();
-  // AdjustReactions (TChem_Impl_AdjustReactions.hpp:52-96), in list order
-  if (lane == 0) {
-    for (int i = 0; i < E.nAdjust; ++i) kf[ib[E.oAdjust + 2 * i]] *= x[ib[E.oAdjust + 2 * i + 1]];
-    for (int i = 0; i < E.nProd; ++i) {
-      const int* I = ib + E.oProdI + 7 * i;
-      const double* P = db + E.oProdD + 6 * i;
-      const double fc = P[0] * exp(P[1] * t_1) * x[I[4]] + P[2] * exp(P[3] * t_1) * x[I[5]] +
-                        P[4] * exp(P[5] * t_1) * x[I[6]];
-      for (int k = 0; k < 3; ++k) kf[I[k]] *= kf[I[3]] / fc;
-    }
-  }
-  wave_sync();
-  double* o = out + size_t(cell) * ldOut;
-  if (mode == 0 || mode == 3) {
-    for (int r = lane; r < E.nReac; r += kWave) o[r] = kf[r];
-    return;
-  }
-  // RateofProgress (TChem_Impl_RateofProgress.hpp:73-87)
-  for (int r = lane; r < E.nReac; r += kWave) {
-    double v = kf[r];
-    for (int j = 0; j < ib[E.oNreac + r]; ++j)
-      v *= pow(x[ib[E.oSidx + r * E.maxSpec + j]], double(abs(int(db[E.oNuki + r * E.maxSpec + j]))));
-    rop[r] = v;
-  }
-  wave_sync();
-  if (mode == 1) {
-    for (int r = lane; r < E.nReac; r += kWave) o[r] = rop[r];
-    return;
-  }
-  // NetProductionRates (TChem_Impl_NetProductionRates.hpp:60-104): external
-  // sources, then nu . rop over active species in reaction order
-  for (int a = lane; a < m; a += kWave) om[a] = ext ? ext[size_t(cell) * m + a] : 0.0;
-  wave_sync();
-  if (lane == 0) {
-    const int joff = E.maxSpec / 2;
-    for (int r = 0; r < E.nReac; ++r) {
-      for (int j = 0; j < ib[E.oNreac + r]; ++j) {
-        const int k = ib[E.oSidx + r * E.maxSpec + j];
-        if (k < m) om[k] += db[E.oNuki + r * E.maxSpec + j] * rop[r];
-      }
-      for (int j = 0; j < ib[E.oNprod + r]; ++j) {
-        const int k = ib[E.oSidx + r * E.maxSpec + j + joff];
-        if (k < m) om[k] += db[E.oNuki + r * E.maxSpec + j + joff] * rop[r];
-      }
-    }
-  }
-  wave_sync();
-  for (int a = lane; a < ldOut; a += kWave) o[a] = a < m ? om[a] : 0.0;
-}
-
 // ---- discrete adjoint --------------------------------------------------------
 // Reverse-mode derivative of the recorded TR-BDF2 trajectory (accepted steps
 // only, step sizes held fixed) with respect to the initial active species
@@ -2297,54 +2170,12 @@ __global__ void update_tadv_kernel(int n, tchem_time_advance_t* tadv, const doub
   }
 }
 
-template <typename TA>
-__device__ void load_concentrations(const DevMech& M, const CellLds<TA>& L, int lane, const double* row) {
-  for (int a = lane; a < M.m; a += kWave) L.c[a] = row[3 + M.perm()[a]];
-  for (int i = M.m + lane; i < M.nSpec; i += kWave) L.c[i] = row[3 + i];
-}
-
-// Source term per cell (one wavefront per cell), reference species order.
-template <int QM>
-__global__ __launch_bounds__(64) void sourceterm_kernel(DevMech M, int nBatch, const double* state,
-                                                        const double* photo, const double* ext, double* omega) {
-  extern __shared__ __align__(16) char lds_raw[];
-  const CellLds<double> L = carve<double>(lds_raw, M, false);  // no matrix region
-  const int lane = threadIdx.x, cell = blockIdx.x;
-  if (cell >= nBatch) return;
-  const double* row = state + size_t(cell) * (M.nSpec + 3);
-  load_rate_constants(M, L, lane, row[2], row[1], photo ? photo + size_t(cell) * M.nPhoto : nullptr);
-  load_concentrations(M, L, lane, row);
-  wave_sync();
-  double f[QM];
-  source_term_from_lds<QM>(M, L, lane, f);
-#pragma unroll
-  for (int q = 0; q < QM; ++q) {
-    const int a = lane + kWave * q;
-    if (a < M.m) {
-      const size_t o = size_t(cell) * M.m + M.perm()[a];
-      omega[o] = f[q] + (ext ? ext[o] : 0.0);
-    }
-  }
-}
-
-// Jacobian per cell: assembled in LDS in reference order, written out coalesced.
-__global__ __launch_bounds__(64) void jacobian_kernel(DevMech M, int nBatch, const double* state, const double* photo,
-                                                      double* jac) {
-  extern __shared__ __align__(16) char lds_raw[];
-  const CellLds<double> L = carve<double>(lds_raw, M);
-  const int lane = threadIdx.x, cell = blockIdx.x;
-  if (cell >= nBatch) return;
-  const double* row = state + size_t(cell) * (M.nSpec + 3);
-  load_rate_constants(M, L, lane, row[2], row[1], photo ? photo + size_t(cell) * M.nPhoto : nullptr);
-  load_concentrations(M, L, lane, row);
-  wave_sync();
-  assemble_jacobian_from_lds(M, L, lane, 0.0, 1.0, true);
-  const int total = M.m * M.m;
-  double* out = jac + size_t(cell) * total;
-  for (int idx = lane; idx < total; idx += kWave) out[idx] = L.A[idx];
-}
-
 }  // namespace
+}  // namespace tchem_amd
+
+#include "batch_kernels.hpp"
+
+namespace tchem_amd {
 
 // ---- launchers (called from the C ABI) --------------------------------------
 
@@ -2529,12 +2360,38 @@ hipError_t launchAdjointSetup(int nBatch, int maxSteps, const tchem_time_advance
   return hipGetLastError();
 }
 
+// Cells per workgroup of the source term and the E3SM kinetics.  64 keeps a
+// wavefront on one reaction and has the highest throughput once its groups
+// (one per CU) cover most of the chip; below, 16 and then 4 spread the batch.
+// Measured us with 64 / 16 / 4 cells, source term: 131040 cells 188 / 292 /
+// 493, 16411: 43 / 47 / 64, 8192: 24 / 21 / 33, 4096: 23 / 18 / 17, 1: 22 /
+// 16 / 14; net production rates: 181 / 219 / 335, 41 / 38 / 48, 22 / 17 / 24,
+// 22 / 14 / 13, 19 / 14 / 13.  Fewer where the LDS does not hold as many (0:
+// not even one).  bytes(C): LDS of a workgroup.
+template <class Bytes>
+static int cellsPerGroup(int nBatch, int numCUs, size_t maxLds, Bytes bytes) {
+  if (nBatch > 40 * (long long)numCUs && bytes(64) <= maxLds) return 64;
+  if (nBatch > 12 * (long long)numCUs && bytes(16) <= maxLds) return 16;
+  return bytes(4) <= maxLds ? 4 : (bytes(1) <= maxLds ? 1 : 0);
+}
+
+size_t e3smGroupBytes(const DevE3sm& E, int C) {
+  return sizeof(double) * (size_t(C) * oddStride(E.nSpec + 3) + size_t(E.nReac + 1) * oddStride(C));
+}
 hipError_t launchE3smKinetics(const DevE3sm& E, int mode, int nBatch, const double* state, const double* photo,
-                              int nPhoto, const double* ext, double* out, int ldOut, hipStream_t stream) {
+                              int nPhoto, const double* ext, double* out, int ldOut, int numCUs, size_t maxLds,
+                              hipStream_t stream) {
   if (nBatch <= 0) return hipSuccess;
-  const size_t lds = sizeof(double) * (size_t(E.nSpec) + 2 * size_t(E.nReac) + size_t(E.nSpec - E.nConst));
-  hipLaunchKernelGGL(e3sm_kinetics_kernel, dim3(nBatch), dim3(64), lds, stream, E, mode, nBatch, state, photo, nPhoto,
-                     ext, out, ldOut);
+  const int C = cellsPerGroup(nBatch, numCUs, maxLds, [&](int c) { return e3smGroupBytes(E, c); });
+#define TCHEM_E3SM(c)                                                                                             \
+  hipLaunchKernelGGL(e3sm_kinetics_kernel<c>, dim3((nBatch + c - 1) / c), dim3(groupThreads(c)),                  \
+                     e3smGroupBytes(E, c), stream, E, mode, nBatch, state, photo, nPhoto, ext, out, ldOut)
+  if (C == 64) TCHEM_E3SM(64);
+  else if (C == 16) TCHEM_E3SM(16);
+  else if (C == 4) TCHEM_E3SM(4);
+  else if (C == 1) TCHEM_E3SM(1);
+  else return hipErrorInvalidConfiguration;
+#undef TCHEM_E3SM
   return hipGetLastError();
 }
 
@@ -2575,14 +2432,21 @@ hipError_t launchLoopControl(int n, const double* t_out, const tchem_time_advanc
 }
 
 hipError_t launchSourceTerm(const DevMech& M, int nBatch, const double* state, const double* photo, const double* ext,
-                            double* omega, hipStream_t stream) {
-  const int qm = qmOf(M.m);
-  if (qm == 0) return hipErrorInvalidValue;
+                            double* omega, int numCUs, size_t maxLds, hipStream_t stream) {
   if (nBatch <= 0) return hipSuccess;
-  const size_t lds = integratorLdsBytes(M, 0);
-  if (qm == 1) hipLaunchKernelGGL(sourceterm_kernel<1>, dim3(nBatch), dim3(64), lds, stream, M, nBatch, state, photo, ext, omega);
-  else if (qm == 2) hipLaunchKernelGGL(sourceterm_kernel<2>, dim3(nBatch), dim3(64), lds, stream, M, nBatch, state, photo, ext, omega);
-  else hipLaunchKernelGGL(sourceterm_kernel<4>, dim3(nBatch), dim3(64), lds, stream, M, nBatch, state, photo, ext, omega);
+  auto bytes = [&](int c) {
+    return sizeof(double) * (size_t(c) * oddStride(M.nSpec + 4) + size_t(M.nReac + 1) * oddStride(c));
+  };
+  const int C = cellsPerGroup(nBatch, numCUs, maxLds, bytes);
+#define TCHEM_SOURCE(c)                                                                                         \
+  hipLaunchKernelGGL(sourceterm_kernel<c>, dim3((nBatch + c - 1) / c), dim3(groupThreads(c)), bytes(c), stream, \
+                     M, nBatch, state, photo, ext, omega)
+  if (C == 64) TCHEM_SOURCE(64);
+  else if (C == 16) TCHEM_SOURCE(16);
+  else if (C == 4) TCHEM_SOURCE(4);
+  else if (C == 1) TCHEM_SOURCE(1);
+  else return hipErrorInvalidConfiguration;
+#undef TCHEM_SOURCE
   return hipGetLastError();
 }
 
@@ -2627,10 +2491,29 @@ hipError_t launchDenseMfmaSolve(int n, int nBatch, const double* A, const double
 }
 
 hipError_t launchJacobian(const DevMech& M, int nBatch, const double* state, const double* photo, double* jac,
-                          hipStream_t stream) {
+                          int numCUs, size_t maxLds, hipStream_t stream) {
   if (nBatch <= 0) return hipSuccess;
-  const size_t lds = integratorLdsBytes(M, sizeof(double));
-  hipLaunchKernelGGL(jacobian_kernel, dim3(nBatch), dim3(64), lds, stream, M, nBatch, state, photo, jac);
+  auto bytes = [&](int c) {
+    const size_t inner = size_t(c) * oddStride(M.nSpec + 4) + size_t(M.nReac) * oddStride(c);
+    const size_t list = size_t(1 + M.nSerJ) * oddStride(c);
+    return sizeof(double) * (size_t(M.nPairs + 1) * oddStride(c) + (inner > list ? inner : list));
+  };
+  // 4 cells (two groups to a CU, one stores while the other computes) or 16,
+  // which compute faster and win where one group per CU takes the whole batch:
+  // 4096 cells 54 us against 67, but 2000: 48 against 36, 16411: 272 against 242
+  int C = nBatch > 10 * (long long)numCUs && nBatch <= 16 * (long long)numCUs ? 16 : 4;
+  while (C > 1 && bytes(C) > maxLds) C /= 4;
+  if (bytes(C) > maxLds) return hipErrorInvalidConfiguration;
+  const size_t map = 4 * ((size_t(M.m) * M.m + 1) / 2);
+  const int staged = bytes(C) + map <= maxLds ? 1 : 0;  // else the position table is read from device memory
+  const size_t lds = bytes(C) + (staged ? map : 0);
+#define TCHEM_JAC(c)                                                                                           \
+  hipLaunchKernelGGL(jacobian_kernel<c>, dim3((nBatch + c - 1) / c), dim3(groupThreads(c)), lds, stream, M, nBatch, \
+                     state, photo, jac, staged)
+  if (C == 16) TCHEM_JAC(16);
+  else if (C == 4) TCHEM_JAC(4);
+  else TCHEM_JAC(1);
+#undef TCHEM_JAC
   return hipGetLastError();
 }
 

@@ -62,12 +62,13 @@ struct Lowering {
   std::vector<std::pair<int, int>> powers;  // (species, exponent >= 2) with a slot of their own
   std::vector<std::pair<int, int>> scaled;  // (reaction, factor >= 2) with a kf slot of their own
   int powerSlot(int sp, int n) {
-    if (n == 0) return d.oneC;
+    if (n <= 0) return d.oneC;
     if (n == 1) return d.oC + 8 * sp;
     const auto it = std::find(powers.begin(), powers.end(), std::make_pair(sp, n));
     return d.oC + 8 * (t.nSpec + int(it - powers.begin()));
   }
   int kfSlot(int r, int n) {
+    if (n == 0) return d.zero8;
     if (n == 1) return d.oK + 8 * r;
     const auto it = std::find(scaled.begin(), scaled.end(), std::make_pair(r, n));
     return d.oK + 8 * (kLanes * s.ropRounds + int(it - scaled.begin()));

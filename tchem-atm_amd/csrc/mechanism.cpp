@@ -181,11 +181,17 @@ MechTables compileMechanism(const KineticModel& km) {
           if (km.sidx(r, j + joff) < m) smap[{t.iperm[km.sidx(r, j + joff)], col}].push_back({p, km.nuki(r, j + joff)});
         ++p;
       }
+    // longest lists first: lanes that walk neighbouring entries walk lists of
+    // similar length
+    std::vector<const decltype(smap)::value_type*> byLength;
+    for (const auto& e : smap) byLength.push_back(&e);
+    std::stable_sort(byLength.begin(), byLength.end(),
+                     [](const auto* x, const auto* y) { return x->second.size() > y->second.size(); });
     t.serJPtr.push_back(0);
-    for (const auto& e : smap) {
-      t.serJRow.push_back(e.first.first);
-      t.serJCol.push_back(e.first.second);
-      for (const auto& c : e.second) {
+    for (const auto* e : byLength) {
+      t.serJRow.push_back(e->first.first);
+      t.serJCol.push_back(e->first.second);
+      for (const auto& c : e->second) {
         t.serJPair.push_back(c.first);
         t.serJCoef.push_back(c.second);
       }

@@ -83,7 +83,7 @@ struct MechTables {
   std::vector<int> serOmegaPtr;     // [m+1]
   std::vector<int> serOmegaReac;    // [nSerOmega]
   std::vector<double> serOmegaCoef; // [nSerOmega]
-  std::vector<int> serJRow, serJCol; // [nSerJ] structural entries, row-major
+  std::vector<int> serJRow, serJCol; // [nSerJ] structural entries, longest list first
   std::vector<int> serJPtr;         // [nSerJ+1]
   std::vector<int> serJPair;        // [nSerContrib]
   std::vector<double> serJCoef;     // [nSerContrib]

@@ -51,3 +51,76 @@ def test_encoded_programs_with_shifted_fields(checker, pkg, tmp_path, n_species,
                                    n_radicals=8, window=20, coupling="cascade")
     out = _run(checker, f)
     assert "shift 2" in out and "shift 3" in out
+
+
+def test_encoded_programs_of_reactant_powers(checker, tmp_path):
+    """Powers 0 (a fractional coefficient), 1, 2, 3 and 4, one of them on a
+    constant species; every derivative factor of each."""
+    f = tmp_path / "powers.yaml"
+    f.write_text(POWERS)
+    _run(checker, str(f))
+
+
+POWERS = """NCAR-version: v1.0
+environmental_conditions:
+  pressure:
+    initial_value: [101325]
+    units: Pa
+  temperature:
+    initial_value: [298.0]
+    units: K
+initial_state:
+  A:
+    initial_value: [0.1]
+    units: mol m-3
+  B:
+    initial_value: [0.2]
+    units: mol m-3
+  D:
+    initial_value: [0.3]
+    units: mol m-3
+  M:
+    initial_value: [10.0]
+    units: mol m-3
+constant_species:
+- description: third body
+  name: M
+species:
+- description: a
+  name: A
+- description: b
+  name: B
+- description: d
+  name: D
+reactions:
+- MUSICA_name: R1
+  reactants:
+    A: 3
+    B: 2
+    M: 1
+  products:
+    D: 1
+  type: ARRHENIUS
+  coefficients:
+    A: 2.0
+- MUSICA_name: R2
+  reactants:
+    A: 0.5
+    D: 4
+  products:
+    B: 2
+  type: ARRHENIUS
+  coefficients:
+    A: 0.5
+    C: -10.0
+- MUSICA_name: R3
+  reactants:
+    B: 1
+    M: 2
+  products:
+    A: 1
+  type: ARRHENIUS
+  coefficients:
+    A: 1.5
+    B: 0.3
+"""
