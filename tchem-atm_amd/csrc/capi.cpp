@@ -709,8 +709,8 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
   }
   // sparse programs (mechanisms they cannot express, or whose cell region
   // exceeds the LDS, run the dense form only)
-  auto pack = [&](const SparseSchedule& sc, int bytesT, bool adjoint, DevLowered* w) {
-    LoweredProgram p = lowerProgram(t, sc, bytesT, adjoint);
+  auto pack = [&](const SparseSchedule& sc, const LoweredSlots& slots, int bytesT, bool adjoint, DevLowered* w) {
+    LoweredProgram p = lowerProgram(t, sc, bytesT, adjoint, slots);
     stageTolerances(p.d, t.m, size_t(p.d.cellBytes), k->maxLds);
     if (sparseStageBytes(p.d, t.m, false) + size_t(p.d.cellBytes) > k->maxLds) return;
     *w = p.d;
@@ -721,14 +721,15 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
     if (!k->boxModel) throw std::runtime_error("no box model");
     const SparseSchedule fwd = buildSparseSchedule(t);
     k->nnzF = fwd.nnzF;
-    pack(fwd, 8, false, &k->low64);
-    pack(fwd, 4, false, &k->low32);
+    const LoweredSlots fs = chooseSlots(t, fwd);
+    pack(fwd, fs, 8, false, &k->low64);
+    pack(fwd, fs, 4, false, &k->low32);
     // the adjoint shares one cell layout between the forward programs and
     // the transposed ones: the transposed factor pattern has the same size
     const SparseSchedule trn = buildSparseSchedule(t, true);
     if (k->low64.enabled && trn.nnzF == fwd.nnzF && trn.pairSlots == fwd.pairSlots) {
-      pack(fwd, 8, true, &k->lowAdj);
-      pack(trn, 8, true, &k->lowAdjT);
+      pack(fwd, fs, 8, true, &k->lowAdj);
+      pack(trn, chooseSlots(t, trn, &fs), 8, true, &k->lowAdjT);
     }
   } catch (const std::exception&) {
     // what was encoded so far stands
@@ -1686,14 +1687,14 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
     std::vector<std::array<int, 2>> ent;  // (row, col) of every transfer derivative, table order
     const MechTables ta = aerosolTables(t, am, &ent);
     const SparseSchedule sc = buildSparseSchedule(ta, false);
+    LoweredProgram p = lowerProgram(ta, sc, 8, false, chooseSlots(ta, sc));
     auto position = [&](int r, int c) {  // the LDS slot of factor entry (r, c)
       for (int q = sc.rowPtr[r]; q < sc.rowPtr[r + 1]; ++q)
-        if (sc.colIdx[q] == c) return sc.slotOf[size_t(q)];
+        if (sc.colIdx[q] == c) return p.slot[size_t(sc.slotOf[size_t(q)])];
       throw std::runtime_error("transfer derivative outside the factor pattern");
     };
     X.oJpos = int(ib.size());
     for (const auto& e : ent) ib.push_back(position(e[0], e[1]));
-    LoweredProgram p = lowerProgram(ta, sc, 8, false);
     stageTolerances(p.d, mt, aerosolSparseCellBytes(p.d, X), kmcd->maxLds);
     h->W = p.d;
     pib.assign(p.words.begin(), p.words.end());

@@ -510,7 +510,9 @@ struct DenseBackend {
     atol = a.tol_time[2 * xs];
     rtol = a.tol_time[2 * xs + 1];
   }
-  static __device__ __forceinline__ void ready(const IntegratorArgs&, const Lds&, int) {}
+  static __device__ __forceinline__ void load_rates(const IntegratorArgs& a, const Lds& L, const double* kf, int lane) {
+    for (int r = lane; r < a.M.nReac; r += kWave) L.kf[r] = kf[r];
+  }
   // per-cell bindings: this cell's external sources
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
@@ -591,8 +593,8 @@ struct SparseBackend {
                                     a.cellBytes, wave);
   }
   static __device__ void init(const IntegratorArgs& a, const Lds& L, int lane) { sp_init(a.W, L, a.M.m, lane); }
-  static __device__ __forceinline__ void ready(const IntegratorArgs& a, const Lds& L, int lane) {
-    sp_scaled_rates<SH>(a.W, L, a.M.nReac, lane);
+  static __device__ __forceinline__ void load_rates(const IntegratorArgs& a, const Lds& L, const double* kf, int lane) {
+    sp_load_rates<SH>(a.W, L, kf, lane);
   }
   static __device__ __forceinline__ void put_c(const IntegratorArgs& a, const Lds& L, int lane, const double (&u)[QM]) {
 #pragma unroll
@@ -654,7 +656,8 @@ struct SparseBackend {
   static __device__ __forceinline__ bool factor_solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM],
                                                       Fact&) {
     TCHEM_PT_BEGIN(lu)
-    const bool ok = sp_lu<SH>(L, L.w, a.W.oLuHdr, a.W.oLu, a.W.oLu1, a.W.nLu, lane);
+    sp_lu<SH>(L, L.w, a.W.oLuHdr, a.W.oLu, a.W.oLu1, a.W.nLu, lane);
+    const bool ok = sp_pivots<SH, QM>(a.W, L, a.M.m, lane);
     TCHEM_PT_END(lu, 9)
     if (!ok) return false;
     TCHEM_PT_BEGIN(back)
@@ -736,10 +739,7 @@ __device__ void integrate_cell(const IntegratorArgs& a, const typename B::Lds& L
   const double k_err = (-3.0 * gam * gam + 4.0 * gam - 2.0) / (12.0 * (2.0 - gam));
 
   TCHEM_PT_BEGIN(cell)
-  {
-    const double* kf = a.kf + size_t(cell) * M.nReac;
-    for (int r = lane; r < M.nReac; r += kWave) L.kf[r] = kf[r];
-  }
+  B::load_rates(a, L, a.kf + size_t(cell) * M.nReac, lane);
   for (int i = mg + lane; i < nSpec; i += kWave) L.c[i] = row[3 + i];
 
   // un (state) and fn (f at un) live across steps; u, bc, est per step
@@ -763,7 +763,6 @@ __device__ void integrate_cell(const IntegratorArgs& a, const typename B::Lds& L
     for (int i = m + lane; i < nSpec; i += kWave) a.rec.consts[size_t(cell) * (nSpec - m) + (i - m)] = row[3 + i];
   }
   wave_sync();
-  B::ready(a, L, lane);
 
   const int max_it = ta._num_time_iterations_per_interval;
   const int max_newton = ta._max_num_newton_iterations;
@@ -1049,7 +1048,9 @@ struct MfmaBackend {
     atol = a.tol_time[2 * xs];
     rtol = a.tol_time[2 * xs + 1];
   }
-  static __device__ __forceinline__ void ready(const IntegratorArgs&, const Lds&, int) {}
+  static __device__ __forceinline__ void load_rates(const IntegratorArgs& a, const Lds& L, const double* kf, int lane) {
+    for (int r = lane; r < a.M.nReac; r += kWave) L.kf[r] = kf[r];
+  }
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
   }
@@ -1406,7 +1407,9 @@ struct AerosolLayout {
     rtol = a.tol_time[2 * xs + 1];
   }
   template <class LdsT>
-  static __device__ __forceinline__ void ready(const IntegratorArgs&, const LdsT&, int) {}
+  static __device__ __forceinline__ void load_rates(const IntegratorArgs& a, const LdsT& L, const double* kf, int lane) {
+    for (int r = lane; r < a.M.nReac; r += kWave) L.kf[r] = kf[r];
+  }
   // this cell's number concentrations, temperature and pressure, and the
   // SIMPOL constants (functions of T and p only)
   template <class LdsT>
@@ -1613,8 +1616,8 @@ struct AerosolSparseBackend : AerosolLayout {
   }
   static __device__ Lds carve(char* base, const IntegratorArgs& a, int wave) { return carve_aero_sparse(base, a, wave); }
   static __device__ void init(const IntegratorArgs& a, const Lds& L, int lane) { sp_init(a.W, L, a.X.mt, lane); }
-  static __device__ __forceinline__ void ready(const IntegratorArgs& a, const Lds& L, int lane) {
-    sp_scaled_rates<SH>(a.W, L, a.M.nReac, lane);
+  static __device__ __forceinline__ void load_rates(const IntegratorArgs& a, const Lds& L, const double* kf, int lane) {
+    sp_load_rates<SH>(a.W, L, kf, lane);
   }
   static __device__ void evaluate(const IntegratorArgs& a, const Lds& L, int lane, const double (&u)[QM],
                                   const double (&bc)[QM], double ch, bool newton, bool refresh, double (&f)[QM],
@@ -1717,7 +1720,8 @@ struct AerosolSparseBackend : AerosolLayout {
     }
   }
   static __device__ bool factor_solve(const IntegratorArgs& a, const Lds& L, int lane, double (&x)[QM], Fact&) {
-    if (!sp_lu<SH>(L, L.w, a.W.oLuHdr, a.W.oLu, a.W.oLu1, a.W.nLu, lane)) return false;
+    sp_lu<SH>(L, L.w, a.W.oLuHdr, a.W.oLu, a.W.oLu1, a.W.nLu, lane);
+    if (!sp_pivots<SH, QM>(a.W, L, a.X.mt, lane)) return false;
     sp_back<SH>(a.W, L, lane);
     get_x(a, L, lane, x);
     return true;
@@ -1769,11 +1773,15 @@ __global__ __launch_bounds__(64) void aerosol_rhs_kernel(IntegratorArgs a) {
 // iteration, sixteen took 76 k), not flops or bytes: the encoded programs
 // (lowered.hpp, sparse_exec.hpp) replaced an interpreter of the rounds that
 // decoded kind, length and indices per round and waited for scalar loads.
-// Measured, interpreter -> encoded: 131040 cells mixed, 80 TR-BDF2
-// iterations 305.2 -> 160.5 ms; 16411 cells FP64, 100 iterations 69.8 ->
-// 36.8 ms; one cell, 10 iterations 594 -> 309 us; E3SM 40960 cells to 1800 s
-// 63.6 -> 32.3 ms; CB05 + SOA, one particle, 8192 cells, 60 iterations 52.8
-// -> 33.7 ms (same bits).
+// Then slots spread over the LDS banks and pivots inverted once per
+// factorisation.  Measured, interpreter -> encoded -> spread: 131040 cells
+// mixed, 80 TR-BDF2 iterations 305.2 -> 160.5 -> 145.3 ms; 16411 cells FP64,
+// 100 iterations 69.8 -> 36.8 -> 36.2 ms; one cell, 10 iterations 594 -> 309
+// -> 304 us; E3SM 40960 cells to 1800 s 63.6 -> 32.3 -> 30.6 ms; CB05 + SOA,
+// one particle, 8192 cells, 60 iterations 52.8 -> 33.7 -> 33.0 ms (same bits).
+// Reading the stream 4 to 7 rounds ahead instead of 2, or a section's first
+// records a section early, gave -4 to +4 %: the rounds wait for their own
+// operands and instructions, not for the stream.
 template <class B, int QM, int kThreads, bool REC>
 __global__ __launch_bounds__(kThreads) void trbdf2_kernel(IntegratorArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
@@ -1902,7 +1910,8 @@ __device__ __forceinline__ bool adjoint_solve(const AdjointArgs& a, const SpLds<
   }
   sp_jacobian<SH>(W, LT, lane, -ch);
   wave_sync();
-  const bool ok = sp_lu<SH>(LT, LT.w, W.oLuHdr, W.oLu, W.oLu1, W.nLu, lane);
+  sp_lu<SH>(LT, LT.w, W.oLuHdr, W.oLu, W.oLu1, W.nLu, lane);
+  const bool ok = sp_pivots<SH, QM>(W, LT, m, lane);
   sp_back<SH>(W, LT, lane);
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
@@ -1922,10 +1931,13 @@ __device__ __forceinline__ bool adjoint_solve(const AdjointArgs& a, const SpLds<
 
 // grad_r += c rop_r w_r
 __device__ __forceinline__ void accumulate_grad(const DevLowered& W, const SpLds<double, false>& L, double* g,
-                                                int nReac, int lane, double c) {
-  for (int r = lane; r < nReac; r += kWave)
-    g[r] += c * lds_get<double>(L.cell + W.oP + 8 * r) *
-            lds_get<double>(L.cell + L.w.template rec<unsigned>(W.oWmap, r / kWave, lane));
+                                                int lane, double c) {
+  for (int s = 0; s < W.nRop; ++s) {
+    const int r = int(L.w.template rec<unsigned>(W.oKf, s, lane));
+    if (r >= 0)
+      g[r] += c * lds_get<double>(L.cell + W.oP + 8 * (kWave * s + lane)) *
+              lds_get<double>(L.cell + L.w.template rec<unsigned>(W.oWmap, s, lane));
+  }
 }
 
 template <int QM>
@@ -1956,10 +1968,7 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L
   const double atol = a.tol[0], rtol = a.tol[1];
   const int max_newton = a.newton[2 * cell], jint = a.newton[2 * cell + 1];
 
-  for (int r = lane; r < nReac; r += kWave) {
-    L.kf[r] = f.kf[size_t(cell) * nReac + r];
-    g[r] = 0.0;
-  }
+  for (int r = lane; r < nReac; r += kWave) g[r] = 0.0;
   for (int i = m + lane; i < nSpec; i += kWave) L.c[i] = f.rec.consts[size_t(cell) * (nSpec - m) + (i - m)];
   double lam[QM];
 #pragma unroll
@@ -1968,7 +1977,7 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L
     lam[q] = ai < m ? a.lambda_in[size_t(cell) * nSpec + M.perm()[ai]] : 0.0;
   }
   wave_sync();
-  sp_scaled_rates<SH>(f.W, L, nReac, lane);
+  sp_load_rates<SH>(f.W, L, f.kf + size_t(cell) * nReac, lane);
 
   using B = SparseBackend<double, QM, false>;
   double* tr = a.traj + size_t(cell) * kTraj * m;
@@ -2015,7 +2024,7 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L
         wave_sync();
       }
       ok &= adjoint_solve<QM>(a, LT, lane, c_bdf * h, lam, mu2);
-      accumulate_grad(a.WT, LT, g, nReac, lane, c_bdf * h);
+      accumulate_grad(a.WT, LT, g, lane, c_bdf * h);
       load_vec<QM>(tr + size_t(kAdjointSegment + 1 + j) * m, m, lane, u);
       B::put_c(f, L, lane, u);
       sp_rates<SH>(a.WT, LT, lane, true);
@@ -2023,12 +2032,12 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L
 #pragma unroll
       for (int q = 0; q < QM; ++q) rhs[q] = a_g * mu2[q];
       ok &= adjoint_solve<QM>(a, LT, lane, c_tr * h, rhs, mu1);
-      accumulate_grad(a.WT, LT, g, nReac, lane, c_tr * h);
+      accumulate_grad(a.WT, LT, g, lane, c_tr * h);
       load_vec<QM>(tr + size_t(j) * m, m, lane, u);
       B::put_c(f, L, lane, u);
       sp_rates<SH>(a.WT, LT, lane, true);
       wave_sync();
-      accumulate_grad(a.WT, LT, g, nReac, lane, c_tr * h);
+      accumulate_grad(a.WT, LT, g, lane, c_tr * h);
       sp_sums<SH>(LT, a.WT.oJtvHdr, a.WT.oJtv, a.WT.nJtv, LT.cell, LT.cell + a.WT.oV, lane);
       wave_sync();
 #pragma unroll
@@ -2055,7 +2064,7 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L
 
 // One wavefront per cell, cells taken from a device work queue.  Bound by the
 // same chain as trbdf2_kernel; gradient of 2000 CB05 cells over 1 ms of model
-// time, forward and backward: 583 ms with the rounds interpreted, 253 ms
+// time, forward and backward: 583 ms with the rounds interpreted, 249 ms
 // encoded.
 template <int QM>
 __global__ __launch_bounds__(512) __attribute__((flatten)) void adjoint_kernel(AdjointArgs a) {
@@ -2069,6 +2078,7 @@ __global__ __launch_bounds__(512) __attribute__((flatten)) void adjoint_kernel(A
   const SpLds<double, false> L = carve_sparse<double, false>(a.fw.W, ib + a.fw.W.oWords, 0, lds_raw, a.cellBytes, wave);
   SpLds<double, false> LT = L;
   LT.w.g = ib + a.WT.oWords;
+  LT.w.bytes = 4 * a.WT.words;
   double* g = reinterpret_cast<double*>(lds_raw + sparseStageBytes(a.WT, 0, false) +
                                         size_t(wave) * size_t(a.cellBytes) + adjointRegionBytes(a.fw.W, a.WT));
   sp_init(a.WT, L, M.m, lane);

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <map>
 #include <numeric>
+#include <random>
 #include <stdexcept>
 
 namespace tchem_amd {
@@ -17,17 +18,239 @@ constexpr int kLanes = 64;
 int al16(int x) { return (x + 15) & ~15; }
 int ceilDiv(int a, int b) { return (a + b - 1) / b; }
 
+// LDS reads of one instruction: the distinct entries 32 lanes (half a
+// wavefront) read together.  Entries whose slots are equal modulo 32 conflict
+// (32 banks for 4-byte reads, 32 pairs of 64 for 8-byte reads; reads of one
+// address do not; stores take the time of two passes anyway).
+using Gather = std::vector<int>;
+
+// Slots of n entries such that the gathers take few passes: swaps of two
+// entries' slots are kept when they do not add passes.  slot[] holds the
+// starting assignment (a permutation); entries >= n of a gather are slots
+// that do not move.  Deterministic; at most `tries` swaps.
+void spreadOverBanks(std::vector<int>& slot, const std::vector<Gather>& gathers, long tries) {
+  constexpr int kBanks = 32;
+  const int n = int(slot.size());
+  std::vector<std::array<unsigned char, kBanks>> cnt(gathers.size());
+  std::vector<std::vector<int>> in(static_cast<size_t>(n));
+  for (size_t g = 0; g < gathers.size(); ++g) {
+    cnt[g].fill(0);
+    for (int e : gathers[g]) {
+      ++cnt[g][size_t((e < n ? slot[size_t(e)] : e) % kBanks)];
+      if (e < n) in[size_t(e)].push_back(int(g));
+    }
+  }
+  auto passes = [](const std::array<unsigned char, kBanks>& c) { return int(*std::max_element(c.begin(), c.end())); };
+  std::mt19937_64 rng(0x5eedULL);
+  std::vector<int> mark(gathers.size(), 0);
+  int stamp = 0;
+  for (long it = 0; it < tries && n > 1; ++it) {
+    const size_t a = size_t(rng() % unsigned(n)), b = size_t(rng() % unsigned(n));
+    const size_t ra = size_t(slot[a] % kBanks), rb = size_t(slot[b] % kBanks);
+    if (ra == rb || (in[a].empty() && in[b].empty())) continue;
+    ++stamp;
+    for (int g : in[b]) mark[size_t(g)] = stamp;
+    int delta = 0;
+    auto move = [&](int g, size_t from, size_t to) {
+      auto& c = cnt[size_t(g)];
+      const int before = passes(c);
+      --c[from];
+      ++c[to];
+      return passes(c) - before;
+    };
+    std::vector<int> onlyA, onlyB;  // gathers that hold both keep their counts
+    for (int g : in[a]) {
+      if (mark[size_t(g)] == stamp) mark[size_t(g)] = -stamp;
+      else onlyA.push_back(g);
+    }
+    for (int g : in[b])
+      if (mark[size_t(g)] == stamp) onlyB.push_back(g);
+    for (int g : onlyA) delta += move(g, ra, rb);
+    for (int g : onlyB) delta += move(g, rb, ra);
+    if (delta <= 0) {
+      std::swap(slot[a], slot[b]);
+    } else {
+      for (int g : onlyA) move(g, rb, ra);
+      for (int g : onlyB) move(g, ra, rb);
+    }
+  }
+}
+// the gathers of 64 lanes' entries, half a wavefront each (repeats dropped)
+void addGathers(std::vector<Gather>& out, const std::vector<int>& lanes) {
+  for (size_t h = 0; h < lanes.size(); h += 32) {
+    Gather g(lanes.begin() + long(h), lanes.begin() + long(std::min(lanes.size(), h + 32)));
+    std::sort(g.begin(), g.end());
+    g.erase(std::unique(g.begin(), g.end()), g.end());
+    if (g.size() > 1) out.push_back(std::move(g));
+  }
+}
+
+// ---- Jacobian chains cut into the records' chunks --------------------------
+struct Chunk {
+  int target = 0;  // factor position of the rounds' numbering, or -1 - partial slot
+  unsigned flags = 0;
+  std::vector<std::pair<int, double>> e;  // (pair, coefficient)
+};
+struct Join {
+  int target = 0, first = 0, count = 0;
+  bool diag = false;
+};
+struct Chunks {
+  std::vector<Chunk> j4, j2, j1;
+  std::vector<Join> joins;
+  int nPartial = 0;
+};
+Chunks jacobianChunks(const MechTables& t, const SparseSchedule& s) {
+  Chunks k;
+  std::map<std::pair<int, int>, int> at;
+  for (int n = 0; n < t.nnzJ(); ++n)
+    at[s.transposed ? std::make_pair(t.jnzCol[n], t.jnzRow[n]) : std::make_pair(t.jnzRow[n], t.jnzCol[n])] = n;
+  constexpr size_t kC = SparseSchedule::kMaxChain;
+  for (int i = 0; i < s.m; ++i)
+    for (int q = s.rowPtr[i]; q < s.rowPtr[i + 1]; ++q) {
+      const int j = s.colIdx[size_t(q)];
+      Chunk c;
+      c.target = s.slotOf[size_t(q)];
+      const bool diag = i == j;
+      const auto it = at.find({i, j});
+      if (it != at.end())
+        for (int e = t.jnzPtr[it->second]; e < t.jnzPtr[it->second + 1]; ++e) c.e.push_back({t.jcPair[e], t.jcCoef[e]});
+      if (!diag && c.e.size() <= 1) {
+        k.j1.push_back(c);
+      } else if (!diag && c.e.size() == 2) {
+        k.j2.push_back(c);
+      } else if (c.e.size() <= kC) {
+        c.flags = diag ? 1u : 0u;
+        k.j4.push_back(c);
+      } else {
+        Join x;
+        x.target = c.target;
+        x.first = k.nPartial;
+        x.diag = diag;
+        for (size_t b = 0; b < c.e.size(); b += kC) {
+          Chunk part;
+          part.target = -1 - k.nPartial++;
+          part.flags = 2u;
+          part.e.assign(c.e.begin() + long(b), c.e.begin() + long(std::min(c.e.size(), b + kC)));
+          k.j4.push_back(part);
+          ++x.count;
+        }
+        k.joins.push_back(x);
+      }
+    }
+  std::stable_sort(k.joins.begin(), k.joins.end(), [](const Join& a, const Join& b) { return a.count > b.count; });
+  return k;
+}
+
+// segments by descending length: the order the SUM section takes them in
+std::vector<int> segmentOrder(const MechTables& t) {
+  std::vector<int> o(size_t(t.nSeg()));
+  std::iota(o.begin(), o.end(), 0);
+  std::stable_sort(o.begin(), o.end(), [&](int a, int b) { return t.segEnd[a] - t.segBegin[a] > t.segEnd[b] - t.segBegin[b]; });
+  return o;
+}
+
+// ---- slots: gathers of every round spread over the LDS banks ----------------
+std::vector<int> factorSlots(const SparseSchedule& s) {
+  using SS = SparseSchedule;
+  std::vector<int> slot(size_t(s.nnzF));
+  std::iota(slot.begin(), slot.end(), 0);
+  std::vector<Gather> gs;
+  // right-hand sides sit after the factor, two units apart; the zero slot
+  // is nnzF; the trash slot is only read by idle lanes
+  const int rhs0 = (s.nnzF + 2 + 3) & ~3;
+  auto at = [&](unsigned ix) {
+    const int i = int(ix);
+    if (i < s.nnzF) return i;
+    return i < s.nnzF + s.m ? rhs0 + 2 * (i - s.nnzF) : s.nnzF;
+  };
+  size_t b = 0;
+  for (int r = 0; r < s.luRounds + s.backRounds; ++r) {
+    const int kind = int(s.progHdr[size_t(r)] >> 16), len = int(s.progHdr[size_t(r)] & 0xffff);
+    const int words = kind == SS::kMul ? 1 : 1 + len;
+    auto gather = [&](int j, int shift, unsigned mask) {
+      std::vector<int> lanes;
+      for (int l = 0; l < kLanes; ++l)
+        lanes.push_back(at((s.progBody[b + size_t(kLanes) * size_t(j) + size_t(l)] >> shift) & mask));
+      addGathers(gs, lanes);
+    };
+    if (kind == SS::kMul) {
+      gather(0, 16, 0xffffu);
+    } else if (kind == SS::kUpd) {
+      gather(0, 0, 0xffffu);
+      for (int j = 1; j <= len; ++j) gather(j, 0, 0xffffu), gather(j, 16, 0xffffu);
+    } else if (kind == SS::kMulUpd) {
+      gather(0, 0, 0xffffu);
+      gather(1, 0, 0xffffu), gather(1, 16, 0xffffu);
+      gather(2, 0, 0x7fffu);
+      for (int j = 3; j <= len; ++j) gather(j, 0, 0xffffu), gather(j, 16, 0xffffu);
+    } else {
+      for (int j = 1; j <= len; ++j) gather(j, 0, 0xffffu);
+    }
+    b += size_t(kLanes) * size_t(words);
+  }
+  spreadOverBanks(slot, gs, std::min<long>(140L * s.nnzF, 120000L));
+  return slot;
+}
+std::vector<int> pairSlots(const SparseSchedule& s, const Chunks& chunks) {
+  std::vector<int> pairSlot(size_t(kLanes) * size_t(s.pairRounds));
+  std::iota(pairSlot.begin(), pairSlot.end(), 0);
+  std::vector<Gather> gs;
+  auto gather = [&](const std::vector<Chunk>& v, size_t per, size_t k, size_t e) {
+    for (size_t r = 0; r * per * kLanes < v.size(); ++r) {
+      std::vector<int> lanes;
+      for (size_t l = 0; l < size_t(kLanes); ++l) {
+        const size_t i = (per * r + k) * kLanes + l;
+        lanes.push_back(i < v.size() && e < v[i].e.size() ? v[i].e[e].first : 1 << 20);
+      }
+      addGathers(gs, lanes);
+    }
+  };
+  for (size_t e = 0; e < 4; ++e) gather(chunks.j4, 1, 0, e);
+  for (size_t k = 0; k < 2; ++k)
+    for (size_t e = 0; e < 2; ++e) gather(chunks.j2, 2, k, e);
+  for (size_t k = 0; k < 4; ++k) gather(chunks.j1, 4, k, 0);
+  spreadOverBanks(pairSlot, gs, std::min<long>(120L * long(pairSlot.size()), 60000L));
+  return pairSlot;
+}
+// rates of progress and rate constants share their slots
+std::vector<int> reactionSlots(const MechTables& t, const SparseSchedule& s, const std::vector<int>& pairSlot) {
+  const std::vector<int> segOrder = segmentOrder(t);
+  std::vector<int> ropSlot(size_t(kLanes) * size_t(s.ropRounds));
+  std::iota(ropSlot.begin(), ropSlot.end(), 0);
+  std::vector<Gather> gs;
+  for (size_t g = 0; g < segOrder.size(); g += kLanes) {
+    const int first = segOrder[g], most = t.segEnd[first] - t.segBegin[first];
+    for (int e = 0; e < most; ++e) {
+      std::vector<int> lanes;
+      for (size_t l = g; l < std::min(segOrder.size(), g + kLanes); ++l) {
+        const int at = t.segBegin[segOrder[l]] + e;
+        lanes.push_back(at < t.segEnd[segOrder[l]] ? t.omegaReac[at] : 1 << 20);
+      }
+      addGathers(gs, lanes);
+    }
+  }
+  std::vector<int> reacOf(pairSlot.size(), 1 << 20);
+  for (int r = 0; r < t.nReac; ++r)
+    for (int p = t.pairPtr[r]; p < t.pairPtr[r + 1]; ++p) reacOf[size_t(pairSlot[size_t(p)])] = r;
+  for (size_t i = 0; i < reacOf.size(); i += kLanes)
+    addGathers(gs, std::vector<int>(reacOf.begin() + long(i), reacOf.begin() + long(i + kLanes)));
+  spreadOverBanks(ropSlot, gs, std::min<long>(200L * long(ropSlot.size()), 60000L));
+  return ropSlot;
+}
+
 struct Lowering {
   const MechTables& t;
   const SparseSchedule& s;
   const int T;
   const bool adjoint;
+  const LoweredSlots& slots;
   LoweredProgram out;
   DevLowered& d;
   std::vector<uint32_t>& W;
 
-  Lowering(const MechTables& t_, const SparseSchedule& s_, int bytesT, bool adj)
-      : t(t_), s(s_), T(bytesT), adjoint(adj), d(out.d), W(out.words) {}
+  Lowering(const MechTables& t_, const SparseSchedule& s_, int bytesT, bool adj, const LoweredSlots& sl)
+      : t(t_), s(s_), T(bytesT), adjoint(adj), slots(sl), d(out.d), W(out.words), ropSlot(sl.rop), pairSlot(sl.pair) {}
 
   int readAhead = 0;  // words a section's loop may read past its end
 
@@ -46,9 +269,8 @@ struct Lowering {
   void end(int recordWords, int ahead = 2) { readAhead = std::max(readAhead, int(W.size()) + ahead * recordWords); }
 
   // ---- addresses of the cell region
-  int slotA(int p) const { return p * T; }  // factor slot (bank-aware numbering)
+  int slotA(int p) const { return T * out.slot[size_t(p)]; }  // slot of the rounds' numbering
   int rhs(int i) const { return d.oR + 2 * T * i; }
-  int rdiag(int i) const { return rhs(i) + T; }
   // an index of the rounds' matrix array: factor slot, RHS, zero, trash
   unsigned matrix(unsigned ix) const {
     const int i = int(ix);
@@ -59,6 +281,7 @@ struct Lowering {
     throw std::runtime_error("lowered programs: matrix index out of range");
   }
 
+  const std::vector<int>&ropSlot, &pairSlot;  // of LoweredSlots
   std::vector<std::pair<int, int>> powers;  // (species, exponent >= 2) with a slot of their own
   std::vector<std::pair<int, int>> scaled;  // (reaction, factor >= 2) with a kf slot of their own
   int powerSlot(int sp, int n) {
@@ -69,7 +292,7 @@ struct Lowering {
   }
   int kfSlot(int r, int n) {
     if (n == 0) return d.zero8;
-    if (n == 1) return d.oK + 8 * r;
+    if (n == 1) return d.oK + 8 * ropSlot[size_t(r)];
     const auto it = std::find(scaled.begin(), scaled.end(), std::make_pair(r, n));
     return d.oK + 8 * (kLanes * s.ropRounds + int(it - scaled.begin()));
   }
@@ -94,66 +317,9 @@ struct Lowering {
       }
   }
 
-  // ---- Jacobian chains: (target slot, diagonal, entries)
-  struct Chain {
-    int target = 0;
-    bool diag = false;
-    std::vector<std::pair<int, double>> e;  // (pair, coefficient)
-  };
-  struct Chunk {
-    int target = 0;  // byte offset
-    unsigned flags = 0;
-    std::vector<std::pair<int, double>> e;
-  };
   std::vector<Chunk> j4, j2, j1;
-  struct Join {
-    int target = 0, first = 0, count = 0;
-    bool diag = false;
-  };
   std::vector<Join> joins;
   int nPartial = 0;
-
-  void jacobianChains() {
-    const int m = s.m;
-    std::map<std::pair<int, int>, int> at;
-    for (int n = 0; n < t.nnzJ(); ++n)
-      at[s.transposed ? std::make_pair(t.jnzCol[n], t.jnzRow[n]) : std::make_pair(t.jnzRow[n], t.jnzCol[n])] = n;
-    constexpr size_t kC = SparseSchedule::kMaxChain;
-    for (int i = 0; i < m; ++i)
-      for (int q = s.rowPtr[i]; q < s.rowPtr[i + 1]; ++q) {
-        const int j = s.colIdx[size_t(q)];
-        Chunk c;
-        c.target = slotA(s.slotOf[size_t(q)]);
-        const bool diag = i == j;
-        const auto it = at.find({i, j});
-        if (it != at.end())
-          for (int e = t.jnzPtr[it->second]; e < t.jnzPtr[it->second + 1]; ++e)
-            c.e.push_back({t.jcPair[e], t.jcCoef[e]});
-        if (!diag && c.e.size() <= 1) {
-          j1.push_back(c);
-        } else if (!diag && c.e.size() == 2) {
-          j2.push_back(c);
-        } else if (c.e.size() <= kC) {
-          c.flags = diag ? 1u : 0u;
-          j4.push_back(c);
-        } else {
-          Join x;
-          x.target = c.target;
-          x.first = nPartial;
-          x.diag = diag;
-          for (size_t b = 0; b < c.e.size(); b += kC) {
-            Chunk part;
-            part.target = -1 - nPartial++;  // partial slot, placed when the layout is known
-            part.flags = 2u;
-            part.e.assign(c.e.begin() + long(b), c.e.begin() + long(std::min(c.e.size(), b + kC)));
-            j4.push_back(part);
-            ++x.count;
-          }
-          joins.push_back(x);
-        }
-      }
-    std::stable_sort(joins.begin(), joins.end(), [](const Join& a, const Join& b) { return a.count > b.count; });
-  }
 
   void layout() {
     const int m = s.m;
@@ -278,19 +444,23 @@ struct Lowering {
                        : pack(field(d.oneC), field(d.trashC)));
       W.push_back(live ? uint32_t(powers[i].second) : 1u);
     }
+    std::vector<int> reactionAt(ropSlot.size(), -1);
+    for (int r = 0; r < t.nReac; ++r) reactionAt[size_t(ropSlot[size_t(r)])] = r;
+    d.oKf = begin();
+    for (int r : reactionAt) W.push_back(uint32_t(r));
     d.oKfx = begin();
     d.nKfx = ceilDiv(int(scaled.size()), kLanes);
     for (int i = 0; i < kLanes * d.nKfx; ++i) {
       const bool live = i < int(scaled.size());
-      W.push_back(live ? uint32_t(scaled[i].first) : 0u);
+      W.push_back(live ? uint32_t(ropSlot[size_t(scaled[i].first)]) : 0u);
       W.push_back(live ? pack(field(kfSlot(scaled[i].first, scaled[i].second)), unsigned(scaled[i].second))
                        : pack(field(d.trashC), 1u));
     }
     // rates of progress
     d.oRop = begin();
     d.nRop = s.ropRounds;
-    for (int r = 0; r < kLanes * d.nRop; ++r) {
-      const bool live = r < t.nReac;
+    for (int r : reactionAt) {
+      const bool live = r >= 0;
       W.push_back(live ? pack(field(factorSlot(r, 0)), field(factorSlot(r, 1))) : pack(field(d.oneC), field(d.oneC)));
       W.push_back(live ? field(factorSlot(r, 2)) : field(d.oneC));
     }
@@ -299,17 +469,17 @@ struct Lowering {
     d.oPair = begin();
     d.nPair = s.pairRounds;
     {
-      std::vector<std::array<uint32_t, 2>> rec;
+      std::vector<std::array<uint32_t, 2>> rec(pairSlot.size(), {pack(field(d.zero8), field(d.oneC)),
+                                                                 pack(field(d.oneC), field(d.oneC))});
       for (int r = 0; r < t.nReac; ++r)
         for (int p = t.pairPtr[r]; p < t.pairPtr[r + 1]; ++p) {
           const int js = t.pairSlot[p], n = power(r, js);
           std::vector<int> g;
           for (int j = 0; j < 3; ++j)
             if (j != js) g.push_back(factorSlot(r, j));
-          rec.push_back({pack(field(kfSlot(r, n)), field(powerSlot(spec(r, js), n - 1))), pack(field(g[0]), field(g[1]))});
+          rec[size_t(pairSlot[size_t(p)])] = {pack(field(kfSlot(r, n)), field(powerSlot(spec(r, js), n - 1))),
+                                              pack(field(g[0]), field(g[1]))};
         }
-      while (int(rec.size()) < kLanes * d.nPair)
-        rec.push_back({pack(field(d.zero8), field(d.oneC)), pack(field(d.oneC), field(d.oneC))});
       for (const auto& x : rec) W.insert(W.end(), x.begin(), x.end());
     }
     end(2 * kLanes);
@@ -319,7 +489,7 @@ struct Lowering {
       for (int g = 0; g < t.nSeg(); ++g) {
         ch.emplace_back();
         for (int e = t.segBegin[g]; e < t.segEnd[g]; ++e)
-          ch.back().push_back(pack(field(d.oP + 8 * t.omegaReac[e]), coef(t.omegaCoef[e])));
+          ch.back().push_back(pack(field(d.oP + 8 * ropSlot[size_t(t.omegaReac[e])]), coef(t.omegaCoef[e])));
       }
       const std::vector<int> slot = sums(ch, pack(field(d.zero8), 0), &d.oSegHdr, &d.oSeg, &d.nSeg);
       const int rows = int(t.rowSegPtr.size()) - 1;
@@ -345,8 +515,8 @@ struct Lowering {
   }
 
   void jacobian() {
-    auto target = [&](int x) { return field(x < 0 ? d.oPS + T * (-1 - x) : x); };
-    auto dpr = [&](const Chunk* c, size_t k) { return field(c && k < c->e.size() ? d.oD + T * c->e[k].first : d.zeroA); };
+    auto target = [&](int x) { return field(x < 0 ? d.oPS + T * (-1 - x) : slotA(x)); };
+    auto dpr = [&](const Chunk* c, size_t k) { return field(c && k < c->e.size() ? d.oD + T * pairSlot[size_t(c->e[k].first)] : d.zeroA); };
     std::vector<double> cf;
     auto coefs = [&](const Chunk* c, size_t n) {
       for (size_t k = 0; k < n; ++k) cf.push_back(c && k < c->e.size() ? c->e[k].second : 0.0);
@@ -406,7 +576,7 @@ struct Lowering {
     d.nJx = ceilDiv(int(joins.size()), kLanes);
     for (int i = 0; i < kLanes * d.nJx; ++i) {
       const bool live = i < int(joins.size());
-      W.push_back(live ? pack(field(joins[i].target), field(d.oPS + T * joins[i].first))
+      W.push_back(live ? pack(target(joins[i].target), field(d.oPS + T * joins[i].first))
                        : pack(field(d.trashA), field(d.oPS)));
       W.push_back(live ? uint32_t(joins[i].count) | (joins[i].diag ? 0x80000000u : 0u) : 0u);
     }
@@ -418,7 +588,7 @@ struct Lowering {
     using SS = SparseSchedule;
     std::vector<unsigned char> bits;
     std::vector<uint32_t> w4, w1;
-    const unsigned z = field(d.zeroA), trashR = field(rdiag(s.m + 1)), tr = field(d.trashA);
+    const unsigned z = field(d.zeroA), tr = field(d.trashA);
     for (int r = r0; r < r0 + n; ++r) {
       const int kind = int(s.progHdr[size_t(r)] >> 16), len = int(s.progHdr[size_t(r)] & 0xffff);
       auto word = [&](int j, int l) { return s.progBody[b + size_t(kLanes) * size_t(j) + size_t(l)]; };
@@ -426,14 +596,10 @@ struct Lowering {
       for (int l = 0; l < kLanes; ++l) {
         unsigned f[10];
         std::fill(f, f + 10, z);
-        f[9] = 0;
         if (kind == SS::kMul) {
           const unsigned dst = word(0, l) & 0xffff, src = word(0, l) >> 16;
-          const bool piv = (dst & 0x8000u) != 0;
-          f[0] = piv ? tr : matrix(dst);
+          f[0] = (dst & 0x8000u) ? tr : matrix(dst);
           f[1] = matrix(src);
-          f[2] = piv ? field(rdiag(int(dst & 0x7fff))) : trashR;
-          f[3] = piv ? 2u : 0u;
         } else if (kind == SS::kUpd) {
           f[0] = matrix(word(0, l));
           for (int j = 0; j < len; ++j) {
@@ -441,18 +607,17 @@ struct Lowering {
             f[2 + 2 * j] = matrix(word(1 + j, l) >> 16);
           }
         } else if (kind == SS::kMulUpd) {
-          const unsigned w2 = word(2, l);
-          const int ri = int(w2 >> 16);
           f[0] = matrix(word(0, l));
           f[1] = matrix(word(1, l) & 0xffff);
           f[2] = matrix(word(1, l) >> 16);
-          f[3] = matrix(w2 & 0x7fff);
-          f[4] = field(rdiag(ri));
+          f[3] = matrix(word(2, l) & 0x7fff);
           for (int j = 0; j < len - 2; ++j) {
-            f[5 + 2 * j] = matrix(word(3 + j, l) & 0xffff);
-            f[6 + 2 * j] = matrix(word(3 + j, l) >> 16);
+            f[4 + 2 * j] = matrix(word(3 + j, l) & 0xffff);
+            f[5 + 2 * j] = matrix(word(3 + j, l) >> 16);
           }
-          f[9] = ((w2 & 0x8000u) ? 1u : 0u) | (ri != s.m + 1 ? 2u : 0u);
+          // the device tells a multiplier lane by its target being its own multiplier
+          if (((word(2, l) & 0x8000u) != 0) != (f[0] == f[1]))
+            throw std::runtime_error("lowered programs: ambiguous multiplier lane");
         } else {
           throw std::runtime_error("lowered programs: unexpected round in the LU program");
         }
@@ -475,6 +640,9 @@ struct Lowering {
     static_assert(SparseSchedule::kMaxChain == 4 && SparseSchedule::kMaxMulUpdChain == 2, "record layout");
     d.nLu = s.luRounds;
     luRounds(0, s.luRounds, 0, &d.oLuHdr, &d.oLu, &d.oLu1);
+    d.oDiag = begin();
+    for (int i = 0; i < kLanes * ceilDiv(s.m, kLanes); ++i)
+      W.push_back(uint32_t(i < s.m ? slotA(s.slotOf[size_t(s.diagIdx[size_t(i)])]) : d.zeroA));
     // back substitution: a round of n-entry chains is n single-entry rounds
     // (no round reads an entry it writes)
     {
@@ -522,11 +690,12 @@ struct Lowering {
     const std::vector<int> w = sums(nu, pack(field(d.oMu + 8 * m), 0), &d.oNutHdr, &d.oNut, &d.nNut);
     for (int r = 0; r < t.nReac; ++r)
       for (int p = t.pairPtr[r]; p < t.pairPtr[r + 1]; ++p)
-        jt[size_t(spec(r, t.pairSlot[p]))].push_back(pack(field(d.oD + T * p), field(d.oW + 8 * w[size_t(r)])));
+        jt[size_t(spec(r, t.pairSlot[p]))].push_back(pack(field(d.oD + T * pairSlot[size_t(p)]), field(d.oW + 8 * w[size_t(r)])));
     const std::vector<int> v = sums(jt, pack(field(d.zeroA), field(d.zero8)), &d.oJtvHdr, &d.oJtv, &d.nJtv);
-    d.oWmap = begin();
-    for (int r = 0; r < kLanes * ceilDiv(t.nReac, kLanes); ++r)
-      W.push_back(uint32_t(r < t.nReac ? d.oW + 8 * w[size_t(r)] : d.zero8));
+    d.oWmap = begin();  // by slot of the reaction
+    std::vector<uint32_t> at(ropSlot.size(), uint32_t(d.zero8));
+    for (int r = 0; r < t.nReac; ++r) at[size_t(ropSlot[size_t(r)])] = uint32_t(d.oW + 8 * w[size_t(r)]);
+    W.insert(W.end(), at.begin(), at.end());
     d.oVmap = begin();
     for (int i = 0; i < kLanes * ceilDiv(m, kLanes); ++i) W.push_back(uint32_t(i < m ? d.oV + 8 * v[size_t(i)] : d.zero8));
   }
@@ -534,8 +703,13 @@ struct Lowering {
   void run() {
     if (T != 4 && T != 8) throw std::runtime_error("lowered programs: entry size");
     if (adjoint && T != 8) throw std::runtime_error("lowered programs: the adjoint is FP64");
+    out.slot = slots.factor;
     collect();
-    jacobianChains();
+    {
+      Chunks k = jacobianChunks(t, s);
+      j4 = std::move(k.j4), j2 = std::move(k.j2), j1 = std::move(k.j1), joins = std::move(k.joins);
+      nPartial = k.nPartial;
+    }
     layout();
     evaluation();
     linearAlgebra();
@@ -555,8 +729,22 @@ struct Lowering {
 
 }  // namespace
 
-LoweredProgram lowerProgram(const MechTables& t, const SparseSchedule& s, int bytesT, bool adjoint) {
-  Lowering L(t, s, bytesT, adjoint);
+LoweredSlots chooseSlots(const MechTables& t, const SparseSchedule& s, const LoweredSlots* shared) {
+  LoweredSlots o;
+  o.factor = factorSlots(s);
+  if (shared) {
+    o.pair = shared->pair;
+    o.rop = shared->rop;
+  } else {
+    o.pair = pairSlots(s, jacobianChunks(t, s));
+    o.rop = reactionSlots(t, s, o.pair);
+  }
+  return o;
+}
+
+LoweredProgram lowerProgram(const MechTables& t, const SparseSchedule& s, int bytesT, bool adjoint,
+                            const LoweredSlots& slots) {
+  Lowering L(t, s, bytesT, adjoint, slots);
   L.run();
   return std::move(L.out);
 }

@@ -15,6 +15,8 @@
 //     that holds 1;
 //   * right-hand side and reciprocal pivot of a row are neighbours (one read
 //     in the back substitution).
+//   * reactions, derivative pairs and factor entries are numbered so that the
+//     gathers of the rounds fall on distinct LDS banks (spreadOverBanks).
 // The value of every slot is the rounds' value bit for bit: the same
 // operations on the same operands in the same order per target (a Jacobian
 // chain keeps its partial sums of kMaxChain contributions).
@@ -22,8 +24,10 @@
 // Sections (words are 32-bit, a record of w words per lane is stored as
 // [lane][w], 64 records per round):
 //   POW   w 2: source field | destination field << 16, exponent
-//   KFX   w 2: reaction, destination field | factor << 16   (once per cell)
-//   ROP   w 2: f0 | f1 << 16, f2; rop[64 r + lane] = kf * f0 * f1 * f2
+//   KF    w 1: reaction whose rate constant is in this slot, -1 for a zero
+//         (once per cell)
+//   KFX   w 2: slot, destination field | factor << 16   (once per cell)
+//   ROP   w 2: f0 | f1 << 16, f2; rop[64 r + lane] = kf[64 r + lane] f0 f1 f2
 //   PAIR  w 2: kf | fd << 16, g0 | g1 << 16; dpr[64 r + lane] = kf fd g0 g1
 //   SUM   (segments; nu^T mu and J^T mu of the adjoint) w 4: four entries
 //         x | y << 16; acc = fma(y, x, acc); sums go to out[64 p + lane] for
@@ -37,12 +41,14 @@
 //         targets of one (words 2, 3)
 //   JX    w 2: target | first partial << 16, count | diagonal << 31 (largest
 //         count first): partials added to the initial value in order
-//   LU    w 4 and w 1 (ten fields); per 64 rounds a header of two 64-bit
-//         masks: rounds of kind kLMul, rounds of kind kLUpd (others kLMulUpd)
+//   LU    w 4 and w 1; per 64 rounds a header of two 64-bit masks: rounds of
+//         kind kLMul, rounds of kind kLUpd (others kLMulUpd)
 //         kLUpd: target, lo0, hi0, .. lo3, hi3, -
-//         kLMulUpd: target, ik, kj, kk, rdiag, lo0, hi0, lo1, hi1,
-//                   flags (1 multiplier lane, 2 pivot lane)
-//         kLMul: dst, src, rdiag, flags (2 pivot lane), -
+//         kLMulUpd: target, ik, kj, kk, lo0, hi0, lo1, hi1, -, - (a multiplier
+//                   lane's target is ik)
+//         kLMul: dst, src, -, ..
+//   DIAG  w 1: byte offset of the pivot of row 64 r + lane (reciprocal pivots
+//         are stored, and pivots checked, once after the last round)
 //   FWD   LU rounds of kind kLUpd (factor reuse)
 //   BACK  w 4: two single-entry rounds, each target | U << 16, pair
 #pragma once
@@ -72,25 +78,37 @@ struct DevLowered {
   int oR;                 // (rhs, reciprocal pivot) pairs, rows m (zeros) and m + 1 (trash) after the m unknowns
   int oD, oPS;            // derivative pairs; partial sums, in the place of what is dead while J is assembled
   int oC, oneC, trashC;   // concentrations, the slot that holds 1
-  int oK, nK, zero8;      // kf: zeros from nReac to 64 nRop, n * kf slots, the slot that holds 0 (the last)
+  int oK, nK, zero8;      // kf: 64 nRop slots, n * kf slots, the slot that holds 0 (the last)
   int oP, oS;             // rates of progress, segment sums
   // sections
-  int oPow, nPow, oKfx, nKfx, oRop, nRop, oPair, nPair;
+  int oPow, nPow, oKf, oKfx, nKfx, oRop, nRop, oPair, nPair;
   int oSegHdr, oSeg, nSeg;
   int oRow, nRow[4];
   int oJac, oJacC, nJ4, nJ2, nJ1, oJx, nJx;
-  int oLuHdr, oLu, oLu1, nLu, oBack, nBack, oFwdHdr, oFwd, oFwd1, nFwd;
+  int oLuHdr, oLu, oLu1, nLu, oDiag, oBack, nBack, oFwdHdr, oFwd, oFwd1, nFwd;
   // adjoint programs only
   int oNutHdr, oNut, nNut, oJtvHdr, oJtv, nJtv;
   int oMu, oW, oV;  // mu [m + 1] (mu[m] = 0), w sums, v sums (byte offsets in the cell region)
-  int oWmap, oVmap;        // [64 ceil(nReac / 64)] byte offset of w_r, [64 ceil(m / 64)] of v_i
+  int oWmap, oVmap;        // byte offset of w_r by slot of reaction r, [64 ceil(m / 64)] of v_i
 };
 
 struct LoweredProgram {
   DevLowered d{};
   std::vector<uint32_t> words;
   std::vector<double> coef;  // coefficient table, [0] = 0
+  std::vector<int> slot;     // factor slot of the rounds' numbering (SparseSchedule::slotOf) -> slot in the cell
 };
+
+// Where reactions, derivative pairs and factor entries live, so that the
+// gathers of the rounds fall on distinct LDS banks.  Programs that run on one
+// cell region (the adjoint's forward and transposed programs) share the slots
+// of reactions and pairs: `shared` are the other program's.
+struct LoweredSlots {
+  std::vector<int> factor;  // of the rounds' numbering (SparseSchedule::slotOf)
+  std::vector<int> pair;    // [64 pairRounds], the first nPairs are the derivative pairs
+  std::vector<int> rop;     // [64 ropRounds], the first nReac are the reactions
+};
+LoweredSlots chooseSlots(const MechTables& t, const SparseSchedule& s, const LoweredSlots* shared = nullptr);
 
 // Lowers the programs of `s` (built from `t`) for matrix entries of
 // bytesT bytes (4 or 8).  shift 0 when the cell region is at most 64 KiB,
@@ -98,6 +116,7 @@ struct LoweredProgram {
 // programs' extra sections; the cell layout depends on sizes only, so the
 // forward and transposed programs of one mechanism share it.  Throws
 // std::runtime_error when a field does not fit.
-LoweredProgram lowerProgram(const MechTables& t, const SparseSchedule& s, int bytesT, bool adjoint);
+LoweredProgram lowerProgram(const MechTables& t, const SparseSchedule& s, int bytesT, bool adjoint,
+                            const LoweredSlots& slots);
 
 }  // namespace tchem_amd

@@ -47,28 +47,38 @@ __device__ __forceinline__ unsigned lds_address(const char* p) {
 #endif
 }
 
-// the instruction stream, in device memory or staged in LDS
-template <bool STAGED>
+// The instruction stream, in device memory or staged in LDS.  With RSRC device
+// memory is read through a buffer resource: the lane's offset is one register
+// for all records of a size, the record's a scalar, and there is no vector
+// address arithmetic.  Measured, plain loads -> buffer loads: FP32 factors
+// (at their 128-register limit) 131040 CB05 cells 154.1 -> 145.5 ms; FP64
+// (registers to spare) 16411 cells 36.4 -> 37.4 ms, so only FP32 uses it.
+template <bool STAGED, bool RSRC>
 struct WordStream {
   const unsigned* g;  // device memory
   unsigned l;         // LDS address
-  template <typename V>
-  __device__ __forceinline__ V get(int word) const {
-#ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (STAGED) return lds_get<V>(l + 4u * unsigned(word));
-    return *(const __attribute__((address_space(1))) V*)(g + word);
-#else
-    return V();
-#endif
-  }
+  int bytes;          // stream length in device memory
   // record of this lane in round r of a section at word o
   template <typename V>
   __device__ __forceinline__ V rec(int o, int r, int lane) const {
     constexpr int w = int(sizeof(V) / 4);
     if constexpr (STAGED) return lds_get<V>(l + 4u * unsigned(o + 64 * w * r) + unsigned(4 * w * lane));
 #ifdef __HIP_DEVICE_COMPILE__
-    const auto* p = (const __attribute__((address_space(1))) char*)(g + o + 64 * w * r);
-    return *(const __attribute__((address_space(1))) V*)(p + unsigned(4 * w * lane));
+    if constexpr (!RSRC)
+      return *(const __attribute__((address_space(1))) V*)(g + o + 64 * w * r + w * lane);
+    const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned*>(g), 0, bytes, 0x00027000);
+    // readfirstlane keeps the uniform offset scalar whatever the loop optimiser does
+    const int v = 4 * w * lane, s = __builtin_amdgcn_readfirstlane(4 * (o + 64 * w * r));
+    if constexpr (w == 1) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(b, v, s, 0));
+    else if constexpr (w == 2) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(b, v, s, 0));
+    else if constexpr (w == 4) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(b, v, s, 0));
+    else {
+      static_assert(w == 8 || w <= 4, "record size");
+      struct Two { u32x4 a, b; } t;
+      t.a = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, v, s, 0));
+      t.b = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, v + 16, s, 0));
+      return __builtin_bit_cast(V, t);
+    }
 #else
     return V();
 #endif
@@ -82,8 +92,8 @@ struct WordStream {
       return (unsigned long long)p[0] | ((unsigned long long)p[1] << 32);
     }
 #endif
-    const unsigned lo = __builtin_amdgcn_readfirstlane(get<unsigned>(word));
-    const unsigned hi = __builtin_amdgcn_readfirstlane(get<unsigned>(word + 1));
+    const unsigned lo = __builtin_amdgcn_readfirstlane(lds_get<unsigned>(l + 4u * unsigned(word)));
+    const unsigned hi = __builtin_amdgcn_readfirstlane(lds_get<unsigned>(l + 4u * unsigned(word + 1)));
     return (unsigned long long)lo | ((unsigned long long)hi << 32);
   }
 };
@@ -125,8 +135,9 @@ __device__ __forceinline__ void rotate(int n, Load load, Exec exec) {
 template <typename TA_, bool STAGED_>
 struct SpLds {
   using TA = TA_;
-  WordStream<STAGED_> w;
-  __device__ __forceinline__ WordStream<false> memory() const { return WordStream<false>{w.g, 0u}; }
+  static constexpr bool RSRC = sizeof(TA) == 4;
+  WordStream<STAGED_, RSRC> w;
+  __device__ __forceinline__ WordStream<false, RSRC> memory() const { return WordStream<false, RSRC>{w.g, 0u, w.bytes}; }
   unsigned cell;      // cell region
   unsigned coef;      // coefficient table
   unsigned tol;       // (atol, rtol) per unknown
@@ -149,11 +160,14 @@ __device__ __forceinline__ void sp_init(const DevLowered& W, const L& S, int m, 
   wave_sync();
 }
 
-// After the cell's rate constants are in LDS: zeros up to the last full
-// round, and the n * kf slots.
+// The cell's rate constants into their slots, and the n * kf slots.
 template <int SH, typename L>
-__device__ __forceinline__ void sp_scaled_rates(const DevLowered& W, const L& S, int nReac, int lane) {
-  for (int r = nReac + lane; r < kWave * W.nRop; r += kWave) lds_put<double>(S.cell + W.oK + 8 * r, 0.0);
+__device__ __forceinline__ void sp_load_rates(const DevLowered& W, const L& S, const double* kf, int lane) {
+  for (int g = 0; g < W.nRop; ++g) {
+    const int r = int(S.w.template rec<unsigned>(W.oKf, g, lane));
+    lds_put<double>(S.cell + W.oK + 8 * (kWave * g + lane), r >= 0 ? kf[r] : 0.0);
+  }
+  wave_sync();
   for (int g = 0; g < W.nKfx; ++g) {
     const u32x2 x = S.w.template rec<u32x2>(W.oKfx, g, lane);
     lds_put<double>(at_lo<SH>(x.y, S.cell), lds_get<double>(S.cell + W.oK + 8 * x.x) * double(x.y >> 16));
@@ -263,7 +277,7 @@ __device__ __forceinline__ void sp_jacobian(const DevLowered& W, const L& S, int
     vec4<TA> c;
   };
   const unsigned cb = S.cell;
-  const WordStream<false> words = S.memory();
+  const auto words = S.memory();
   const int n4 = W.nJ4, n2 = n4 + W.nJ2;
   rotate<Rec>(
       n2 + W.nJ1,
@@ -321,16 +335,16 @@ __device__ __forceinline__ TA pivot_recip(TA p) {
 }
 
 // Rounds of the factorisation (and of the forward substitution with stored
-// factors).  Returns false when a pivot is zero or not finite.
-template <int SH, typename L, bool STAGED>
-__device__ __forceinline__ bool sp_lu(const L& S, const WordStream<STAGED>& words, int oHdr, int o4, int o1, int n, int lane) {
+// factors).
+template <int SH, typename L, typename Words>
+__device__ __forceinline__ void sp_lu(const L& S, const Words& words, int oHdr, int o4, int o1, int n,
+                                      int lane) {
   using TA = typename L::TA;
   struct Rec {
     u32x4 w;
     unsigned z;
   };
   const unsigned cb = S.cell;
-  bool bad = false;
   for (int r0 = 0; r0 < n; r0 += 64) {
     const unsigned long long mul = words.mask(oHdr + r0 / 16), upd = words.mask(oHdr + r0 / 16 + 2);
     rotate<Rec>(
@@ -343,11 +357,7 @@ __device__ __forceinline__ bool sp_lu(const L& S, const WordStream<STAGED>& word
           const unsigned t = at_lo<SH>(x.w.x, cb);
           if ((mul >> r) & 1) {
             const TA p = lds_get<TA>(at_hi<SH>(x.w.x, cb));
-            const TA a = lds_get<TA>(t);
-            const TA inv = pivot_recip(p);
-            lds_put<TA>(t, a * inv);
-            lds_put<TA>(at_lo<SH>(x.w.y, cb), inv);
-            bad |= (x.w.y & 0x20000u) && !(p != TA(0) && isfinite(p) && isfinite(inv));
+            lds_put<TA>(t, lds_get<TA>(t) * pivot_recip(p));
           } else if ((upd >> r) & 1) {
             TA acc = lds_get<TA>(t);
             const TA l0 = lds_get<TA>(at_hi<SH>(x.w.x, cb)), u0 = lds_get<TA>(at_lo<SH>(x.w.y, cb));
@@ -362,17 +372,35 @@ __device__ __forceinline__ bool sp_lu(const L& S, const WordStream<STAGED>& word
             const TA p = lds_get<TA>(at_hi<SH>(x.w.y, cb));
             const TA a = lds_get<TA>(at_hi<SH>(x.w.x, cb)), b = lds_get<TA>(at_lo<SH>(x.w.y, cb));
             TA acc = lds_get<TA>(t);
-            const TA l0 = lds_get<TA>(at_hi<SH>(x.w.z, cb)), u0 = lds_get<TA>(at_lo<SH>(x.w.w, cb));
-            const TA l1 = lds_get<TA>(at_hi<SH>(x.w.w, cb)), u1 = lds_get<TA>(at_lo<SH>(x.z, cb));
+            const TA l0 = lds_get<TA>(at_lo<SH>(x.w.z, cb)), u0 = lds_get<TA>(at_hi<SH>(x.w.z, cb));
+            const TA l1 = lds_get<TA>(at_lo<SH>(x.w.w, cb)), u1 = lds_get<TA>(at_hi<SH>(x.w.w, cb));
             const TA inv = pivot_recip(p);
             const TA l = a == TA(0) ? TA(0) : a * inv;
             acc = fma(-l0, u0, acc);
             acc = fma(-l1, u1, acc);
-            lds_put<TA>(t, (x.z & 0x10000u) ? l : fma(-l, b, acc));
-            lds_put<TA>(at_lo<SH>(x.w.z, cb), inv);
-            bad |= (x.z & 0x20000u) && !(p != TA(0) && isfinite(p) && isfinite(inv));
+            lds_put<TA>(t, at_hi<SH>(x.w.x, cb) == t ? l : fma(-l, b, acc));
           }
         });
+  }
+  wave_sync();
+}
+
+// Reciprocal pivots of the m rows, kept beside their right-hand sides (the
+// rounds multiply with the same values).  Returns false when a pivot is zero
+// or not finite.
+template <int SH, int QM, typename L>
+__device__ __forceinline__ bool sp_pivots(const DevLowered& W, const L& S, int m, int lane) {
+  using TA = typename L::TA;
+  bool bad = false;
+#pragma unroll
+  for (int q = 0; q < QM; ++q) {
+    const int i = lane + kWave * q;
+    if (i < m) {
+      const TA p = lds_get<TA>(S.cell + S.w.template rec<unsigned>(W.oDiag, q, lane));
+      const TA inv = pivot_recip(p);
+      lds_put<TA>(S.cell + W.oR + 2 * sizeof(TA) * i + sizeof(TA), inv);
+      bad |= !(p != TA(0) && isfinite(p) && isfinite(inv));
+    }
   }
   wave_sync();
   return ballot(bad) == 0;
@@ -421,6 +449,7 @@ __device__ __forceinline__ SpLds<TA, STAGED> carve_sparse(const DevLowered& W, c
   const unsigned b = lds_address(base);
   L.w.g = words;
   L.w.l = b;
+  L.w.bytes = 4 * W.words;
   L.coef = b + (STAGED ? 4u * unsigned(W.stagedWords) : 0u);
   L.tol = b + unsigned(sparseStageBytes(W, 0, STAGED));
   const size_t at = sparseStageBytes(W, m, STAGED) + size_t(wave) * size_t(cellBytes);

@@ -10,6 +10,7 @@
 // the stream may be touched.
 //
 // usage: lowered_check <mechanism.yaml> [<aerosol.yaml>]
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -153,6 +154,7 @@ struct Stream {
   const MechTables& t;
   std::vector<unsigned char> lds;
   bool bad = false;
+  std::vector<int> ropAt;  // slot of each reaction
   Stream(const LoweredProgram& p, const MechTables& t_) : P(p), d(p.d), t(t_), lds(size_t(p.d.cellBytes), 0xff) {}
   uint32_t word(int o) {
     CHECK(o >= 0 && o < d.words && o < int(P.words.size()), "stream word %d of %d", o, d.words);
@@ -191,7 +193,14 @@ struct Stream {
     put<T>(d.oR + 2 * int(sizeof(T)) * m + int(sizeof(T)), T(0));
     put<double>(d.oneC, 1.0);
     put<double>(d.zero8, 0.0);
-    for (int r = 0; r < 64 * d.nRop; ++r) put<double>(d.oK + 8 * r, r < t.nReac ? kf[size_t(r)] : 0.0);
+    ropAt.assign(size_t(t.nReac), -1);
+    for (int i = 0; i < 64 * d.nRop; ++i) {
+      const int r = int(word(d.oKf + i));
+      CHECK(r < t.nReac && (r < 0 || ropAt[size_t(r)] < 0), "reaction %d in slot %d", r, i);
+      if (r >= 0) ropAt[size_t(r)] = i;
+      put<double>(d.oK + 8 * i, r >= 0 ? kf[size_t(r)] : 0.0);
+    }
+    for (int r = 0; r < t.nReac; ++r) CHECK(ropAt[size_t(r)] >= 0, "reaction %d has no slot", r);
     for (int i = 0; i < 64 * d.nKfx; ++i) {
       const uint32_t w0 = word(d.oKfx + 2 * i), w1 = word(d.oKfx + 2 * i + 1);
       put<double>(lo(w1), get<double>(d.oK + 8 * int(w0)) * double(w1 >> 16));
@@ -298,12 +307,8 @@ struct Stream {
         w[4] = word(o1 + 64 * r + l);
         int f[10];
         for (int j = 0; j < 5; ++j) f[2 * j] = lo(w[j]), f[2 * j + 1] = hi(w[j]);
-        const unsigned flags = (bit(oHdr, r, 0) ? w[1] : w[4]) >> 16;
         if (bit(oHdr, r, 0)) {
-          const T p = get<T>(f[1]), inv = T(1) / p;
-          out.push_back({f[0], get<T>(f[0]) * inv});
-          out.push_back({f[2], inv});
-          bad |= (flags & 2) && !(p != T(0) && std::isfinite(p) && std::isfinite(inv));
+          out.push_back({f[0], get<T>(f[0]) * (T(1) / get<T>(f[1]))});
         } else if (bit(oHdr, r, 1)) {
           T acc = get<T>(f[0]);
           for (int j = 0; j < 4; ++j) acc = fmaT(-get<T>(f[1 + 2 * j]), get<T>(f[2 + 2 * j]), acc);
@@ -312,13 +317,18 @@ struct Stream {
           const T p = get<T>(f[3]), a = get<T>(f[1]), b = get<T>(f[2]), inv = T(1) / p;
           const T lv = a == T(0) ? T(0) : a * inv;
           T acc = get<T>(f[0]);
-          for (int j = 0; j < 2; ++j) acc = fmaT(-get<T>(f[5 + 2 * j]), get<T>(f[6 + 2 * j]), acc);
-          out.push_back({f[0], (flags & 1) ? lv : fmaT(-lv, b, acc)});
-          out.push_back({f[4], inv});
-          bad |= (flags & 2) && !(p != T(0) && std::isfinite(p) && std::isfinite(inv));
+          for (int j = 0; j < 2; ++j) acc = fmaT(-get<T>(f[4 + 2 * j]), get<T>(f[5 + 2 * j]), acc);
+          out.push_back({f[0], f[1] == f[0] ? lv : fmaT(-lv, b, acc)});
         }
       }
       flush<T>(out);
+    }
+  }
+  void pivots(int m) {
+    for (int i = 0; i < m; ++i) {
+      const T p = get<T>(int(word(d.oDiag + i))), inv = T(1) / p;
+      put<T>(d.oR + 2 * int(sizeof(T)) * i + int(sizeof(T)), inv);
+      bad |= !(p != T(0) && std::isfinite(p) && std::isfinite(inv));
     }
   }
   void back() {
@@ -337,14 +347,19 @@ struct Stream {
 
 template <typename T>
 static void check(const MechTables& t, const SS& s, const SS& partner, bool adjoint, const char* what) {
-  const LoweredProgram P = lowerProgram(t, s, int(sizeof(T)), adjoint);
+  // adjoint programs share the slots of the forward one
+  const LoweredSlots fs = chooseSlots(t, s.transposed ? partner : s);
+  const LoweredProgram P = lowerProgram(t, s, int(sizeof(T)), adjoint, s.transposed ? chooseSlots(t, s, &fs) : fs);
   const DevLowered& d = P.d;
   std::printf("%s FP%zu: cell %d B, stream %d words, shift %d, rounds rop %d pair %d seg %d row %d jac %d+%d+%d join %d lu %d back %d fwd %d\n",
               what, 8 * sizeof(T), d.cellBytes, d.words, d.shift, d.nRop, d.nPair, d.nSeg, d.nRow[0] + d.nRow[1], d.nJ4, d.nJ2,
               d.nJ1, d.nJx, d.nLu, d.nBack, d.nFwd);
   CHECK(d.words == int(P.words.size()) && d.nCoef == int(P.coef.size()) && d.cellBytes % 16 == 0, "sizes");
   if (adjoint) {  // forward and transposed programs run on one cell layout
-    const DevLowered e = lowerProgram(t, partner, int(sizeof(T)), true).d;
+    const LoweredProgram Q = lowerProgram(t, partner, int(sizeof(T)), true, partner.transposed ? chooseSlots(t, partner, &fs) : fs);
+    const DevLowered& e = Q.d;
+    for (int i = 0; i < 64 * d.nRop; ++i)
+      CHECK(P.words[size_t(d.oKf + i)] == Q.words[size_t(e.oKf + i)], "slot %d holds another reaction", i);
     CHECK(d.zeroA == e.zeroA && d.oR == e.oR && d.oD == e.oD && d.oC == e.oC && d.oneC == e.oneC && d.oK == e.oK && d.nK == e.nK &&
               d.zero8 == e.zero8 && d.oP == e.oP && d.oS == e.oS && d.oMu == e.oMu && d.oW == e.oW && d.oV == e.oV && d.shift == e.shift,
           "cell layouts of the forward and transposed programs differ");
@@ -362,8 +377,15 @@ static void check(const MechTables& t, const SS& s, const SS& partner, bool adjo
     S.init(kf, m);
     S.rates(c);
     R.rates(c, kf);
-    for (int r = 0; r < t.nReac; ++r) CHECK(same(R.rop[size_t(r)], S.template get<double>(d.oP + 8 * r)), "rate of progress %d", r);
-    for (int p = 0; p < t.nPairs(); ++p) CHECK(same(R.dpr[size_t(p)], S.template get<T>(d.oD + int(sizeof(T)) * p)), "pair %d", p);
+    for (int r = 0; r < t.nReac; ++r) CHECK(same(R.rop[size_t(r)], S.template get<double>(d.oP + 8 * S.ropAt[size_t(r)])), "rate of progress %d", r);
+    {  // derivative pairs, in some order of slots (the matrix entries below tell which)
+      std::vector<T> x(R.dpr.begin(), R.dpr.begin() + t.nPairs()), y;
+      for (int p = 0; p < 64 * d.nPair; ++p) y.push_back(S.template get<T>(d.oD + int(sizeof(T)) * p));
+      x.resize(y.size(), T(0));
+      std::sort(x.begin(), x.end());
+      std::sort(y.begin(), y.end());
+      CHECK(x == y, "derivative pairs");
+    }
     R.eval(1.0, -ch);
     S.segments();
     const int rows = int(t.rowSegPtr.size()) - 1;
@@ -373,7 +395,7 @@ static void check(const MechTables& t, const SS& s, const SS& partner, bool adjo
       CHECK(same(f, S.row(a, t.emission[size_t(a)])), "source term of species %d", a);
     }
     S.jacobian(T(-ch));
-    for (int p = 0; p < s.nnzF; ++p) CHECK(same(R.A[size_t(p)], S.template get<T>(int(sizeof(T)) * p)), "matrix slot %d", p);
+    for (int p = 0; p < s.nnzF; ++p) CHECK(same(R.A[size_t(p)], S.template get<T>(int(sizeof(T)) * P.slot[size_t(p)])), "matrix slot %d", p);
     for (int pass = 0; pass < 2; ++pass) {  // factorise and solve, then solve again with the stored factors
       for (int i = 0; i < m; ++i) {
         const T b = T(U(rng) - 0.5);
@@ -383,12 +405,13 @@ static void check(const MechTables& t, const SS& s, const SS& partner, bool adjo
       if (pass == 0) {
         R.run(0, s.luRounds, 0);
         S.lu(d.oLuHdr, d.oLu, d.oLu1, d.nLu);
+        S.pivots(m);
       } else {
         R.run(s.luRounds + s.backRounds, s.fwdRounds, size_t(s.fwdBody));
         S.lu(d.oFwdHdr, d.oFwd, d.oFwd1, d.nFwd);
       }
       CHECK(R.bad == S.bad && !R.bad, "pivots");
-      for (int p = 0; p < s.nnzF; ++p) CHECK(same(R.A[size_t(p)], S.template get<T>(int(sizeof(T)) * p)), "factor slot %d", p);
+      for (int p = 0; p < s.nnzF; ++p) CHECK(same(R.A[size_t(p)], S.template get<T>(int(sizeof(T)) * P.slot[size_t(p)])), "factor slot %d", p);
       R.run(s.luRounds, s.backRounds, size_t(s.backBody));
       S.back();
       for (int i = 0; i < m; ++i) {
@@ -411,7 +434,7 @@ static void check(const MechTables& t, const SS& s, const SS& partner, bool adjo
           double& x = v[size_t(R.spec(r, t.pairSlot[p]))];
           x = fmaT(double(R.dpr[size_t(p)]), w[size_t(r)], x);
         }
-      for (int r = 0; r < t.nReac; ++r) CHECK(same(w[size_t(r)], S.template get<double>(int(S.word(d.oWmap + r)))), "w %d", r);
+      for (int r = 0; r < t.nReac; ++r) CHECK(same(w[size_t(r)], S.template get<double>(int(S.word(d.oWmap + S.ropAt[size_t(r)])))), "w %d", r);
       for (int i = 0; i < m; ++i) CHECK(same(v[size_t(i)], S.template get<double>(int(S.word(d.oVmap + i)))), "v %d", i);
     }
   }
