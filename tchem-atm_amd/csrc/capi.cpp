@@ -38,6 +38,7 @@ hipError_t launchAutotuneSample(int n, long long stride, int nb, int np, int ite
                                 tchem_time_advance_t* ta, double* tt0, int* live, hipStream_t stream);
 hipError_t launchCopyWords(void* dst, const void* src, size_t words, hipStream_t stream);
 size_t mfmaCellLdsBytes(const DevMech& M);
+size_t mfmaLaunchLdsBytes(const DevMech& M);
 hipError_t launchDenseMfmaSolve(int n, int nBatch, const double* A, const double* b, double* x, hipStream_t stream);
 hipError_t noAllocScratch(void** ptr, size_t* bytes);
 hipError_t launchRates(const DevMech& M, int nBatch, const double* state, const double* photo, const double* lscale,
@@ -312,6 +313,12 @@ size_t ldsBytes(const tchem_kmcd_s* k, const tchem_atmchem_options_t& o) {
   return integratorLdsBytes(k->dev, bytesA);
 }
 
+// LDS bytes the launch asks for (the MFMA instance of a small order needs
+// less than the form's bound)
+size_t launchLdsBytes(const tchem_kmcd_s* k, const tchem_atmchem_options_t& o) {
+  return o.lu == TCHEM_LU_MFMA ? mfmaLaunchLdsBytes(k->dev) : ldsBytes(k, o);
+}
+
 // Grows the per-cell rate-constant buffer to nBatch cells (allocation only
 // when a larger batch arrives; the previous buffer may still be read by work
 // queued on s, so s is synchronised first).
@@ -337,7 +344,7 @@ int resolveBlocksPerCU(const tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& 
   if (*bpc > 0) return TCHEM_OK;
   const int sparse = o.lu == TCHEM_LU_MFMA ? 3 : (o.lu == TCHEM_LU_SPARSE ? (sparseStaged(o) ? 1 : 2) : 0);
   hipError_t e = integratorMaxBlocksPerCU(o.precision, sparse, kmcd->dev.m, kmcd->lowered(o.precision),
-                                          64 * o.cells_per_block, ldsBytes(kmcd, o), bpc, rec);
+                                          64 * o.cells_per_block, launchLdsBytes(kmcd, o), bpc, rec);
   if (e != hipSuccess) return hipFail(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
   if (*bpc < 1) *bpc = 1;
   return TCHEM_OK;
@@ -347,7 +354,7 @@ int resolveBlocksPerCU(const tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& 
 // launch for the resolved options; a carries the per-call arrays.
 int runIntegrator(tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& o, const double* lscale, int lstride,
                   IntegratorArgs& a, hipStream_t s, const char* who, bool ratesReady = false) {
-  const size_t lds = ldsBytes(kmcd, o);
+  const size_t lds = launchLdsBytes(kmcd, o);
   if (lds > kmcd->maxLds)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": mechanism needs " + std::to_string(lds) +
                                                " bytes of LDS per workgroup, device limit " +

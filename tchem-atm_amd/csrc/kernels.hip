@@ -1002,9 +1002,10 @@ __device__ __forceinline__ void derivative_pairs(const DevMech& M, const double*
 // LDS bytes of one cell of the MFMA form: the dense cell region without a
 // matrix, the FP32 derivative pairs, the source term, then the
 // factorisation's region
-inline size_t mfmaCellBytes(const DevMech& M) {
+inline size_t mfmaCellBytes(const DevMech& M, int tiles) {
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-  return al(integratorLdsBytes(M, 0)) + al(4 * size_t(M.nPairs + 1)) + al(8 * size_t(M.m)) + mfma::luLdsBytes();
+  return al(integratorLdsBytes(M, 0)) + al(4 * size_t(M.nPairs + 1)) + al(8 * size_t(M.m)) +
+         mfma::luLdsBytes(tiles);
 }
 
 // The source term by the whole workgroup (256 threads): rates of progress,
@@ -1029,9 +1030,10 @@ __device__ void mfma_rhs_collective(const IntegratorArgs& a, const Lds& L) {
   __syncthreads();
 }
 
-template <int QM>
+template <int NB_>
 struct MfmaBackend {
   using TA = float;
+  static constexpr int NB = NB_, QM = NB / 2;  // 64 unknowns per slot, 32 per tile
   static constexpr bool kCollective = true;  // factorisation by the whole workgroup (collective_solve)
   struct Lds : CellLds<float> {
     float* pairs;   // [nPairs] derivative pairs of the last Jacobian refresh (FP32)
@@ -1064,7 +1066,7 @@ struct MfmaBackend {
     off += al(4 * size_t(a.M.nPairs + 1));
     L.fbuf = reinterpret_cast<double*>(base + off);
     off += al(8 * size_t(a.M.m));
-    L.lu = mfma::carveLu(base + off);
+    L.lu = mfma::carveLu(base + off, NB);
     return L;
   }
   static __device__ void init(const IntegratorArgs&, const Lds&, int) {}
@@ -1106,11 +1108,11 @@ struct MfmaBackend {
 };
 
 // Assembly of I - c h J (FP32 sums of the serial Jacobian lists) plus the
-// identity padding and the right-hand side (stashed in z) as column 255,
-// by column quarters through LDS into the tiles of the four wavefronts,
+// identity padding and the right-hand side (stashed in z) as the last column,
+// by strips of 64 columns through LDS into the tiles of the four wavefronts,
 // then the factorisation and back substitution.
-template <int QM>
-__device__ __forceinline__ void mfma_collective(const IntegratorArgs& a, const typename MfmaBackend<QM>::Lds& L,
+template <int NB>
+__device__ __forceinline__ void mfma_collective(const IntegratorArgs& a, const typename MfmaBackend<NB>::Lds& L,
                                                 int wave, int lane) {
 #pragma clang fp contract(off)
   using namespace mfma;
@@ -1121,12 +1123,13 @@ __device__ __forceinline__ void mfma_collective(const IntegratorArgs& a, const t
   if (L.lu.cmd[2]) derivative_pairs(M, L.c, L.kf, L.pairs, tid, 256);  // refresh: pairs of the current iterate
   TCHEM_PT_END(dp, 1)
   const float scale = float(-*L.lu.ch);
-  f32x16 acc[16];
+  f32x16 acc[NB * NB / 4];
   TCHEM_PT_BEGIN(asm)
+  constexpr int rows = kTile * NB;
   float4* stage4 = reinterpret_cast<float4*>(L.lu.stage);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {  // unrolled: the tiles of quarter q are known at compile time
-    for (int idx = tid; idx < int(kStageWords / 4); idx += 256) stage4[idx] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int q = 0; q < NB / 2; ++q) {  // unrolled: the tiles of strip q are known at compile time
+    for (int idx = tid; idx < rows * 65 / 4; idx += 256) stage4[idx] = float4{0.0f, 0.0f, 0.0f, 0.0f};
     __syncthreads();
     {  // this thread's run of terms: coalesced, independent loads
       const int j1 = M.mfjQuarter()[q + 1];
@@ -1141,30 +1144,30 @@ __device__ __forceinline__ void mfma_collective(const IntegratorArgs& a, const t
         }
       }
     }
-    for (int p = m + tid; p < kN - 1; p += 256)
+    for (int p = m + tid; p < rows - 1; p += 256)
       if ((p >> 6) == q) L.lu.stage[p * 65 + (p - 64 * q)] = 1.0f;
-    if (q == 3) {
+    if (q == NB / 2 - 1) {
       for (int i = tid; i < m; i += 256) L.lu.stage[i * 65 + 63] = L.lu.z[i];
-      if (tid == 0) L.lu.stage[(kN - 1) * 65 + 63] = 1.0f;
+      if (tid == 0) L.lu.stage[(rows - 1) * 65 + 63] = 1.0f;
     }
     __syncthreads();
-    if (q == 0) loadQuarter<0>(acc, L.lu.stage, wave, lane);
-    if (q == 1) loadQuarter<1>(acc, L.lu.stage, wave, lane);
-    if (q == 2) loadQuarter<2>(acc, L.lu.stage, wave, lane);
-    if (q == 3) loadQuarter<3>(acc, L.lu.stage, wave, lane);
+    if constexpr (NB >= 2) if (q == 0) loadStrip<NB, 0>(acc, L.lu.stage, wave, lane);
+    if constexpr (NB >= 4) if (q == 1) loadStrip<NB, 1>(acc, L.lu.stage, wave, lane);
+    if constexpr (NB >= 6) if (q == 2) loadStrip<NB, 2>(acc, L.lu.stage, wave, lane);
+    if constexpr (NB >= 8) if (q == 3) loadStrip<NB, 3>(acc, L.lu.stage, wave, lane);
     __syncthreads();
   }
   TCHEM_PT_END(asm, 4)
-  factorAndSolve(acc, L.lu, wave, lane);
+  factorAndSolve<NB>(acc, L.lu, wave, lane);
 }
 
-template <int QM>
-__device__ bool MfmaBackend<QM>::factor_solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM], Fact&) {
+template <int NB>
+__device__ bool MfmaBackend<NB>::factor_solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM], Fact&) {
   return collective_solve(a, L, lane, x, true);
 }
 
-template <int QM>
-__device__ bool MfmaBackend<QM>::collective_solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM],
+template <int NB>
+__device__ bool MfmaBackend<NB>::collective_solve(const IntegratorArgs& a, const Lds& L, int lane, TA (&x)[QM],
                                                   bool refresh) {
   const int m = a.M.m;
 #pragma unroll
@@ -1178,8 +1181,8 @@ __device__ bool MfmaBackend<QM>::collective_solve(const IntegratorArgs& a, const
     L.lu.cmd[2] = refresh ? 1 : 0;
   }
   __syncthreads();  // hands the matrix to the workgroup
-  mfma_collective<QM>(a, L, 0, lane);
-  // x = -(U^-1 e_255)[0..m)
+  mfma_collective<NB>(a, L, 0, lane);
+  // x = -(U^-1 e_last)[0..m)
 #pragma unroll
   for (int q = 0; q < QM; ++q) {
     const int i = lane + kWave * q;
@@ -1191,12 +1194,13 @@ __device__ bool MfmaBackend<QM>::collective_solve(const IntegratorArgs& a, const
   return ok;
 }
 
-template <int QM>
+template <int NB>
 __global__ __launch_bounds__(256, 1) void trbdf2_mfma_kernel(IntegratorArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   if (a.skip && __builtin_amdgcn_readfirstlane(*a.skip)) return;
   TCHEM_PT_RESET()
-  using B = MfmaBackend<QM>;
+  using B = MfmaBackend<NB>;
+  constexpr int QM = B::QM;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // uniform: tile choices are scalar branches
   typename B::Lds L = B::carve(lds_raw, a, 0);
@@ -1209,7 +1213,7 @@ __global__ __launch_bounds__(256, 1) void trbdf2_mfma_kernel(IntegratorArgs a) {
       if (cmd == 2) {
         mfma_rhs_collective(a, L);
       } else {
-        mfma_collective<QM>(a, L, wave, lane);
+        mfma_collective<NB>(a, L, wave, lane);
       }
     }
     return;
@@ -1233,37 +1237,53 @@ __global__ __launch_bounds__(256, 1) void trbdf2_mfma_kernel(IntegratorArgs a) {
 
 // Batched dense solve A x = b (n <= 255, FP64 in and out, FP32 MFMA
 // factorisation without interchanges): the LU of the MFMA form on its own.
-__global__ __launch_bounds__(256, 1) void dense_mfma_solve_kernel(int n, int nBatch, const double* A, const double* b,
-                                                                  double* x) {
+// Every wavefront reads its tiles of [A | b | padding] straight into the
+// registers of the C layout (a register of a tile is two rows of 32
+// consecutive columns), with all loads of a tile row in flight.
+template <int NB>
+__global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void dense_mfma_solve_kernel(int n, int nBatch, const double* A,
+                                                                                const double* b, double* x) {
   extern __shared__ __align__(16) char lds_raw[];
   using namespace mfma;
+  constexpr int T = NB / 2;
   const int cell = blockIdx.x;
   if (cell >= nBatch) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);  // uniform: tile choices are scalar branches
-  const Lu L = carveLu(lds_raw);
+  const Lu L = carveLu(lds_raw, NB);
   const double* Ac = A + size_t(cell) * n * n;
   const double* bc = b + size_t(cell) * n;
   if (threadIdx.x == 0) L.cmd[1] = 0;
-  f32x16 acc[16];
-  // [A | b] padded with the identity, by column quarters through LDS
+  f32x16 acc[T * T];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    for (int idx = threadIdx.x; idx < kN * 64; idx += blockDim.x) {
-      const int row = idx >> 6, col = 64 * q + (idx & 63);
-      float v = (row == col) ? 1.0f : 0.0f;
-      if (row < n && col < n) v = float(Ac[size_t(row) * n + col]);
-      else if (col == kN - 1) v = row < n ? float(bc[row]) : (row == kN - 1 ? 1.0f : 0.0f);
-      L.stage[row * 65 + (idx & 63)] = v;
+  for (int o = 0; o < T; ++o) {
+#pragma unroll
+    for (int p = 0; p < T; ++p) {
+      const int i0 = kTile * (2 * o + (wave >> 1)), j = kTile * (2 * p + (wave & 1)) + (lane & 31);
+      double v[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = i0 + crow(r, lane);
+        const int ic = i < n ? i : n - 1, jc = j < n ? j : n - 1;
+        v[r] = Ac[ic * n + jc];
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = i0 + crow(r, lane);
+        acc[o * T + p][r] = (i < n && j < n) ? float(v[r]) : (i == j ? 1.0f : 0.0f);
+      }
+      if (p == T - 1 && (wave & 1)) {  // the right-hand side: column 31 of the last block column
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int i = i0 + crow(r, lane);
+          const double rhs = bc[i < n ? i : n - 1];
+          if (j == kTile * NB - 1 && i < n) acc[o * T + p][r] = float(rhs);
+        }
+      }
+      if (p & 1) __builtin_amdgcn_sched_barrier(0);  // two tiles' loads in flight, not all (registers)
     }
-    __syncthreads();
-    if (q == 0) loadQuarter<0>(acc, L.stage, wave, lane);
-    if (q == 1) loadQuarter<1>(acc, L.stage, wave, lane);
-    if (q == 2) loadQuarter<2>(acc, L.stage, wave, lane);
-    if (q == 3) loadQuarter<3>(acc, L.stage, wave, lane);
-    __syncthreads();
   }
-  factorAndSolve(acc, L, wave, lane);
+  factorAndSolve<NB>(acc, L, wave, lane);
   for (int i = threadIdx.x; i < n; i += blockDim.x) x[size_t(cell) * n + i] = L.cmd[1] ? NAN : -double(L.z[i]);
 }
 
@@ -2214,12 +2234,12 @@ int sparseMaxCellsPerGroup(int precision, int m) {
 // 2 programs in device memory; species slots per lane; recording for the
 // adjoint, FP64 sparse forms only; cells per workgroup); nullptr when there
 // is none
-static const void* integratorKernel(int precision, int sparse, int qm, bool rec, int cells) {
+static const void* integratorKernel(int precision, int sparse, int qm, bool rec, int cells, int mfmaTiles) {
   if (sparse == 3) {  // dense LU on the matrix cores: mixed precision only
     if (rec || precision != TCHEM_PRECISION_MIXED) return nullptr;
-    return qm == 1 ? reinterpret_cast<const void*>(&trbdf2_mfma_kernel<1>)
-                   : (qm == 2 ? reinterpret_cast<const void*>(&trbdf2_mfma_kernel<2>)
-                              : reinterpret_cast<const void*>(&trbdf2_mfma_kernel<4>));
+    return mfmaTiles == 4 ? reinterpret_cast<const void*>(&trbdf2_mfma_kernel<4>)
+                          : (mfmaTiles == 6 ? reinterpret_cast<const void*>(&trbdf2_mfma_kernel<6>)
+                                            : reinterpret_cast<const void*>(&trbdf2_mfma_kernel<8>));
   }
 #define TCHEM_PICK_D(TA) \
   return qm == 1 ? integratorFn<DenseBackend<TA, 1>, 1, 64>() \
@@ -2260,7 +2280,8 @@ static const void* integratorKernel(int precision, int sparse, int qm, bool rec,
 hipError_t launchIntegrator(const IntegratorArgs& a, int precision, int grid, size_t lds, hipStream_t stream) {
   const int qm = qmOf(a.M.m, a.sparse == 1 || a.sparse == 2 ? &a.W : nullptr);
   if (qm == 0) return hipErrorInvalidValue;
-  const void* fn = integratorKernel(precision, a.sparse, qm, a.rec.h != nullptr, a.cellsPerGroup);
+  const void* fn = integratorKernel(precision, a.sparse, qm, a.rec.h != nullptr, a.cellsPerGroup,
+                                    mfma::tilesFor(a.M.m));
   if (!fn) return hipErrorInvalidValue;
   hipFuncAttributes attr;
   const hipError_t ea = hipFuncGetAttributes(&attr, fn);
@@ -2277,7 +2298,7 @@ size_t integratorStaticLds(int precision, int sparse, int m, const DevLowered& w
   const int qm = qmOf(m, &w);
   if (qm == 0) return 0;
   hipFuncAttributes attr;
-  if (hipFuncGetAttributes(&attr, integratorKernel(precision, sparse, qm, false, 1)) != hipSuccess) return 0;
+  if (hipFuncGetAttributes(&attr, integratorKernel(precision, sparse, qm, false, 1, mfma::tilesFor(m))) != hipSuccess) return 0;
   return attr.sharedSizeBytes;
 }
 
@@ -2285,7 +2306,7 @@ hipError_t integratorMaxBlocksPerCU(int precision, int sparse, int m, const DevL
                                     int* blocks, bool rec) {
   const int qm = qmOf(m, sparse == 1 || sparse == 2 ? &w : nullptr);
   if (qm == 0) return hipErrorInvalidValue;
-  const void* fn = integratorKernel(precision, sparse, qm, rec, threads / 64);
+  const void* fn = integratorKernel(precision, sparse, qm, rec, threads / 64, mfma::tilesFor(m));
   if (sparse == 3) threads = 256;
   if (!fn) return hipErrorInvalidValue;
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks, fn, threads, lds);
@@ -2491,12 +2512,16 @@ hipError_t noAllocScratch(void** ptr, size_t* bytes) {
   return hipSuccess;
 }
 
-size_t mfmaCellLdsBytes(const DevMech& M) { return mfmaCellBytes(M); }
+// LDS of a cell with all 8 x 8 tiles: which mechanisms the form takes
+size_t mfmaCellLdsBytes(const DevMech& M) { return mfmaCellBytes(M, 8); }
+// LDS of the instance that runs
+size_t mfmaLaunchLdsBytes(const DevMech& M) { return mfmaCellBytes(M, mfma::tilesFor(M.m)); }
 
 hipError_t launchDenseMfmaSolve(int n, int nBatch, const double* A, const double* b, double* x, hipStream_t stream) {
   if (nBatch <= 0) return hipSuccess;
-  hipLaunchKernelGGL(dense_mfma_solve_kernel, dim3(nBatch), dim3(256), mfma::luLdsBytes(), stream, n, nBatch, A, b,
-                     x);
+  const int tiles = mfma::tilesFor(n);
+  auto* fn = tiles == 4 ? dense_mfma_solve_kernel<4> : (tiles == 6 ? dense_mfma_solve_kernel<6> : dense_mfma_solve_kernel<8>);
+  hipLaunchKernelGGL(fn, dim3(nBatch), dim3(256), mfma::luLdsBytes(tiles), stream, n, nBatch, A, b, x);
   return hipGetLastError();
 }
 
