@@ -299,6 +299,9 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   return TCHEM_OK;
 }
 
+// whether the caller left the cells per workgroup to the library
+bool autoCells(const tchem_atmchem_options_t* opts) { return !opts || opts->cells_per_block == 0; }
+
 // whether the sparse programs are staged into LDS (resolved options)
 bool sparseStaged(const tchem_atmchem_options_t& o) { return o.programs == TCHEM_PROGRAMS_LDS; }
 
@@ -350,10 +353,32 @@ int resolveBlocksPerCU(const tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& 
   return TCHEM_OK;
 }
 
+// Cells per workgroup for a batch, at most `most` (the LDS of a CU holds that
+// many).  A wavefront alone on its SIMD goes through its rounds faster than
+// one of three or four, so a batch smaller than the chip is spread over all
+// CUs.  Full workgroups -> spread: CB05 FP64, 6 x 10 iterations, 363 cells
+// 4196 -> 3257 us, 2000 cells 4270 -> 3708 us; mixed 1000 cells, 80 iterations
+// 5197 -> 4223 us; CB05 + SOA 500 cells 8331 -> 7179 us; gradient of 500 cells
+// 236 -> 214 ms.  With even, a grid of w such batches has w even ones instead
+// of full ones and a remainder: FP64 4000 cells 8324 -> 7334 us, 6000 12317 ->
+// 10883 us; not for a work queue, which evens itself out, nor for the mixed
+// and aerosol forms (5000 cells mixed 8678 -> 8840 us, CB05 + SOA 24.5 -> 24.7 ms).
+int cellsForBatch(int nBatch, int most, int numCUs, bool even) {
+  const long long chip = (long long)most * numCUs;
+  const long long waves = (nBatch + chip - 1) / chip;
+  if (waves > 1 && !even) return most;
+  return int(std::max<long long>(1, (nBatch + waves * numCUs - 1) / std::max<long long>(1, waves * numCUs)));
+}
+
 // Rate constants (optionally log-scaled) into a.kf, then the integrator
-// launch for the resolved options; a carries the per-call arrays.
-int runIntegrator(tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& o, const double* lscale, int lstride,
+// launch for the resolved options; a carries the per-call arrays.  With
+// spread the cells per workgroup were left to the library.
+int runIntegrator(tchem_kmcd_s* kmcd, tchem_atmchem_options_t o, bool spread, const double* lscale, int lstride,
                   IntegratorArgs& a, hipStream_t s, const char* who, bool ratesReady = false) {
+  if (spread && o.lu == TCHEM_LU_SPARSE)
+    o.cells_per_block =
+        cellsForBatch(a.nBatch, o.cells_per_block, kmcd->numCUs,
+                      o.schedule == TCHEM_SCHEDULE_GRID && o.precision == TCHEM_PRECISION_FP64);
   const size_t lds = launchLdsBytes(kmcd, o);
   if (lds > kmcd->maxLds)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": mechanism needs " + std::to_string(lds) +
@@ -928,7 +953,7 @@ int tchem_atmchem_run_device_batch(const tchem_atmchem_options_t* opts, int nBat
   a.state_out = state_out;
   a.stats = stats;
   a.kf = kmcd->kf;
-  return runIntegrator(kmcd, o, nullptr, 0, a, s, "run_device_batch");
+  return runIntegrator(kmcd, o, autoCells(opts), nullptr, 0, a, s, "run_device_batch");
 }
 
 int tchem_atmchem_run_device_batch_noalloc(const tchem_atmchem_options_t* opts, int nBatch,
@@ -974,7 +999,7 @@ int tchem_atmchem_run_device_batch_noalloc(const tchem_atmchem_options_t* opts, 
   a.stats = stats;
   a.kf = static_cast<double*>(scr);
   a.queue = reinterpret_cast<int*>(static_cast<char*>(scr) + kfBytes);
-  return runIntegrator(kmcd, o, nullptr, 0, a, static_cast<hipStream_t>(stream), who);
+  return runIntegrator(kmcd, o, autoCells(opts), nullptr, 0, a, static_cast<hipStream_t>(stream), who);
 }
 
 int tchem_dense_lu_solve_mfma(int n, int nBatch, const double* A, const double* b, double* x, void* stream) {
@@ -1027,7 +1052,7 @@ int tchem_atmchem_e3sm_run_device_batch(const tchem_atmchem_options_t* opts, int
   a.stats = stats;
   a.kf = kmcd->kf;
   a.ext = external_sources;
-  return runIntegrator(kmcd, o, nullptr, 0, a, s, who, true);
+  return runIntegrator(kmcd, o, autoCells(opts), nullptr, 0, a, s, who, true);
 }
 
 int tchem_atmchem_update_time_advance(int nBatch, tchem_time_advance_t* tadv, const double* t_out,
@@ -1127,7 +1152,7 @@ int tchem_adjoint_forward(int nBatch, const double* tol_newton, const double* to
   a.rec.ckpt = reinterpret_cast<double*>(ws + W.ckpt);
   a.rec.consts = reinterpret_cast<double*>(ws + W.consts);
   a.rec.maxSteps = maxSteps;
-  return runIntegrator(kmcd, o, log_rate_scale, log_rate_scale_stride, a, s, who);
+  return runIntegrator(kmcd, o, true, log_rate_scale, log_rate_scale_stride, a, s, who);
 }
 
 int tchem_adjoint_backward(int nBatch, const double* lambda, double* lambda_out, double* grad, void* workspace,
@@ -1152,6 +1177,7 @@ int tchem_adjoint_backward(int nBatch, const double* lambda, double* lambda_out,
   if (stageB + cellB > kmcd->maxLds)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": one cell needs " + std::to_string(cellB) +
                                                " bytes of LDS, device limit " + std::to_string(kmcd->maxLds));
+  cpg = cellsForBatch(nBatch, cpg, kmcd->numCUs, false);
   const size_t lds = stageB + size_t(cpg) * cellB;
   const AdjointLayout W = adjointLayout(M, nBatch, maxSteps);
   char* ws = static_cast<char*>(workspace);
@@ -1278,7 +1304,7 @@ int tchem_atmchem_graph_create(const tchem_atmchem_options_t* opts, int nBatch, 
     a.stats = stats;
     a.kf = g->kf;
     a.queue = g->ctl + 64;
-    rc = runIntegrator(kmcd, o, nullptr, 0, a, cs, who);
+    rc = runIntegrator(kmcd, o, autoCells(opts), nullptr, 0, a, cs, who);
     if (rc == TCHEM_OK) {
       e = launchUpdateTadv(nBatch, tadv, t_out, dt_out, g->ctl, cs);
       if (e != hipSuccess) rc = hipFail(e, "update_tadv_kernel");
@@ -1438,7 +1464,7 @@ int tchem_atmchem_autotune(tchem_atmchem_options_t* opts, int nBatch, const doub
     // (under some profilers they complete early); a trial runs for ms
     if ((ex = hipStreamSynchronize(s)) != hipSuccess) return hipFail(ex, "hipStreamSynchronize");
     const auto t0 = std::chrono::steady_clock::now();
-    const int r = runIntegrator(kmcd, o, nullptr, 0, a, s, who);
+    const int r = runIntegrator(kmcd, o, false, nullptr, 0, a, s, who);
     if (r) return r;
     if ((ex = hipStreamSynchronize(s)) != hipSuccess) return hipFail(ex, "hipStreamSynchronize");
     *ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1830,7 +1856,7 @@ int tchem_aerosolchem_run_device_batch(const tchem_atmchem_options_t* opts, int 
     if (cells > 8) cells = 8;
   }
   if (cells < 1) return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": one cell does not fit the LDS");
-  const int perGroup = cells < nBatch ? cells : nBatch;
+  const int perGroup = cellsForBatch(nBatch, cells, k->numCUs, false);
   a.cellsPerGroup = perGroup;
   const int grid = (nBatch + perGroup - 1) / perGroup;
   e = launchAerosol(a, grid, stageB + size_t(perGroup) * size_t(a.cellBytes), s);
