@@ -357,7 +357,7 @@ int resolveBlocksPerCU(const tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& 
 // many).  A wavefront alone on its SIMD goes through its rounds faster than
 // one of three or four, so a batch smaller than the chip is spread over all
 // CUs.  Full workgroups -> spread: CB05 FP64, 6 x 10 iterations, 363 cells
-// 4196 -> 3257 us, 2000 cells 4270 -> 3708 us; mixed 1000 cells, 80 iterations
+// 4058 -> 3302 us, 2000 cells 4270 -> 3708 us; mixed 1000 cells, 80 iterations
 // 5197 -> 4223 us; CB05 + SOA 500 cells 8331 -> 7179 us; gradient of 500 cells
 // 236 -> 214 ms.  With even, a grid of w such batches has w even ones instead
 // of full ones and a remainder: FP64 4000 cells 8324 -> 7334 us, 6000 12317 ->

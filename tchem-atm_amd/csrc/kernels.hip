@@ -1796,9 +1796,9 @@ __global__ __launch_bounds__(64) void aerosol_rhs_kernel(IntegratorArgs a) {
 // Then slots spread over the LDS banks and pivots inverted once per
 // factorisation.  Measured, interpreter -> encoded -> spread: 131040 cells
 // mixed, 80 TR-BDF2 iterations 305.2 -> 160.5 -> 145.3 ms; 16411 cells FP64,
-// 100 iterations 69.8 -> 36.8 -> 36.2 ms; one cell, 10 iterations 594 -> 309
-// -> 304 us; E3SM 40960 cells to 1800 s 63.6 -> 32.3 -> 30.6 ms; CB05 + SOA,
-// one particle, 8192 cells, 60 iterations 52.8 -> 33.7 -> 33.0 ms (same bits).
+// 100 iterations 69.8 -> 36.8 -> 37.4 ms; one cell, 10 iterations 594 -> 309
+// -> 300 us; E3SM 40960 cells to 1800 s 63.6 -> 32.3 -> 30.7 ms; CB05 + SOA,
+// one particle, 8192 cells, 60 iterations 52.8 -> 33.7 -> 33.6 ms (same bits).
 // Reading the stream 4 to 7 rounds ahead instead of 2, or a section's first
 // records a section early, gave -4 to +4 %: the rounds wait for their own
 // operands and instructions, not for the stream.
@@ -2084,7 +2084,7 @@ __device__ void adjoint_cell(const AdjointArgs& a, const SpLds<double, false>& L
 
 // One wavefront per cell, cells taken from a device work queue.  Bound by the
 // same chain as trbdf2_kernel; gradient of 2000 CB05 cells over 1 ms of model
-// time, forward and backward: 583 ms with the rounds interpreted, 249 ms
+// time, forward and backward: 583 ms with the rounds interpreted, 248 ms
 // encoded.
 template <int QM>
 __global__ __launch_bounds__(512) __attribute__((flatten)) void adjoint_kernel(AdjointArgs a) {

@@ -47,13 +47,15 @@ __device__ __forceinline__ unsigned lds_address(const char* p) {
 #endif
 }
 
-// The instruction stream, in device memory or staged in LDS.  With RSRC device
-// memory is read through a buffer resource: the lane's offset is one register
-// for all records of a size, the record's a scalar, and there is no vector
-// address arithmetic.  Measured, plain loads -> buffer loads: FP32 factors
-// (at their 128-register limit) 131040 CB05 cells 154.1 -> 145.5 ms; FP64
-// (registers to spare) 16411 cells 36.4 -> 37.4 ms, so only FP32 uses it.
-template <bool STAGED, bool RSRC>
+// The instruction stream, in device memory or staged in LDS.  Device memory
+// is read through a buffer resource: the lane's offset is one register for
+// all records of a size, the record's a scalar, there is no vector address
+// arithmetic, and no instance of the integrator spills vector registers (with
+// plain loads the FP64 gas, aerosol and adjoint ones did, and the spilled
+// 4-slot aerosol instance failed its Newton iterations).  Measured, plain ->
+// buffer loads: 131040 CB05 cells mixed 154.1 -> 145.5 ms; 363 cells FP64
+// 4177 -> 4058 us; 16411 cells FP64 36.3 -> 37.4 ms.
+template <bool STAGED>
 struct WordStream {
   const unsigned* g;  // device memory
   unsigned l;         // LDS address
@@ -64,8 +66,6 @@ struct WordStream {
     constexpr int w = int(sizeof(V) / 4);
     if constexpr (STAGED) return lds_get<V>(l + 4u * unsigned(o + 64 * w * r) + unsigned(4 * w * lane));
 #ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (!RSRC)
-      return *(const __attribute__((address_space(1))) V*)(g + o + 64 * w * r + w * lane);
     const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned*>(g), 0, bytes, 0x00027000);
     // readfirstlane keeps the uniform offset scalar whatever the loop optimiser does
     const int v = 4 * w * lane, s = __builtin_amdgcn_readfirstlane(4 * (o + 64 * w * r));
@@ -135,9 +135,8 @@ __device__ __forceinline__ void rotate(int n, Load load, Exec exec) {
 template <typename TA_, bool STAGED_>
 struct SpLds {
   using TA = TA_;
-  static constexpr bool RSRC = sizeof(TA) == 4;
-  WordStream<STAGED_, RSRC> w;
-  __device__ __forceinline__ WordStream<false, RSRC> memory() const { return WordStream<false, RSRC>{w.g, 0u, w.bytes}; }
+  WordStream<STAGED_> w;
+  __device__ __forceinline__ WordStream<false> memory() const { return WordStream<false>{w.g, 0u, w.bytes}; }
   unsigned cell;      // cell region
   unsigned coef;      // coefficient table
   unsigned tol;       // (atol, rtol) per unknown
