@@ -64,7 +64,8 @@ typedef struct {
 #define TCHEM_LU_MFMA 3   /* dense FP32 LU on the matrix cores, pivots fixed by the fill-reducing order: one cell
                              per workgroup of 4 wavefronts; mixed precision, m <= 255 */
 #define TCHEM_PROGRAMS_AUTO 0   /* LDS when they leave room for 4 cells, device memory otherwise */
-#define TCHEM_PROGRAMS_LDS 1    /* staged into LDS once per workgroup, shared by its cells */
+#define TCHEM_PROGRAMS_LDS 1    /* staged into LDS once per workgroup, shared by its cells (all but the Jacobian assembly
+                                   and the factor-reuse solve, which are read from memory) */
 #define TCHEM_PROGRAMS_MEMORY 2 /* read from device memory (L2-resident); the LDS holds the cells and the
                                    coefficient table */
 typedef struct {
