@@ -49,12 +49,13 @@ __device__ __forceinline__ unsigned lds_address(const char* p) {
 
 // The instruction stream, in device memory or staged in LDS.  Device memory
 // is read through a buffer resource: the lane's offset is one register for
-// all records of a size, the record's a scalar, there is no vector address
-// arithmetic, and no instance of the integrator spills vector registers (with
-// plain loads the FP64 gas, aerosol and adjoint ones did, and the spilled
-// 4-slot aerosol instance failed its Newton iterations).  Measured, plain ->
-// buffer loads: 131040 CB05 cells mixed 154.1 -> 145.5 ms; 363 cells FP64
-// 4177 -> 4058 us; 16411 cells FP64 36.3 -> 37.4 ms.
+// all records of a size, the record's a scalar, and there is no vector address
+// arithmetic.  With plain loads several FP64, aerosol and adjoint instances
+// spilled vector registers, and in the 4-slot aerosol one the compiler stored
+// a spill (the largest step length) under the wrong lane mask, so its cells
+// lost their step control; check_exec_mask.py refuses a build with such a
+// store.  Measured, plain -> buffer loads: 131040 CB05 cells mixed 154.1 ->
+// 145.5 ms; 363 cells FP64 4177 -> 4058 us; 16411 cells FP64 36.3 -> 37.4 ms.
 template <bool STAGED>
 struct WordStream {
   const unsigned* g;  // device memory
