@@ -153,12 +153,15 @@ struct IntegratorArgs {
 // constants [nSimpol][4], particle sums [nPart][4] and transfer terms
 // [nPart * nSimpol][6].
 // LDS bytes of one cell of the sparse aerosol integrator: the cell region of
-// the encoded programs plus the unknown copy, source term and SIMPOL scratch
-// of aerosolLdsBytes.
+// the encoded programs, whose part that is dead once the Jacobian is
+// assembled takes the unknown copy, source term and SIMPOL scratch of
+// aerosolLdsBytes, as far as it reaches; then the SIMPOL constants.
+__host__ __device__ inline size_t aerosolScratchEnd(const DevLowered& W, const DevAerosol& X) {
+  const size_t end = size_t(W.oFree) + 8 * (2 * size_t(X.mt) + 4 * size_t(X.nPart) + 6 * size_t(X.nPart) * size_t(X.nSimpol));
+  return end > size_t(W.cellBytes) ? end : size_t(W.cellBytes);
+}
 inline size_t aerosolSparseCellBytes(const DevLowered& W, const DevAerosol& X) {
-  auto al = [](size_t x) { return (x + 15) & ~size_t(15); };
-  return size_t(W.cellBytes) + al(8 * (2 * size_t(X.mt) + 4 * size_t(X.nSimpol) + 4 * size_t(X.nPart) +
-                                       6 * size_t(X.nPart) * size_t(X.nSimpol)));
+  return (aerosolScratchEnd(W, X) + 32 * size_t(X.nSimpol) + 15) & ~size_t(15);
 }
 
 inline size_t aerosolLdsBytes(const DevMech& M, const DevAerosol& X, bool withMatrix = true) {

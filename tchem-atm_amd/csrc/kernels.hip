@@ -1587,7 +1587,7 @@ struct AerosolBackend : AerosolLayout {
 // order.
 struct AeroSpLds : SpLds<double, false> {
   double* A;    // factor slots
-  double* x;    // [mt] unknowns
+  double* x;    // [mt] unknowns, with f, ps and pd in the place of what is dead once the Jacobian is assembled
   double* f;    // [mt] source term
   double* sc;   // [nSimpol][4]
   double* ps;   // [nPart][4]
@@ -1603,11 +1603,11 @@ __device__ AeroSpLds carve_aero_sparse(char* base, const IntegratorArgs& a, int 
       a.W, reinterpret_cast<const unsigned*>(X.pib) + a.W.oWords, X.mt, base, a.cellBytes, wave);
   char* cell = base + sparseStageBytes(a.W, X.mt, false) + size_t(wave) * size_t(a.cellBytes);
   L.A = reinterpret_cast<double*>(cell);
-  L.x = reinterpret_cast<double*>(cell + a.W.cellBytes);
+  L.x = reinterpret_cast<double*>(cell + a.W.oFree);
   L.f = L.x + X.mt;
-  L.sc = L.f + X.mt;
-  L.ps = L.sc + 4 * X.nSimpol;
+  L.ps = L.f + X.mt;
   L.pd = L.ps + 4 * X.nPart;
+  L.sc = reinterpret_cast<double*>(cell + aerosolScratchEnd(a.W, X));
   L.nc = nullptr;
   L.T = L.p = 0.0;
   return L;
@@ -1650,7 +1650,6 @@ struct AerosolSparseBackend : AerosolLayout {
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
       fg[q] = i < M.m ? M.emission()[i] : 0.0;
-      if (i < mt) L.x[i] = u[q];
       if (i < M.m) L.c[i] = u[q];
     }
     wave_sync();
@@ -1667,9 +1666,11 @@ struct AerosolSparseBackend : AerosolLayout {
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int i = lane + kWave * q;
+      if (i < mt) L.x[i] = u[q];
       if (i < mt) L.f[i] = i < M.m ? fg[q] : 0.0;
     }
-    simpol_terms(a, L, lane);  // syncs first
+    wave_sync();
+    simpol_terms(a, L, lane);
     // Transfer terms and derivatives.  Targets in a particle's own rows or
     // columns are written by that particle's lane, the shared gas-species
     // targets (f_g and the (g, g) entries) by lane 0 afterwards; each target

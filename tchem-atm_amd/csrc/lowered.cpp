@@ -192,8 +192,14 @@ std::vector<int> factorSlots(const SparseSchedule& s) {
   spreadOverBanks(slot, gs, std::min<long>(140L * s.nnzF, 120000L));
   return slot;
 }
-std::vector<int> pairSlots(const SparseSchedule& s, const Chunks& chunks) {
-  std::vector<int> pairSlot(size_t(kLanes) * size_t(s.pairRounds));
+// Live items keep to the first slots, so that the last slots of a section's
+// rounds belong to idle lanes and need no room of their own (layout).
+std::vector<int> withIdleLanes(std::vector<int> slot, int rounds) {
+  for (int i = int(slot.size()); i < kLanes * rounds; ++i) slot.push_back(i);
+  return slot;
+}
+std::vector<int> pairSlots(const SparseSchedule& s, const Chunks& chunks, int nPairs) {
+  std::vector<int> pairSlot(static_cast<size_t>(nPairs));
   std::iota(pairSlot.begin(), pairSlot.end(), 0);
   std::vector<Gather> gs;
   auto gather = [&](const std::vector<Chunk>& v, size_t per, size_t k, size_t e) {
@@ -211,12 +217,12 @@ std::vector<int> pairSlots(const SparseSchedule& s, const Chunks& chunks) {
     for (size_t e = 0; e < 2; ++e) gather(chunks.j2, 2, k, e);
   for (size_t k = 0; k < 4; ++k) gather(chunks.j1, 4, k, 0);
   spreadOverBanks(pairSlot, gs, std::min<long>(120L * long(pairSlot.size()), 60000L));
-  return pairSlot;
+  return withIdleLanes(std::move(pairSlot), s.pairRounds);
 }
 // rates of progress and rate constants share their slots
 std::vector<int> reactionSlots(const MechTables& t, const SparseSchedule& s, const std::vector<int>& pairSlot) {
   const std::vector<int> segOrder = segmentOrder(t);
-  std::vector<int> ropSlot(size_t(kLanes) * size_t(s.ropRounds));
+  std::vector<int> ropSlot(static_cast<size_t>(t.nReac));
   std::iota(ropSlot.begin(), ropSlot.end(), 0);
   std::vector<Gather> gs;
   for (size_t g = 0; g < segOrder.size(); g += kLanes) {
@@ -236,7 +242,7 @@ std::vector<int> reactionSlots(const MechTables& t, const SparseSchedule& s, con
   for (size_t i = 0; i < reacOf.size(); i += kLanes)
     addGathers(gs, std::vector<int>(reacOf.begin() + long(i), reacOf.begin() + long(i + kLanes)));
   spreadOverBanks(ropSlot, gs, std::min<long>(200L * long(ropSlot.size()), 60000L));
-  return ropSlot;
+  return withIdleLanes(std::move(ropSlot), s.ropRounds);
 }
 
 struct Lowering {
@@ -284,17 +290,18 @@ struct Lowering {
   const std::vector<int>&ropSlot, &pairSlot;  // of LoweredSlots
   std::vector<std::pair<int, int>> powers;  // (species, exponent >= 2) with a slot of their own
   std::vector<std::pair<int, int>> scaled;  // (reaction, factor >= 2) with a kf slot of their own
+  int oPowers = 0, oScaled = 0;             // byte offsets of those slots
   int powerSlot(int sp, int n) {
     if (n <= 0) return d.oneC;
     if (n == 1) return d.oC + 8 * sp;
     const auto it = std::find(powers.begin(), powers.end(), std::make_pair(sp, n));
-    return d.oC + 8 * (t.nSpec + int(it - powers.begin()));
+    return oPowers + 8 * int(it - powers.begin());
   }
   int kfSlot(int r, int n) {
     if (n == 0) return d.zero8;
     if (n == 1) return d.oK + 8 * ropSlot[size_t(r)];
     const auto it = std::find(scaled.begin(), scaled.end(), std::make_pair(r, n));
-    return d.oK + 8 * (kLanes * s.ropRounds + int(it - scaled.begin()));
+    return oScaled + 8 * int(it - scaled.begin());
   }
   int spec(int r, int j) const { return j < t.maxReactants ? t.reacSpec[size_t(r) * t.maxReactants + j] : -1; }
   int power(int r, int j) const { return j < t.maxReactants ? t.reacPow[size_t(r) * t.maxReactants + j] : 0; }
@@ -321,53 +328,68 @@ struct Lowering {
   std::vector<Join> joins;
   int nPartial = 0;
 
+  // Regions share room where one is dead while the other lives: powers and
+  // partial sums lie with the segment sums (and, in the adjoint, all of them
+  // with w and v).  The slots that the last round of a section writes for its
+  // idle lanes fall on the region behind, where that is dead then; the order
+  // of a Newton iteration is powers, rates of progress (P), derivative pairs
+  // (D), segment sums (S), species rows, Jacobian.  Only the last region pays
+  // for its idle lanes, and of the orders S P D, D S P and P D S the smallest
+  // is taken, so that as many cells fit a workgroup as there are items for.
   void layout() {
     const int m = s.m;
+    const int idleK = 8 * (kLanes * s.ropRounds - t.nReac), idleP = idleK;
+    const int idleD = T * (kLanes * s.pairRounds - t.nPairs()), idleS = 8 * (kLanes * ceilDiv(t.nSeg(), kLanes) - t.nSeg());
+    const int sizeP = 8 * t.nReac, sizeD = T * t.nPairs(), sizePS = T * nPartial, sizePow = 8 * int(powers.size());
+    auto al8 = [](int x) { return (x + 7) & ~7; };
     int o = 0;
     d.zeroA = T * s.nnzF;
     d.trashA = T * (s.nnzF + 1);
     o = al16(T * (s.nnzF + 2));
     d.oR = o;
     o = al16(o + 2 * T * (m + 2));
-    d.oD = o;
-    o = al16(o + T * kLanes * s.pairRounds);
     d.oC = o;
-    d.oneC = o + 8 * (t.nSpec + int(powers.size()));
+    d.oneC = o + 8 * t.nSpec;
     d.trashC = d.oneC + 8;
     o = d.trashC + 8;
-    d.oK = o;
-    d.nK = kLanes * s.ropRounds + int(scaled.size()) + 1;
-    d.zero8 = o + 8 * (d.nK - 1);
-    o = al16(o + 8 * d.nK);
-    d.oP = o;
-    o += 8 * kLanes * s.ropRounds;
-    d.oS = o;
-    o = al16(o + 8 * kLanes * std::max(1, ceilDiv(t.nSeg(), kLanes)));
     if (adjoint) {
       d.oMu = o;
       o += 8 * (m + 1);
-      d.oW = o;
-      o += 8 * kLanes * std::max(1, ceilDiv(t.nReac, kLanes));
-      d.oV = o;
-      o = al16(o + 8 * kLanes * std::max(1, ceilDiv(m, kLanes)));
-      // w and v are dead while a Jacobian is assembled (rates of progress are not)
-      if (T * nPartial <= o - d.oW) {
-        d.oPS = d.oW;
-      } else {
-        d.oPS = o;
-        o = al16(o + T * nPartial);
-      }
-    } else {
-      // rates of progress and segment sums are read for the last time before
-      // the Jacobian is assembled
-      if (T * nPartial <= o - d.oP) {
-        d.oPS = d.oP;
-      } else {
-        d.oPS = o;
-        o = al16(o + T * nPartial);
-      }
     }
-    d.cellBytes = o;
+    oScaled = o;
+    d.zero8 = oScaled + 8 * int(scaled.size());
+    d.oK = d.zero8 + 8;
+    d.nK = t.nReac + int(scaled.size()) + 1;
+    o = d.oFree = d.oK + 8 * t.nReac;  // idle lanes of K: on anything behind, loaded before all of it
+    int end = 0;
+    if (adjoint) {
+      // w v P D: w outlives powers and pairs (gradient), P outlives the
+      // Jacobian.  Idle lanes of w fall on v, which has room for its own.
+      d.oS = d.oPS = d.oW = o;
+      d.oV = oPowers = o + 8 * t.nReac;
+      d.oP = std::max({o + 8 * t.nSeg(), o + 8 * t.nSeg() + idleS - sizeP, o + sizePS, oPowers + sizePow,
+                       o + 8 * kLanes * ceilDiv(t.nReac, kLanes), d.oV + 8 * kLanes * std::max(1, ceilDiv(m, kLanes))});
+      d.oD = d.oP + sizeP;
+      end = std::max(d.oD + sizeD + idleD, d.oD + idleP);
+    } else {
+      // S with powers and partial sums, extra: bytes of the neighbour that
+      // partial sums and idle lanes may use too
+      auto sizeS = [&](int extra, int atLeast) {
+        return al8(std::max({8 * t.nSeg(), sizePow, sizePS - extra, 8 * t.nSeg() + idleS - extra, atLeast}));
+      };
+      const int spdS = sizeS(sizeP, 0), spd = spdS + sizeP + std::max(sizeD + idleD, idleP);
+      const int dspS = sizeS(sizeP, idleD), dsp = al8(sizeD) + dspS + sizeP + idleP;
+      const int pdsD = std::max(al8(sizeD), idleP), pdsS = sizeS(0, std::max(idleD, 8 * t.nSeg() + idleS)), pds = sizeP + pdsD + pdsS;
+      if (spd <= dsp && spd <= pds) {
+        d.oS = o, d.oP = o + spdS, d.oD = d.oP + sizeP, end = o + spd;
+      } else if (dsp <= pds) {
+        d.oD = o, d.oS = o + al8(sizeD), d.oP = d.oS + dspS, end = o + dsp;
+      } else {
+        d.oP = o, d.oD = o + sizeP, d.oS = d.oD + pdsD, end = o + pds;
+      }
+      d.oPS = oPowers = d.oS;
+    }
+    d.cellBytes = al16(std::max({end, d.oS + 8 * t.nSeg() + idleS, o + idleK}));
     d.shift = (m > 128 || d.cellBytes > (1 << 16)) ? (T == 8 ? 3 : 2) : 0;
   }
 
@@ -736,7 +758,7 @@ LoweredSlots chooseSlots(const MechTables& t, const SparseSchedule& s, const Low
     o.pair = shared->pair;
     o.rop = shared->rop;
   } else {
-    o.pair = pairSlots(s, jacobianChunks(t, s));
+    o.pair = pairSlots(s, jacobianChunks(t, s), t.nPairs());
     o.rop = reactionSlots(t, s, o.pair);
   }
   return o;

@@ -76,10 +76,12 @@ struct DevLowered {
   int cellBytes;
   int zeroA, trashA;      // slots of the factor array (which starts at 0)
   int oR;                 // (rhs, reciprocal pivot) pairs, rows m (zeros) and m + 1 (trash) after the m unknowns
-  int oD, oPS;            // derivative pairs; partial sums, in the place of what is dead while J is assembled
+  int oD, oPS;            // derivative pairs; partial sums (with the segment sums, which are dead then)
   int oC, oneC, trashC;   // concentrations, the slot that holds 1
-  int oK, nK, zero8;      // kf: 64 nRop slots, n * kf slots, the slot that holds 0 (the last)
+  int oK, nK, zero8;      // rate constants, with n * kf slots and the slot that holds 0 before them (nK in all)
   int oP, oS;             // rates of progress, segment sums
+  int oFree;              // the regions from here to the end (pairs, partial, segment sums, rates of progress) are
+                          // dead once the Jacobian is assembled (not in the adjoint)
   // sections
   int oPow, nPow, oKf, oKfx, nKfx, oRop, nRop, oPair, nPair;
   int oSegHdr, oSeg, nSeg;
@@ -88,7 +90,7 @@ struct DevLowered {
   int oLuHdr, oLu, oLu1, nLu, oDiag, oBack, nBack, oFwdHdr, oFwd, oFwd1, nFwd;
   // adjoint programs only
   int oNutHdr, oNut, nNut, oJtvHdr, oJtv, nJtv;
-  int oMu, oW, oV;  // mu [m + 1] (mu[m] = 0), w sums, v sums (byte offsets in the cell region)
+  int oMu, oW, oV;  // mu [m + 1] (mu[m] = 0), w sums, v sums (byte offsets in the cell region, the sums in oS's place)
   int oWmap, oVmap;        // byte offset of w_r by slot of reaction r, [64 ceil(m / 64)] of v_i
 };
 
