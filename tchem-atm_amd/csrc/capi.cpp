@@ -66,6 +66,8 @@ hipError_t launchJacobian(const DevMech& M, int nBatch, const double* state, con
 using namespace tchem_amd;
 
 namespace {
+constexpr int kMaxAerosolCells = 8;  // wavefronts per workgroup of the sparse aerosol instances (512 threads)
+
 // roctx ranges around the batch calls: the reference's Kokkos::Profiling
 // regions (src/core/TChem_AtmosphericChemistry.cpp:61,166,193,207), seen by
 // rocprofv3 --marker-trace.  The ROCm roctx library is not linked: loading a
@@ -210,12 +212,6 @@ int upload(tchem_kmcd_s* k, const std::vector<T>& v, const T** out) {
   return TCHEM_OK;
 }
 
-// Tolerances are staged where one cell still fits beside them.
-void stageTolerances(DevLowered& w, int m, size_t cellBytes, size_t maxLds) {
-  w.tolStaged = 1;
-  if (sparseStageBytes(w, m, false) + cellBytes > maxLds) w.tolStaged = 0;
-}
-
 // Options after validation, with the LU form resolved.
 int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, tchem_atmchem_options_t* o,
                    const char* who) {
@@ -263,10 +259,8 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   // latency bound: resident cells set its throughput); memory otherwise
   if (o->programs == TCHEM_PROGRAMS_AUTO) {
     const int cap = sparseMaxCellsPerGroup(o->precision, k->dev.m);
-    const size_t prog = sparseStageBytes(W, k->dev.m, true);
-    const size_t coefB = sparseStageBytes(W, k->dev.m, false);
-    const size_t inMem = coefB < maxLds ? std::min<size_t>(cap, cellB ? (maxLds - coefB) / cellB : 0) : 0;
-    const size_t inLds = prog < maxLds ? std::min<size_t>(cap, cellB ? (maxLds - prog) / cellB : 0) : 0;
+    const int inMem = sparseCellsThatFit(W, k->dev.m, false, cellB, maxLds, cap);
+    const int inLds = sparseCellsThatFit(W, k->dev.m, true, cellB, maxLds, cap);
     o->programs = (inLds >= 1 && inLds >= inMem) ? TCHEM_PROGRAMS_LDS : TCHEM_PROGRAMS_MEMORY;
   }
   const bool staged = o->programs == TCHEM_PROGRAMS_LDS;
@@ -743,7 +737,9 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
   // exceeds the LDS, run the dense form only)
   auto pack = [&](const SparseSchedule& sc, const LoweredSlots& slots, int bytesT, bool adjoint, DevLowered* w) {
     LoweredProgram p = lowerProgram(t, sc, bytesT, adjoint, slots);
-    stageTolerances(p.d, t.m, size_t(p.d.cellBytes), k->maxLds);
+    if (!adjoint)
+      stageTolerances(p.d, t.m, size_t(p.d.cellBytes), k->maxLds,
+                      sparseMaxCellsPerGroup(bytesT == 8 ? TCHEM_PRECISION_FP64 : TCHEM_PRECISION_MIXED, t.m));
     if (sparseStageBytes(p.d, t.m, false) + size_t(p.d.cellBytes) > k->maxLds) return;
     *w = p.d;
     w->oWords = addI(std::vector<int>(p.words.begin(), p.words.end()));
@@ -1728,7 +1724,7 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
     };
     X.oJpos = int(ib.size());
     for (const auto& e : ent) ib.push_back(position(e[0], e[1]));
-    stageTolerances(p.d, mt, aerosolSparseCellBytes(p.d, X), kmcd->maxLds);
+    stageTolerances(p.d, mt, aerosolSparseCellBytes(p.d, X), kmcd->maxLds, kMaxAerosolCells);
     h->W = p.d;
     pib.assign(p.words.begin(), p.words.end());
     pdb = std::move(p.coef);
@@ -1852,8 +1848,7 @@ int tchem_aerosolchem_run_device_batch(const tchem_atmchem_options_t* opts, int 
     a.W = amcd->W;
     a.cellBytes = int(aerosolSparseCellBytes(a.W, a.X));
     stageB = sparseStageBytes(a.W, a.X.mt, false);
-    cells = int((k->maxLds - stageB) / size_t(a.cellBytes));
-    if (cells > 8) cells = 8;
+    cells = sparseCellsThatFit(a.W, a.X.mt, false, size_t(a.cellBytes), k->maxLds, kMaxAerosolCells);
   }
   if (cells < 1) return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": one cell does not fit the LDS");
   const int perGroup = cellsForBatch(nBatch, cells, k->numCUs, false);

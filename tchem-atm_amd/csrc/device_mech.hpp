@@ -87,7 +87,24 @@ struct DevMech {
 // of m unknowns.
 __host__ __device__ inline size_t sparseStageBytes(const DevLowered& W, int m, bool staged) {
   return (staged ? 4 * size_t(W.stagedWords) : 0) + ((8 * size_t(W.nCoef) + 15) & ~size_t(15)) +
-         (W.tolStaged ? 16 * size_t(m) : 0);
+         (W.tolStaged[staged] ? 16 * size_t(m) : 0);
+}
+// Cells (at most `most`) of cellBytes that fit beside them.
+inline int sparseCellsThatFit(const DevLowered& W, int m, bool staged, size_t cellBytes, size_t maxLds, int most) {
+  const size_t stage = sparseStageBytes(W, m, staged);
+  const size_t n = stage < maxLds && cellBytes > 0 ? (maxLds - stage) / cellBytes : 0;
+  return n < size_t(most) ? int(n) : most;
+}
+// Tolerances are staged where they cost no cell: they are read once per step,
+// resident cells set the throughput (16 mixed cells of the CB05 + SOA gas
+// phase fit without them, 15 with).
+inline void stageTolerances(DevLowered& W, int m, size_t cellBytes, size_t maxLds, int most) {
+  for (const bool staged : {false, true}) {
+    W.tolStaged[staged] = 0;
+    const int without = sparseCellsThatFit(W, m, staged, cellBytes, maxLds, most);
+    W.tolStaged[staged] = 1;
+    W.tolStaged[staged] = without > 0 && sparseCellsThatFit(W, m, staged, cellBytes, maxLds, most) == without;
+  }
 }
 
 // Forward record of the discrete adjoint: accepted step sizes and the state

@@ -547,10 +547,10 @@ struct DenseBackend {
 
 // time tolerances of unknown ai from the staged table at LDS address tol, or
 // (index: its row) from the caller's
-template <class Index>
+template <bool STAGED, class Index>
 __device__ __forceinline__ void staged_tolerance(const IntegratorArgs& a, unsigned tol, int ai, Index index,
                                                  double& atol, double& rtol) {
-  if (a.W.tolStaged) {
+  if (a.W.tolStaged[STAGED]) {
     const vec2<double> t = lds_get<vec2<double>>(tol + 16 * ai);
     atol = t.x;
     rtol = t.y;
@@ -576,7 +576,7 @@ struct SparseBackend {
   static __device__ __forceinline__ int column(const IntegratorArgs& a, int ai) { return 3 + a.M.perm()[ai]; }
   static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds& L, int ai, double& atol,
                                                    double& rtol) {
-    staged_tolerance(a, L.tol, ai, [&](int i) { return a.M.perm()[i]; }, atol, rtol);
+    staged_tolerance<STAGED>(a, L.tol, ai, [&](int i) { return a.M.perm()[i]; }, atol, rtol);
   }
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
@@ -584,7 +584,7 @@ struct SparseBackend {
   static __device__ void stage(const IntegratorArgs& a, char* base) {
     stage_sparse<STAGED>(a.W, reinterpret_cast<const unsigned*>(a.M.ib) + a.W.oWords, a.M.db + a.W.oCoef, base);
     double* tol = reinterpret_cast<double*>(base + sparseStageBytes(a.W, 0, STAGED));
-    const int n = a.W.tolStaged ? 2 * a.M.m : 0;
+    const int n = a.W.tolStaged[STAGED] ? 2 * a.M.m : 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) tol[i] = a.tol_time[2 * a.M.perm()[i >> 1] + (i & 1)];
     __syncthreads();
   }
@@ -1622,12 +1622,12 @@ struct AerosolSparseBackend : AerosolLayout {
   struct Fact {};
   static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds& L, int ai, double& atol,
                                                    double& rtol) {
-    staged_tolerance(a, L.tol, ai, [&](int i) { return i < a.M.m ? a.M.perm()[i] : i; }, atol, rtol);
+    staged_tolerance<false>(a, L.tol, ai, [&](int i) { return i < a.M.m ? a.M.perm()[i] : i; }, atol, rtol);
   }
   static __device__ void stage(const IntegratorArgs& a, char* base) {
     stage_sparse<false>(a.W, nullptr, a.X.pdb + a.W.oCoef, base);
     double* tol = reinterpret_cast<double*>(base + sparseStageBytes(a.W, 0, false));
-    const int n = a.W.tolStaged ? 2 * a.X.mt : 0;
+    const int n = a.W.tolStaged[0] ? 2 * a.X.mt : 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
       const int ai = i >> 1, xs = ai < a.M.m ? a.M.perm()[ai] : ai;
       tol[i] = a.tol_time[2 * xs + (i & 1)];

@@ -71,7 +71,8 @@ struct DevLowered {
                     // or rarely run; the LDS they would take holds cells)
   int oWords;     // stream start in the mechanism's int buffer
   int nCoef, oCoef;  // coefficient table (staged into LDS), start in the double buffer
-  int tolStaged;     // whether the unknowns' tolerances are staged into LDS too (set by the caller: they fit)
+  int tolStaged[2];  // whether the unknowns' tolerances are staged into LDS too, with the programs in memory and with
+                     // the programs staged (stageTolerances)
   // cell layout
   int cellBytes;
   int zeroA, trashA;      // slots of the factor array (which starts at 0)

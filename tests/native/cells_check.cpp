@@ -1,6 +1,6 @@
 // Prints how many cells of the sparse forms fit a workgroup's LDS: the cell
 // regions of the encoded programs (lowered.cpp) beside the coefficient table
-// and, where they are staged, the programs.
+// and, where they are staged, the programs and tolerances.
 //
 // usage: cells_check <mechanism.yaml> [<aerosol.yaml> <particles>...]
 #include <array>
@@ -16,10 +16,6 @@
 using namespace tchem_amd;
 
 static const size_t kLds = 160 * 1024;
-static int cells(size_t stage, size_t cell, int most) {
-  const size_t n = stage < kLds ? (kLds - stage) / cell : 0;
-  return n < size_t(most) ? int(n) : most;
-}
 
 int main(int argc, char** argv) {
   if (argc < 2) return 2;
@@ -29,10 +25,12 @@ int main(int argc, char** argv) {
     const SparseSchedule s = buildSparseSchedule(t);
     const LoweredSlots fs = chooseSlots(t, s);
     for (int bytes : {8, 4}) {
-      const DevLowered w = lowerProgram(t, s, bytes, false, fs).d;
+      DevLowered w = lowerProgram(t, s, bytes, false, fs).d;
+      const size_t cell = size_t(w.cellBytes);
       const int most = t.m > 128 ? 8 : (bytes == 8 ? 12 : 16);
-      std::printf("fp%d memory %d staged %d\n", 8 * bytes, cells(sparseStageBytes(w, t.m, false), size_t(w.cellBytes), most),
-                  cells(sparseStageBytes(w, t.m, true), size_t(w.cellBytes), most));
+      stageTolerances(w, t.m, cell, kLds, most);
+      std::printf("fp%d memory %d staged %d\n", 8 * bytes, sparseCellsThatFit(w, t.m, false, cell, kLds, most),
+                  sparseCellsThatFit(w, t.m, true, cell, kLds, most));
     }
   }
   for (int i = 3; i < argc; ++i) {
@@ -40,12 +38,14 @@ int main(int argc, char** argv) {
     am.nParticles = std::atoi(argv[i]);
     const MechTables ta = aerosolTables(t, am, nullptr);
     const SparseSchedule s = buildSparseSchedule(ta, false);
-    const DevLowered w = lowerProgram(ta, s, 8, false, chooseSlots(ta, s)).d;
+    DevLowered w = lowerProgram(ta, s, 8, false, chooseSlots(ta, s)).d;
     DevAerosol X{};
     X.mt = ta.m;
     X.nPart = am.nParticles;
     X.nSimpol = int(am.simpol.size());
-    std::printf("particles %d: %d\n", am.nParticles, cells(sparseStageBytes(w, ta.m, false), aerosolSparseCellBytes(w, X), 8));
+    stageTolerances(w, ta.m, aerosolSparseCellBytes(w, X), kLds, 8);
+    std::printf("particles %d: %d\n", am.nParticles,
+                sparseCellsThatFit(w, ta.m, false, aerosolSparseCellBytes(w, X), kLds, 8));
   }
   return 0;
 }

@@ -1,7 +1,7 @@
 """Cells of the sparse forms that fit a workgroup (tests/native/cells_check.cpp):
 at least as many as the items of a cell (factor entries, right-hand side and
 pivots, derivative pairs, concentrations, rate constants, rates of progress,
-segment sums) leave room for, so that no number of cells per workgroup that
+segment sums) leave room for, with or without staged tolerances, so that no number of cells per workgroup that
 such a cell allows is refused or given up.  And the regions that share room
 for it, over several iterations on one cell (lowered_repeat_check.cpp)."""
 import importlib
@@ -49,6 +49,7 @@ def repeat(tmp_path_factory):
     ("uci_v2_test3.yaml", (12, 12), (16, 16)),
     ("troe.yaml", (12, 12), (16, 16)),
     ("cascade129", (7, 3), (8, 5)),
+    ("cascade180", (3, 0), (6, 0)),
     ("uniform60", (6, 0), (10, 0)),
 ])
 def test_gas_cells_per_workgroup(cells, pkg, tmp_path, mech, fp64, fp32):
@@ -56,6 +57,8 @@ def test_gas_cells_per_workgroup(cells, pkg, tmp_path, mech, fp64, fp32):
     f = golden(mech) if mech.endswith(".yaml") else str(tmp_path / "m.yaml")
     if mech == "cascade129":
         S.synthetic_mechanism_yaml(f, seed=5, n_species=129, n_reactions=200, n_radicals=8, window=20, coupling="cascade")
+    elif mech == "cascade180":
+        S.synthetic_mechanism_yaml(f, seed=5, n_species=180, n_reactions=400, n_radicals=8, window=20, coupling="cascade")
     elif mech == "uniform60":
         S.synthetic_mechanism_yaml(f, n_species=60, n_reactions=180)
     (_, *d), (_, *s) = cells(f)
