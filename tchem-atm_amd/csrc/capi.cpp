@@ -30,7 +30,7 @@ namespace tchem_amd {
 hipError_t launchIntegrator(const IntegratorArgs& a, int precision, int grid, size_t lds, hipStream_t stream);
 hipError_t integratorMaxBlocksPerCU(int precision, int sparse, int m, const DevLowered& w, int threads, size_t lds,
                                     int* blocks, bool rec);
-int sparseMaxCellsPerGroup(int precision, int m);
+int sparseMaxCellsPerGroup(int precision, const DevLowered& w);
 size_t integratorStaticLds(int precision, int sparse, int m, const DevLowered& w);
 hipError_t launchResetCounter(int* counter, hipStream_t stream);
 hipError_t launchAutotuneSample(int n, long long stride, int nb, int np, int iters, const double* state,
@@ -258,7 +258,7 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   // cells per workgroup as reading them from memory would (the kernel is
   // latency bound: resident cells set its throughput); memory otherwise
   if (o->programs == TCHEM_PROGRAMS_AUTO) {
-    const int cap = sparseMaxCellsPerGroup(o->precision, k->dev.m);
+    const int cap = sparseMaxCellsPerGroup(o->precision, W);
     const int inMem = sparseCellsThatFit(W, k->dev.m, false, cellB, maxLds, cap);
     const int inLds = sparseCellsThatFit(W, k->dev.m, true, cellB, maxLds, cap);
     o->programs = (inLds >= 1 && inLds >= inMem) ? TCHEM_PROGRAMS_LDS : TCHEM_PROGRAMS_MEMORY;
@@ -272,7 +272,7 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   if (o->lu == TCHEM_LU_SPARSE) {
     if (!W.enabled)
       return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": mechanism has no sparse schedule");
-    const int cap = sparseMaxCellsPerGroup(o->precision, k->dev.m);
+    const int cap = sparseMaxCellsPerGroup(o->precision, W);
     if (o->cells_per_block == 0) {
       int c = cap;
       while (c > 1 && !sparseFits(c)) --c;
@@ -739,7 +739,7 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
     LoweredProgram p = lowerProgram(t, sc, bytesT, adjoint, slots);
     if (!adjoint)
       stageTolerances(p.d, t.m, size_t(p.d.cellBytes), k->maxLds,
-                      sparseMaxCellsPerGroup(bytesT == 8 ? TCHEM_PRECISION_FP64 : TCHEM_PRECISION_MIXED, t.m));
+                      sparseMaxCellsPerGroup(bytesT == 8 ? TCHEM_PRECISION_FP64 : TCHEM_PRECISION_MIXED, p.d));
     if (sparseStageBytes(p.d, t.m, false) + size_t(p.d.cellBytes) > k->maxLds) return;
     *w = p.d;
     w->oWords = addI(std::vector<int>(p.words.begin(), p.words.end()));

@@ -2219,15 +2219,16 @@ static const void* integratorFn() {
   return reinterpret_cast<const void*>(&trbdf2_kernel<B, QM, kThreads, REC>);
 }
 
-// Largest workgroup of the sparse form (m <= 128): 16 wavefronts (cells) for
-// the mixed form, 12 for FP64; 8 for larger mechanisms.  The occupancy of this
+// Largest workgroup of the sparse form: 16 wavefronts (cells) for the mixed
+// form, 12 for FP64; 8 for programs with shifted fields, all those of more
+// than 128 unknowns among them.  The occupancy of this
 // latency-bound kernel sets its throughput, so each workgroup size gets the
 // instance with the largest register budget that still lets its wavefronts
 // be resident: FP64 up to 8 cells 512 threads (256 VGPRs), 9-12 cells 768
 // (168); mixed up to 12 cells 768, 13-16 cells 1024 (128 VGPRs, 4 per SIMD,
 // a few registers spilled).
-int sparseMaxCellsPerGroup(int precision, int m) {
-  if (m > 128) return 8;
+int sparseMaxCellsPerGroup(int precision, const DevLowered& w) {
+  if (w.shift) return 8;
   return precision == TCHEM_PRECISION_MIXED ? 16 : 12;
 }
 

@@ -7,6 +7,7 @@
 #include <map>
 #include <numeric>
 #include <random>
+#include <set>
 #include <stdexcept>
 
 namespace tchem_amd {
@@ -390,7 +391,9 @@ struct Lowering {
       d.oPS = oPowers = d.oS;
     }
     d.cellBytes = al16(std::max({end, d.oS + 8 * t.nSeg() + idleS, o + idleK}));
-    d.shift = (m > 128 || d.cellBytes > (1 << 16)) ? (T == 8 ? 3 : 2) : 0;
+    // the fields address the cell region and the coefficient table
+    const std::set<double> coefs(t.omegaCoef.begin(), t.omegaCoef.end());
+    d.shift = (m > 128 || std::max(size_t(d.cellBytes), 8 * (coefs.size() + 1)) > (1 << 16)) ? (T == 8 ? 3 : 2) : 0;
   }
 
   void masks(const std::vector<unsigned char>& bits) {  // bit 0 -> first mask, bit 1 -> second

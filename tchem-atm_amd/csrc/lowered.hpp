@@ -114,8 +114,9 @@ struct LoweredSlots {
 LoweredSlots chooseSlots(const MechTables& t, const SparseSchedule& s, const LoweredSlots* shared = nullptr);
 
 // Lowers the programs of `s` (built from `t`) for matrix entries of
-// bytesT bytes (4 or 8).  shift 0 when the cell region is at most 64 KiB,
-// log2(bytesT) otherwise.  adjoint: room for mu, w and v, and the transposed
+// bytesT bytes (4 or 8).  shift 0 when at most 128 unknowns, and cell region
+// and coefficient table are at most 64 KiB each, log2(bytesT) otherwise.
+// adjoint: room for mu, w and v, and the transposed
 // programs' extra sections; the cell layout depends on sizes only, so the
 // forward and transposed programs of one mechanism share it.  Throws
 // std::runtime_error when a field does not fit.

@@ -6,6 +6,7 @@ such a cell allows is refused or given up.  And the regions that share room
 for it, over several iterations on one cell (lowered_repeat_check.cpp)."""
 import importlib
 import os
+import random
 import re
 import subprocess
 
@@ -94,3 +95,25 @@ def test_iterations_on_one_aerosol_cell(repeat, particles):
                        capture_output=True, text=True)
     print(r.stdout[-1500:])
     assert r.returncode == 0, r.stdout[-2000:]
+
+
+def test_many_distinct_coefficients(repeat, pkg, tmp_path):
+    """8500 yields, all different, in a small cell: more than 16 bits of byte
+    address for the coefficient table."""
+    species = ["S%02d" % i for i in range(64)]
+    rng = random.Random(1)
+    out = ["NCAR-version: v1.0", "environmental_conditions:", "  pressure:", "    initial_value: [101325]", "    units: Pa", "  temperature:",
+           "    initial_value: [298.0]", "    units: K", "initial_state:"]
+    for s in species + ["M"]:
+        out += [f"  {s}:", "    initial_value: [0.1]", "    units: mol m-3"]
+    out += ["constant_species:", "- description: third body", "  name: M", "species:"]
+    out += [ln for s in species for ln in (f"- description: {s}", f"  name: {s}")] + ["reactions:"]
+    for r in range(170):
+        names = rng.sample(species, 51)
+        out += [f"- MUSICA_name: R{r + 1}", "  reactants:", f"    {names[0]}: 1", "  products:"]
+        out += [f"    {s}: {rng.uniform(0.1, 1.0)!r}" for s in names[1:]]
+        out += ["  type: ARRHENIUS", "  coefficients:", "    A: 1.0"]
+    f = tmp_path / "m.yaml"
+    f.write_text("\n".join(out) + "\n")
+    r = subprocess.run([repeat, str(f)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-500:]
