@@ -747,14 +747,14 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
   };
   try {
     if (!k->boxModel) throw std::runtime_error("no box model");
-    const SparseSchedule fwd = buildSparseSchedule(t);
+    const SparseSchedule fwd = buildSparseSchedule(t, false, false);
     k->nnzF = fwd.nnzF;
     const LoweredSlots fs = chooseSlots(t, fwd);
     pack(fwd, fs, 8, false, &k->low64);
     pack(fwd, fs, 4, false, &k->low32);
     // the adjoint shares one cell layout between the forward programs and
     // the transposed ones: the transposed factor pattern has the same size
-    const SparseSchedule trn = buildSparseSchedule(t, true);
+    const SparseSchedule trn = buildSparseSchedule(t, true, false);
     if (k->low64.enabled && trn.nnzF == fwd.nnzF && trn.pairSlots == fwd.pairSlots) {
       pack(fwd, fs, 8, true, &k->lowAdj);
       pack(trn, chooseSlots(t, trn, &fs), 8, true, &k->lowAdjT);
@@ -1715,7 +1715,7 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
   try {
     std::vector<std::array<int, 2>> ent;  // (row, col) of every transfer derivative, table order
     const MechTables ta = aerosolTables(t, am, &ent);
-    const SparseSchedule sc = buildSparseSchedule(ta, false);
+    const SparseSchedule sc = buildSparseSchedule(ta, false, false);
     LoweredProgram p = lowerProgram(ta, sc, 8, false, chooseSlots(ta, sc));
     auto position = [&](int r, int c) {  // the LDS slot of factor entry (r, c)
       for (int q = sc.rowPtr[r]; q < sc.rowPtr[r + 1]; ++q)

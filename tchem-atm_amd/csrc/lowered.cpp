@@ -190,7 +190,8 @@ std::vector<int> factorSlots(const SparseSchedule& s) {
     }
     b += size_t(kLanes) * size_t(words);
   }
-  spreadOverBanks(slot, gs, std::min<long>(140L * s.nnzF, 120000L));
+  // CB05: 370 extra passes in order, 122 after 140 tries per entry, 110 after 300, 102 after 600
+  spreadOverBanks(slot, gs, std::min<long>(300L * s.nnzF, 400000L));
   return slot;
 }
 // Live items keep to the first slots, so that the last slots of a section's

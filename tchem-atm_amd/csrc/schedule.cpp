@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <array>
 #include <map>
+#include <numeric>
 #include <random>
 #include <stdexcept>
 
@@ -309,7 +310,7 @@ void bankAwareSlots(SparseSchedule& s) {
 
 }  // namespace
 
-SparseSchedule buildSparseSchedule(const MechTables& t, bool transposed) {
+SparseSchedule buildSparseSchedule(const MechTables& t, bool transposed, bool spreadSlots) {
   SparseSchedule s;
   s.transposed = transposed;
   const int m = t.m;
@@ -733,7 +734,12 @@ SparseSchedule buildSparseSchedule(const MechTables& t, bool transposed) {
     s.fwdRounds += emitChains(ch, SparseSchedule::kUpd, T, zz, false, s.progHdr, s.progBody);
   }
   s.progBody.insert(s.progBody.end(), slack, 0u);
-  bankAwareSlots(s);
+  if (spreadSlots) {
+    bankAwareSlots(s);
+  } else {
+    s.slotOf.resize(size_t(s.nnzF));
+    std::iota(s.slotOf.begin(), s.slotOf.end(), 0);
+  }
   return s;
 }
 

@@ -106,6 +106,11 @@ struct SparseSchedule {
 // nSpec < 4095, reactant powers < 16, nReac < 16384, at most 65535 distinct
 // stoichiometric coefficients and nnzF + m + 2 < 32768; throws
 // std::runtime_error otherwise.
-SparseSchedule buildSparseSchedule(const MechTables& t, bool transposed = false);
+// spreadSlots: number the factor positions by bankAwareSlots; without it
+// slotOf is the identity, for callers that place the entries themselves
+// (chooseSlots), as the library does: the search is nearly all of the time
+// this takes (a CB05 kmcd, both searches: 514 ms; this one left out, the other
+// with more tries: 285 ms).
+SparseSchedule buildSparseSchedule(const MechTables& t, bool transposed = false, bool spreadSlots = true);
 
 }  // namespace tchem_amd

@@ -22,7 +22,7 @@ int main(int argc, char** argv) {
   const KineticModel km = loadKineticModel(argv[1], nullptr);
   const MechTables t = compileMechanism(km);
   if (argc == 2) {
-    const SparseSchedule s = buildSparseSchedule(t);
+    const SparseSchedule s = buildSparseSchedule(t, false, false);
     const LoweredSlots fs = chooseSlots(t, s);
     for (int bytes : {8, 4}) {
       DevLowered w = lowerProgram(t, s, bytes, false, fs).d;
@@ -37,7 +37,7 @@ int main(int argc, char** argv) {
     AerosolModel am = loadAerosolModel(argv[2], km);
     am.nParticles = std::atoi(argv[i]);
     const MechTables ta = aerosolTables(t, am, nullptr);
-    const SparseSchedule s = buildSparseSchedule(ta, false);
+    const SparseSchedule s = buildSparseSchedule(ta, false, false);
     DevLowered w = lowerProgram(ta, s, 8, false, chooseSlots(ta, s)).d;
     DevAerosol X{};
     X.mt = ta.m;

@@ -2,7 +2,8 @@
 // kernels' order: regions of a cell share room (lowered.cpp: layout), so what
 // an iteration leaves behind must not reach the next one, and what the adjoint
 // keeps between its sections must survive them.  Executor and reference are
-// those of lowered_check.cpp.
+// those of lowered_check.cpp; the schedules are built as the library builds
+// them, their factor positions in order.
 //
 // usage: lowered_repeat_check <mechanism.yaml> [<aerosol.yaml> <particles>...]
 #include <cstdlib>
@@ -132,7 +133,9 @@ int main(int argc, char** argv) {
   if (argc < 2) return 2;
   const KineticModel km = loadKineticModel(argv[1], nullptr);
   const MechTables t = compileMechanism(km);
-  const SS f = buildSparseSchedule(t), b = buildSparseSchedule(t, true);
+  const SS f = buildSparseSchedule(t, false, false), b = buildSparseSchedule(t, true, false);
+  for (const SS* s : {&f, &b})
+    for (int q = 0; q < s->nnzF; ++q) CHECK(s->slotOf[size_t(q)] == q, "position %d", q);
   repeat<float>(t, f, f, false, "forward");
   repeat<double>(t, f, f, false, "forward");
   repeat<double>(t, f, b, true, "adjoint forward");
@@ -141,7 +144,7 @@ int main(int argc, char** argv) {
     AerosolModel am = loadAerosolModel(argv[2], km);
     am.nParticles = std::atoi(argv[i]);
     const MechTables ta = aerosolTables(t, am, nullptr);
-    const SS s = buildSparseSchedule(ta, false);
+    const SS s = buildSparseSchedule(ta, false, false);
     check<double>(ta, s, s, false, "aerosol");
     repeat<double>(ta, s, s, false, "aerosol");
   }
