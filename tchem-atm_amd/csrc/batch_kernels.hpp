@@ -64,7 +64,9 @@ __device__ __forceinline__ void store_items(const double* items, int n, double* 
 // Rate constants of the CB05 kinetics, store(r, k) for each of this thread's.
 // Reactions come in classes (rateOrder): Arrhenius without temperature
 // dependence (photolysis mostly), Arrhenius with an exponential alone, the
-// rest; the first two are straight-line code, two reactions at a time.
+// rest; the first two are straight-line code, two reactions at a time.  The
+// first keep the factor exp(0 / T) as what it is: 1, or NaN where T is NaN or
+// 1 / T is infinite, so that a cell without a temperature has no rates.
 template <int C, class Store>
 __device__ __forceinline__ void group_rate_constants(const DevMech& M, const GroupThread<C>& g, const double* row,
                                                      const double* photo, Store store) {
@@ -72,6 +74,7 @@ __device__ __forceinline__ void group_rate_constants(const DevMech& M, const Gro
   const double p = row[1], T = row[2];
   const double t_1 = 1.0 / T;
   const double conv = M.convPPM * p * t_1;
+  const double unit = 0.0 * t_1 + 1.0;
   const int* order = M.rateOrder();
   const int n0 = order[M.nReac], n1 = order[M.nReac + 1];  // ends of the first two classes
   int i = g.sub;
@@ -80,7 +83,7 @@ __device__ __forceinline__ void group_rate_constants(const DevMech& M, const Gro
     const int r = order[i], slot = M.photoSlot()[r];
     double A = M.ratePar()[8 * r];
     if (photo != nullptr && slot >= 0) A = photo[slot];
-    store(r, A * tchem_ipow(conv, M.convExp()[r]));
+    store(r, A * unit * tchem_ipow(conv, M.convExp()[r]));
   }
 #pragma unroll 2
   for (; i < n1; i += g.n) {
