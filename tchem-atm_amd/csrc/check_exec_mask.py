@@ -18,6 +18,9 @@ Reported are, between the start of a block and the restore of its mask,
   * any vector instruction, in a block that a branch on an empty mask
     (``s_cbranch_execz``) leads to;
   * any access to scratch memory, in every other block.
+
+Kernels that spill vector registers at all are named, without an error: they
+are where such a store can appear.
 """
 import re
 import sys
@@ -53,13 +56,28 @@ def find(lines):
     return out
 
 
+def spills(lines):
+    """{kernel: spilled vector registers} of the kernels that spill any, from the code object's metadata."""
+    out, name = {}, ""
+    for line in lines:
+        m = re.match(r"\s*\.name:\s+'?(_Z\w+)|\s*\.vgpr_spill_count:\s+(\d+)", line)
+        if m and m.group(1):
+            name = m.group(1)
+        elif m and int(m.group(2)):
+            out[name] = int(m.group(2))
+    return out
+
+
 def main(paths):
     bad = 0
     for path in paths:
         with open(path) as f:
-            for function, block, no, text in find(f):
-                bad += 1
-                print(f"{path}:{no}: {function}: {block}: before the lane mask is restored: {text}")
+            lines = f.readlines()
+        for kernel, n in spills(lines).items():
+            print(f"note: {n} vector registers spilled: {kernel}")
+        for function, block, no, text in find(lines):
+            bad += 1
+            print(f"{path}:{no}: {function}: {block}: before the lane mask is restored: {text}")
     if bad:
         print("This compiler stored registers under the wrong lane mask; change the kernel's register pressure.")
     return 1 if bad else 0

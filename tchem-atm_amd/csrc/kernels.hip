@@ -1239,9 +1239,12 @@ __global__ __launch_bounds__(256, 1) void trbdf2_mfma_kernel(IntegratorArgs a) {
 // factorisation without interchanges): the LU of the MFMA form on its own.
 // Every wavefront reads its tiles of [A | b | padding] straight into the
 // registers of the C layout (a register of a tile is two rows of 32
-// consecutive columns), with all loads of a tile row in flight.
+// consecutive columns), with all loads of a tile row in flight.  Two
+// workgroups share a CU at NB = 4 only: at NB = 6 half the registers spill 104
+// of them (2048 systems of order 160 464 us, one system 59; with one workgroup
+// per CU and no spills 447 and 48).
 template <int NB>
-__global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void dense_mfma_solve_kernel(int n, int nBatch, const double* A,
+__global__ __launch_bounds__(256, NB == 4 ? 2 : 1) void dense_mfma_solve_kernel(int n, int nBatch, const double* A,
                                                                                 const double* b, double* x) {
   extern __shared__ __align__(16) char lds_raw[];
   using namespace mfma;

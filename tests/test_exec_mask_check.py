@@ -67,6 +67,12 @@ def test_the_status_tells(tmp_path):
         assert subprocess.run([sys.executable, SCRIPT, str(f)], capture_output=True).returncode == rc
 
 
+def test_spilling_kernels_are_named(check):
+    meta = "    .name:           _Z1aPf\n    .sgpr_spill_count: 9\n    .vgpr_spill_count: %d\n"
+    assert check.spills((meta % 0).splitlines()) == {}
+    assert check.spills((meta % 155 + (meta % 0).replace("1a", "1b")).splitlines()) == {"_Z1aPf": 155}
+
+
 def test_the_library_is_built_through_the_check():
     """make would check the assembly of the compilation whose object it links."""
     r = subprocess.run(["make", "-n", "-B", "-C", CSRC, "_build/kernels.o"], capture_output=True, text=True, check=True)
