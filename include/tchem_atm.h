@@ -63,18 +63,20 @@ typedef struct {
 #define TCHEM_LU_SPARSE 2 /* level-scheduled sparse LU, pivots fixed by the fill-reducing order */
 #define TCHEM_LU_MFMA 3   /* dense FP32 LU on the matrix cores, pivots fixed by the fill-reducing order: one cell
                              per workgroup of 4 wavefronts; mixed precision, m <= 255 */
-#define TCHEM_PROGRAMS_AUTO 0   /* LDS when they leave room for 4 cells, device memory otherwise */
+#define TCHEM_PROGRAMS_AUTO 0   /* LDS when that leaves room for as many cells as device memory does, memory otherwise */
 #define TCHEM_PROGRAMS_LDS 1    /* staged into LDS once per workgroup, shared by its cells (all but the Jacobian assembly
                                    and the factor-reuse solve, which are read from memory) */
 #define TCHEM_PROGRAMS_MEMORY 2 /* read from device memory (L2-resident); the LDS holds the cells and the
                                    coefficient table */
+                                /* either way the tolerances are in LDS too where they cost no cell */
 typedef struct {
   int precision;         /* TCHEM_PRECISION_* */
   int schedule;          /* TCHEM_SCHEDULE_* */
   int blocks_per_cu;     /* persistent schedule: resident workgroups per CU (0 = from occupancy) */
   int lu;                /* TCHEM_LU_* */
   int cells_per_block;   /* sparse form: cells (wavefronts) per workgroup sharing the LDS-resident
-                            mechanism program (0 = as many as fit); the dense form runs 1 */
+                            mechanism program (0 = as many as fit, fewer where the batch is smaller than the
+                            chip, so that it is spread over all CUs); the dense form runs 1 */
   int programs;          /* sparse form: where the compiled mechanism programs live, TCHEM_PROGRAMS_* */
   int reserved[2];       /* must be zero */
 } tchem_atmchem_options_t;

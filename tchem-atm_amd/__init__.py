@@ -42,7 +42,7 @@ LU_AUTO = 0     # sparse when the mechanism has a sparse schedule, dense otherwi
 LU_DENSE = 1    # dense LU with partial pivoting (the oracle's arithmetic)
 LU_SPARSE = 2   # level-scheduled sparse LU, pivots fixed by the fill-reducing order
 LU_MFMA = 3     # dense FP32 LU on the matrix cores (mixed precision, m <= 255), one cell per 4 wavefronts
-PROGRAMS_AUTO = 0    # sparse form: programs in LDS when they leave room for 4 cells
+PROGRAMS_AUTO = 0    # sparse form: programs in LDS when as many cells fit beside them as without
 PROGRAMS_LDS = 1     # staged into LDS once per workgroup
 PROGRAMS_MEMORY = 2  # read from device memory (L2-resident), all LDS for cells
 

@@ -227,8 +227,11 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   if (o->lu != TCHEM_LU_AUTO && o->lu != TCHEM_LU_DENSE && o->lu != TCHEM_LU_SPARSE && o->lu != TCHEM_LU_MFMA)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": unknown lu");
   // AUTO in mixed precision: the MFMA form when the factor is dense (at
-  // least 30 % of the m^2 entries in the fill-reducing order) and large
-  // enough to fill its 256 x 256 tiles (m >= 128)
+  // least 30 % of the m^2 entries in the fill-reducing order) and m >= 128.
+  // Uniform mechanisms, 2000 cells, 10 iterations, sparse against MFMA: 90
+  // species 3170 / 6338 us, 110 5182 / 6216, 127 10120 / 6410; batches that
+  // leave CUs idle would gain from fewer species on (64 cells, 90 species
+  // 1512 / 811 us).
   if (o->lu == TCHEM_LU_AUTO && o->precision == TCHEM_PRECISION_MIXED && o->cells_per_block <= 1 &&
       k->dev.m >= 128 && k->dev.m <= 255 && k->dev.oMfjTermW != 0 && mfmaCellLdsBytes(k->dev) <= k->maxLds &&
       (k->nnzF == 0 || double(k->nnzF) >= 0.3 * double(k->dev.m) * double(k->dev.m)))
@@ -1378,7 +1381,7 @@ int tchem_atmchem_autotune(tchem_atmchem_options_t* opts, int nBatch, const doub
   }
   for (int lu : {TCHEM_LU_DENSE, TCHEM_LU_MFMA}) {
     if (luIn != TCHEM_LU_AUTO && luIn != lu) continue;
-    if (luIn == TCHEM_LU_AUTO && lu == TCHEM_LU_MFMA && kmcd->dev.m < 128) continue;  // tiles mostly padding
+    if (luIn == TCHEM_LU_AUTO && lu == TCHEM_LU_MFMA && kmcd->dev.m < 128) continue;  // sparse is faster on a full chip (resolveOptions)
     tchem_atmchem_options_t t = base;
     t.lu = lu;
     tchem_atmchem_options_t r;

@@ -1797,8 +1797,9 @@ __global__ __launch_bounds__(64) void aerosol_rhs_kernel(IntegratorArgs a) {
 // iteration, sixteen took 76 k), not flops or bytes: the encoded programs
 // (lowered.hpp, sparse_exec.hpp) replaced an interpreter of the rounds that
 // decoded kind, length and indices per round and waited for scalar loads.
-// Then slots spread over the LDS banks and pivots inverted once per
-// factorisation.  Measured, interpreter -> encoded -> spread: 131040 cells
+// Then slots spread over the LDS banks, and pivots checked (and their
+// reciprocals kept for the back substitution) once after the last round; the
+// multiplier rounds still invert the pivots they use.  Measured, interpreter -> encoded -> spread: 131040 cells
 // mixed, 80 TR-BDF2 iterations 305.2 -> 160.5 -> 145.3 ms; 16411 cells FP64,
 // 100 iterations 69.8 -> 36.8 -> 37.4 ms; one cell, 10 iterations 594 -> 309
 // -> 300 us; E3SM 40960 cells to 1800 s 63.6 -> 32.3 -> 30.7 ms; CB05 + SOA,
@@ -2228,8 +2229,9 @@ static const void* integratorFn() {
 // latency-bound kernel sets its throughput, so each workgroup size gets the
 // instance with the largest register budget that still lets its wavefronts
 // be resident: FP64 up to 8 cells 512 threads (256 VGPRs), 9-12 cells 768
-// (168); mixed up to 12 cells 768, 13-16 cells 1024 (128 VGPRs, 4 per SIMD,
-// a few registers spilled).
+// (168); mixed up to 12 cells 768, 13-16 cells 1024 (128 VGPRs, 4 per SIMD;
+// of these the one for 65 to 128 unknowns with staged programs spills 3
+// registers, no other sparse instance spills any).
 int sparseMaxCellsPerGroup(int precision, const DevLowered& w) {
   if (w.shift) return 8;
   return precision == TCHEM_PRECISION_MIXED ? 16 : 12;

@@ -142,7 +142,6 @@ struct SpLds {
   unsigned coef;      // coefficient table
   unsigned tol;       // (atol, rtol) per unknown
   double* c;          // [nSpec]
-  double* kf;         // [nReac]
   const double* src;  // nullable: this cell's external sources [m], reference order
 };
 
@@ -386,7 +385,7 @@ __device__ __forceinline__ void sp_lu(const L& S, const Words& words, int oHdr, 
 }
 
 // Reciprocal pivots of the m rows, kept beside their right-hand sides (the
-// rounds multiply with the same values).  Returns false when a pivot is zero
+// multiplier rounds form the same values again).  Returns false when a pivot is zero
 // or not finite.
 template <int SH, int QM, typename L>
 __device__ __forceinline__ bool sp_pivots(const DevLowered& W, const L& S, int m, int lane) {
@@ -455,7 +454,6 @@ __device__ __forceinline__ SpLds<TA, STAGED> carve_sparse(const DevLowered& W, c
   const size_t at = sparseStageBytes(W, m, STAGED) + size_t(wave) * size_t(cellBytes);
   L.cell = __builtin_amdgcn_readfirstlane(b + unsigned(at));
   L.c = reinterpret_cast<double*>(base + at + W.oC);
-  L.kf = reinterpret_cast<double*>(base + at + W.oK);
   L.src = nullptr;
   return L;
 }
