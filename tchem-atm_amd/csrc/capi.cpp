@@ -122,8 +122,10 @@ struct tchem_kmcd_s {
   DevMech dev{};
   // encoded sparse programs (enabled 0: none): FP64 and FP32 entries, and
   // the adjoint's forward and transposed programs on their own cell layout
-  DevLowered low64{}, low32{}, lowAdj{}, lowAdjT{};
-  const DevLowered& lowered(int precision) const { return precision == TCHEM_PRECISION_FP64 ? low64 : low32; }
+  DevLowered low64[2]{}, low32[2]{}, lowAdj{}, lowAdjT{};  // [programs in memory, staged]: differ in tolStaged
+  const DevLowered& lowered(int precision, bool staged) const {
+    return (precision == TCHEM_PRECISION_FP64 ? low64 : low32)[staged];
+  }
   std::vector<void*> allocations;
   int device = 0;
   int numCUs = 0;
@@ -253,7 +255,7 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   if (o->programs < TCHEM_PROGRAMS_AUTO || o->programs > TCHEM_PROGRAMS_MEMORY)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": unknown programs placement");
   const size_t bytesA = o->precision == TCHEM_PRECISION_FP64 ? sizeof(double) : sizeof(float);
-  const DevLowered& W = k->lowered(o->precision);
+  const DevLowered& W = k->lowered(o->precision, false);
   const size_t staticLds = integratorStaticLds(o->precision, 1, k->dev.m, W);
   const size_t maxLds = k->maxLds > staticLds ? k->maxLds - staticLds : 0;
   const size_t cellB = size_t(W.cellBytes);
@@ -263,12 +265,12 @@ int resolveOptions(const tchem_atmchem_options_t* opts, const tchem_kmcd_s* k, t
   if (o->programs == TCHEM_PROGRAMS_AUTO) {
     const int cap = sparseMaxCellsPerGroup(o->precision, W);
     const int inMem = sparseCellsThatFit(W, k->dev.m, false, cellB, maxLds, cap);
-    const int inLds = sparseCellsThatFit(W, k->dev.m, true, cellB, maxLds, cap);
+    const int inLds = sparseCellsThatFit(k->lowered(o->precision, true), k->dev.m, true, cellB, maxLds, cap);
     o->programs = (inLds >= 1 && inLds >= inMem) ? TCHEM_PROGRAMS_LDS : TCHEM_PROGRAMS_MEMORY;
   }
   const bool staged = o->programs == TCHEM_PROGRAMS_LDS;
   auto sparseFits = [&](int cells) {
-    return sparseStageBytes(W, k->dev.m, staged) + size_t(cells) * cellB <= maxLds;
+    return sparseStageBytes(k->lowered(o->precision, staged), k->dev.m, staged) + size_t(cells) * cellB <= maxLds;
   };
   if (o->lu == TCHEM_LU_AUTO)
     o->lu = (W.enabled && sparseFits(1)) ? TCHEM_LU_SPARSE : TCHEM_LU_DENSE;
@@ -307,7 +309,7 @@ size_t ldsBytes(const tchem_kmcd_s* k, const tchem_atmchem_options_t& o) {
   if (o.lu == TCHEM_LU_MFMA) return mfmaCellLdsBytes(k->dev);
   const size_t bytesA = o.precision == TCHEM_PRECISION_FP64 ? sizeof(double) : sizeof(float);
   if (o.lu == TCHEM_LU_SPARSE) {
-    const DevLowered& W = k->lowered(o.precision);
+    const DevLowered& W = k->lowered(o.precision, sparseStaged(o));
     return sparseStageBytes(W, k->dev.m, sparseStaged(o)) + size_t(o.cells_per_block) * size_t(W.cellBytes);
   }
   return integratorLdsBytes(k->dev, bytesA);
@@ -343,7 +345,7 @@ int resolveBlocksPerCU(const tchem_kmcd_s* kmcd, const tchem_atmchem_options_t& 
   *bpc = o.blocks_per_cu;
   if (*bpc > 0) return TCHEM_OK;
   const int sparse = o.lu == TCHEM_LU_MFMA ? 3 : (o.lu == TCHEM_LU_SPARSE ? (sparseStaged(o) ? 1 : 2) : 0);
-  hipError_t e = integratorMaxBlocksPerCU(o.precision, sparse, kmcd->dev.m, kmcd->lowered(o.precision),
+  hipError_t e = integratorMaxBlocksPerCU(o.precision, sparse, kmcd->dev.m, kmcd->lowered(o.precision, sparseStaged(o)),
                                           64 * o.cells_per_block, launchLdsBytes(kmcd, o), bpc, rec);
   if (e != hipSuccess) return hipFail(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
   if (*bpc < 1) *bpc = 1;
@@ -385,7 +387,7 @@ int runIntegrator(tchem_kmcd_s* kmcd, tchem_atmchem_options_t o, bool spread, co
   if (hipGetDevice(&cur) != hipSuccess || cur != kmcd->device)
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": kmcd belongs to another device");
   a.M = kmcd->dev;
-  a.W = kmcd->lowered(o.precision);
+  a.W = kmcd->lowered(o.precision, sparseStaged(o));
   a.sparse = o.lu == TCHEM_LU_MFMA ? 3 : (o.lu == TCHEM_LU_SPARSE ? (sparseStaged(o) ? 1 : 2) : 0);
   if (!a.queue) a.queue = kmcd->queue;
   a.persistent = (o.schedule == TCHEM_SCHEDULE_PERSISTENT) ? 1 : 0;
@@ -442,7 +444,7 @@ int adjointCheck(const tchem_kmcd_s* k, int nBatch, int maxSteps, const char* wh
   if (nBatch < 0) return setError(TCHEM_ERR_INVALID, std::string(who) + ": negative nBatch");
   if (maxSteps < 1 || maxSteps > (1 << 24))
     return setError(TCHEM_ERR_INVALID, std::string(who) + ": maxSteps must be in [1, 2^24]");
-  if (!k->low64.enabled || !k->lowAdj.enabled || !k->lowAdjT.enabled)
+  if (!k->low64[0].enabled || !k->lowAdj.enabled || !k->lowAdjT.enabled)
     return setError(TCHEM_ERR_UNSUPPORTED, std::string(who) + ": mechanism has no sparse (transposed) schedule");
   return TCHEM_OK;
 }
@@ -740,25 +742,29 @@ int tchem_kmcd_create(tchem_kmd_t kmd, tchem_kmcd_t* out) {
   // exceeds the LDS, run the dense form only)
   auto pack = [&](const SparseSchedule& sc, const LoweredSlots& slots, int bytesT, bool adjoint, DevLowered* w) {
     LoweredProgram p = lowerProgram(t, sc, bytesT, adjoint, slots);
-    if (!adjoint)
-      stageTolerances(p.d, t.m, size_t(p.d.cellBytes), k->maxLds,
-                      sparseMaxCellsPerGroup(bytesT == 8 ? TCHEM_PRECISION_FP64 : TCHEM_PRECISION_MIXED, p.d));
     if (sparseStageBytes(p.d, t.m, false) + size_t(p.d.cellBytes) > k->maxLds) return;
     *w = p.d;
     w->oWords = addI(std::vector<int>(p.words.begin(), p.words.end()));
     w->oCoef = addD(p.coef);
+  };
+  auto packForms = [&](const SparseSchedule& sc, const LoweredSlots& slots, int bytesT, DevLowered (&w)[2]) {
+    pack(sc, slots, bytesT, false, &w[0]);
+    w[1] = w[0];
+    const int most = sparseMaxCellsPerGroup(bytesT == 8 ? TCHEM_PRECISION_FP64 : TCHEM_PRECISION_MIXED, w[0]);
+    for (const bool staged : {false, true})
+      stageTolerances(w[staged], t.m, staged, size_t(w[0].cellBytes), k->maxLds, most);
   };
   try {
     if (!k->boxModel) throw std::runtime_error("no box model");
     const SparseSchedule fwd = buildSparseSchedule(t, false, false);
     k->nnzF = fwd.nnzF;
     const LoweredSlots fs = chooseSlots(t, fwd);
-    pack(fwd, fs, 8, false, &k->low64);
-    pack(fwd, fs, 4, false, &k->low32);
+    packForms(fwd, fs, 8, k->low64);
+    packForms(fwd, fs, 4, k->low32);
     // the adjoint shares one cell layout between the forward programs and
     // the transposed ones: the transposed factor pattern has the same size
     const SparseSchedule trn = buildSparseSchedule(t, true, false);
-    if (k->low64.enabled && trn.nnzF == fwd.nnzF && trn.pairSlots == fwd.pairSlots) {
+    if (k->low64[0].enabled && trn.nnzF == fwd.nnzF && trn.pairSlots == fwd.pairSlots) {
       pack(fwd, fs, 8, true, &k->lowAdj);
       pack(trn, chooseSlots(t, trn, &fs), 8, true, &k->lowAdjT);
     }
@@ -1727,7 +1733,7 @@ int tchem_amcd_create(tchem_amd_t amd, tchem_kmcd_t kmcd, tchem_amcd_t* out) {
     };
     X.oJpos = int(ib.size());
     for (const auto& e : ent) ib.push_back(position(e[0], e[1]));
-    stageTolerances(p.d, mt, aerosolSparseCellBytes(p.d, X), kmcd->maxLds, kMaxAerosolCells);
+    stageTolerances(p.d, mt, false, aerosolSparseCellBytes(p.d, X), kmcd->maxLds, kMaxAerosolCells);
     h->W = p.d;
     pib.assign(p.words.begin(), p.words.end());
     pdb = std::move(p.coef);

@@ -87,7 +87,7 @@ struct DevMech {
 // of m unknowns.
 __host__ __device__ inline size_t sparseStageBytes(const DevLowered& W, int m, bool staged) {
   return (staged ? 4 * size_t(W.stagedWords) : 0) + ((8 * size_t(W.nCoef) + 15) & ~size_t(15)) +
-         (W.tolStaged[staged] ? 16 * size_t(m) : 0);
+         (W.tolStaged ? 16 * size_t(m) : 0);
 }
 // Cells (at most `most`) of cellBytes that fit beside them.
 inline int sparseCellsThatFit(const DevLowered& W, int m, bool staged, size_t cellBytes, size_t maxLds, int most) {
@@ -98,13 +98,11 @@ inline int sparseCellsThatFit(const DevLowered& W, int m, bool staged, size_t ce
 // Tolerances are staged where they cost no cell: they are read once per step,
 // resident cells set the throughput (16 mixed cells of the CB05 + SOA gas
 // phase fit without them, 15 with).
-inline void stageTolerances(DevLowered& W, int m, size_t cellBytes, size_t maxLds, int most) {
-  for (const bool staged : {false, true}) {
-    W.tolStaged[staged] = 0;
-    const int without = sparseCellsThatFit(W, m, staged, cellBytes, maxLds, most);
-    W.tolStaged[staged] = 1;
-    W.tolStaged[staged] = without > 0 && sparseCellsThatFit(W, m, staged, cellBytes, maxLds, most) == without;
-  }
+inline void stageTolerances(DevLowered& W, int m, bool staged, size_t cellBytes, size_t maxLds, int most) {
+  W.tolStaged = 0;
+  const int without = sparseCellsThatFit(W, m, staged, cellBytes, maxLds, most);
+  W.tolStaged = 1;
+  W.tolStaged = without > 0 && sparseCellsThatFit(W, m, staged, cellBytes, maxLds, most) == without;
 }
 
 // Forward record of the discrete adjoint: accepted step sizes and the state
@@ -169,12 +167,16 @@ struct IntegratorArgs {
 // the source term, reciprocal pivots and interchanges over mt, SIMPOL
 // constants [nSimpol][4], particle sums [nPart][4] and transfer terms
 // [nPart * nSimpol][6].
+__host__ __device__ inline int sparseScratchOffset(const DevLowered& W) {
+  const int a = W.oP < W.oS ? W.oP : W.oS;
+  return a < W.oD ? a : W.oD;
+}
 // LDS bytes of one cell of the sparse aerosol integrator: the cell region of
 // the encoded programs, whose part that is dead once the Jacobian is
 // assembled takes the unknown copy, source term and SIMPOL scratch of
 // aerosolLdsBytes, as far as it reaches; then the SIMPOL constants.
 __host__ __device__ inline size_t aerosolScratchEnd(const DevLowered& W, const DevAerosol& X) {
-  const size_t end = size_t(W.oFree) + 8 * (2 * size_t(X.mt) + 4 * size_t(X.nPart) + 6 * size_t(X.nPart) * size_t(X.nSimpol));
+  const size_t end = size_t(sparseScratchOffset(W)) + 8 * (2 * size_t(X.mt) + 4 * size_t(X.nPart) + 6 * size_t(X.nPart) * size_t(X.nSimpol));
   return end > size_t(W.cellBytes) ? end : size_t(W.cellBytes);
 }
 inline size_t aerosolSparseCellBytes(const DevLowered& W, const DevAerosol& X) {

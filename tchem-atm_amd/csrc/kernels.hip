@@ -547,10 +547,10 @@ struct DenseBackend {
 
 // time tolerances of unknown ai from the staged table at LDS address tol, or
 // (index: its row) from the caller's
-template <bool STAGED, class Index>
+template <class Index>
 __device__ __forceinline__ void staged_tolerance(const IntegratorArgs& a, unsigned tol, int ai, Index index,
                                                  double& atol, double& rtol) {
-  if (a.W.tolStaged[STAGED]) {
+  if (a.W.tolStaged) {
     const vec2<double> t = lds_get<vec2<double>>(tol + 16 * ai);
     atol = t.x;
     rtol = t.y;
@@ -576,7 +576,7 @@ struct SparseBackend {
   static __device__ __forceinline__ int column(const IntegratorArgs& a, int ai) { return 3 + a.M.perm()[ai]; }
   static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds& L, int ai, double& atol,
                                                    double& rtol) {
-    staged_tolerance<STAGED>(a, L.tol, ai, [&](int i) { return a.M.perm()[i]; }, atol, rtol);
+    staged_tolerance(a, L.tol, ai, [&](int i) { return a.M.perm()[i]; }, atol, rtol);
   }
   static __device__ __forceinline__ void bind(const IntegratorArgs& a, Lds& L, int cell) {
     L.src = a.ext ? a.ext + size_t(cell) * a.M.m : nullptr;
@@ -584,7 +584,7 @@ struct SparseBackend {
   static __device__ void stage(const IntegratorArgs& a, char* base) {
     stage_sparse<STAGED>(a.W, reinterpret_cast<const unsigned*>(a.M.ib) + a.W.oWords, a.M.db + a.W.oCoef, base);
     double* tol = reinterpret_cast<double*>(base + sparseStageBytes(a.W, 0, STAGED));
-    const int n = a.W.tolStaged[STAGED] ? 2 * a.M.m : 0;
+    const int n = a.W.tolStaged ? 2 * a.M.m : 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) tol[i] = a.tol_time[2 * a.M.perm()[i >> 1] + (i & 1)];
     __syncthreads();
   }
@@ -1606,7 +1606,7 @@ __device__ AeroSpLds carve_aero_sparse(char* base, const IntegratorArgs& a, int 
       a.W, reinterpret_cast<const unsigned*>(X.pib) + a.W.oWords, X.mt, base, a.cellBytes, wave);
   char* cell = base + sparseStageBytes(a.W, X.mt, false) + size_t(wave) * size_t(a.cellBytes);
   L.A = reinterpret_cast<double*>(cell);
-  L.x = reinterpret_cast<double*>(cell + a.W.oFree);
+  L.x = reinterpret_cast<double*>(cell + sparseScratchOffset(a.W));
   L.f = L.x + X.mt;
   L.ps = L.f + X.mt;
   L.pd = L.ps + 4 * X.nPart;
@@ -1625,12 +1625,12 @@ struct AerosolSparseBackend : AerosolLayout {
   struct Fact {};
   static __device__ __forceinline__ void tolerance(const IntegratorArgs& a, const Lds& L, int ai, double& atol,
                                                    double& rtol) {
-    staged_tolerance<false>(a, L.tol, ai, [&](int i) { return i < a.M.m ? a.M.perm()[i] : i; }, atol, rtol);
+    staged_tolerance(a, L.tol, ai, [&](int i) { return i < a.M.m ? a.M.perm()[i] : i; }, atol, rtol);
   }
   static __device__ void stage(const IntegratorArgs& a, char* base) {
     stage_sparse<false>(a.W, nullptr, a.X.pdb + a.W.oCoef, base);
     double* tol = reinterpret_cast<double*>(base + sparseStageBytes(a.W, 0, false));
-    const int n = a.W.tolStaged[0] ? 2 * a.X.mt : 0;
+    const int n = a.W.tolStaged ? 2 * a.X.mt : 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
       const int ai = i >> 1, xs = ai < a.M.m ? a.M.perm()[ai] : ai;
       tol[i] = a.tol_time[2 * xs + (i & 1)];
@@ -2230,7 +2230,7 @@ static const void* integratorFn() {
 // instance with the largest register budget that still lets its wavefronts
 // be resident: FP64 up to 8 cells 512 threads (256 VGPRs), 9-12 cells 768
 // (168); mixed up to 12 cells 768, 13-16 cells 1024 (128 VGPRs, 4 per SIMD;
-// of these the one for 65 to 128 unknowns with staged programs spills 3
+// of these the one for 65 to 128 unknowns with staged programs spills 2
 // registers, no other sparse instance spills any).
 int sparseMaxCellsPerGroup(int precision, const DevLowered& w) {
   if (w.shift) return 8;

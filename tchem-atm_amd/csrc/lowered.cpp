@@ -362,7 +362,7 @@ struct Lowering {
     d.zero8 = oScaled + 8 * int(scaled.size());
     d.oK = d.zero8 + 8;
     d.nK = t.nReac + int(scaled.size()) + 1;
-    o = d.oFree = d.oK + 8 * t.nReac;  // idle lanes of K: on anything behind, loaded before all of it
+    o = d.oK + 8 * t.nReac;  // idle lanes of K: on anything behind, loaded before all of it
     int end = 0;
     if (adjoint) {
       // w v P D: w outlives powers and pairs (gradient), P outlives the

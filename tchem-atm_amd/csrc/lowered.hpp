@@ -71,8 +71,7 @@ struct DevLowered {
                     // or rarely run; the LDS they would take holds cells)
   int oWords;     // stream start in the mechanism's int buffer
   int nCoef, oCoef;  // coefficient table (staged into LDS), start in the double buffer
-  int tolStaged[2];  // whether the unknowns' tolerances are staged into LDS too, with the programs in memory and with
-                     // the programs staged (stageTolerances)
+  int tolStaged;     // whether the unknowns' tolerances are staged into LDS too (set by the caller: stageTolerances)
   // cell layout
   int cellBytes;
   int zeroA, trashA;      // slots of the factor array (which starts at 0)
@@ -80,8 +79,7 @@ struct DevLowered {
   int oD, oPS;            // derivative pairs; partial sums (with the segment sums, which are dead then)
   int oC, oneC, trashC;   // concentrations, the slot that holds 1
   int oK, nK, zero8;      // rate constants, with n * kf slots and the slot that holds 0 before them (nK in all)
-  int oP, oS;             // rates of progress, segment sums
-  int oFree;              // the regions from here to the end (pairs, partial, segment sums, rates of progress) are
+  int oP, oS;             // rates of progress, segment sums; from the first of oP, oS and oD to the end everything is
                           // dead once the Jacobian is assembled (not in the adjoint)
   // sections
   int oPow, nPow, oKf, oKfx, nKfx, oRop, nRop, oPair, nPair;

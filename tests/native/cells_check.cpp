@@ -28,9 +28,12 @@ int main(int argc, char** argv) {
       DevLowered w = lowerProgram(t, s, bytes, false, fs).d;
       const size_t cell = size_t(w.cellBytes);
       const int most = t.m > 128 ? 8 : (bytes == 8 ? 12 : 16);
-      stageTolerances(w, t.m, cell, kLds, most);
-      std::printf("fp%d memory %d staged %d\n", 8 * bytes, sparseCellsThatFit(w, t.m, false, cell, kLds, most),
-                  sparseCellsThatFit(w, t.m, true, cell, kLds, most));
+      int n[2];
+      for (const bool staged : {false, true}) {
+        stageTolerances(w, t.m, staged, cell, kLds, most);
+        n[staged] = sparseCellsThatFit(w, t.m, staged, cell, kLds, most);
+      }
+      std::printf("fp%d memory %d staged %d\n", 8 * bytes, n[0], n[1]);
     }
   }
   for (int i = 3; i < argc; ++i) {
@@ -43,7 +46,7 @@ int main(int argc, char** argv) {
     X.mt = ta.m;
     X.nPart = am.nParticles;
     X.nSimpol = int(am.simpol.size());
-    stageTolerances(w, ta.m, aerosolSparseCellBytes(w, X), kLds, 8);
+    stageTolerances(w, ta.m, false, aerosolSparseCellBytes(w, X), kLds, 8);
     std::printf("particles %d: %d\n", am.nParticles,
                 sparseCellsThatFit(w, ta.m, false, aerosolSparseCellBytes(w, X), kLds, 8));
   }
